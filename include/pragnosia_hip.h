@@ -236,6 +236,31 @@ int pragnosia_aspin_exact_bwd(const void* q, const void* k, const void* v, const
                               void* dk, void* dv, void* dla, void* dbeta, void* dS0, int64_t B, int64_t H, int64_t T,
                               int64_t Dk, int64_t Dv, int dtype, void* stream);
 
+/* The exact scan's function in chunked form (64-token chunks, fp32 matrix cores), fp32 only: the plain rule when beta
+ * is NULL (any Dk, Dv), the delta rule when given (Dk <= 384). Layouts as pragnosia_aspin_exact_fwd. With NC =
+ * ceil(T / 64), the forward also writes, for the backward and for itself (all required): states (B, H, NC, Dk, Dv), the
+ * state entering every chunk; scores (B, H, NC, 64, 64); gates (2, B, H, NC, 64), the decays from a chunk's start and to
+ * its end; and for the delta rule M and X (B, H, NC, 64, 64), R and U (B, H, T, Dv) and the scratch W (B, H, NC, 64, Dk
+ * rounded up to 16). scores, gates, M, X and W are 16-byte aligned; the other arrays need no more than a float's
+ * alignment (16-byte loads are used when all of them have it and Dk and Dv are multiples of 4). */
+int pragnosia_aspin_exact_chunk_fwd(const float* q, const float* k, const float* v, const float* la, const float* beta,
+                                    const float* S0, float* o, float* S_final, float* states, float* scores,
+                                    float* gates, float* M, float* X, float* R, float* U, float* W, int64_t B,
+                                    int64_t H, int64_t T, int64_t Dk, int64_t Dv, void* stream);
+
+/* Bytes of the backward's workspace (16-byte aligned), or -1 for a shape it refuses; delta != 0 for the delta rule. */
+int64_t pragnosia_aspin_exact_chunk_bwd_workspace_bytes(int64_t B, int64_t H, int64_t T, int64_t Dk, int64_t Dv,
+                                                        int delta);
+
+/* Backward of pragnosia_aspin_exact_chunk_fwd from dO (B, H, T, Dv) and dS_final (or NULL = zero): writes dq, dk, dv,
+ * dla, dbeta (delta rule) and, if non-NULL, dS0. */
+int pragnosia_aspin_exact_chunk_bwd(const float* q, const float* k, const float* v, const float* la, const float* beta,
+                                    const float* states, const float* scores, const float* gates, const float* M,
+                                    const float* X, const float* R, const float* U, const float* dO,
+                                    const float* dS_final, float* dq, float* dk, float* dv, float* dla, float* dbeta,
+                                    float* dS0, float* workspace, int64_t workspace_bytes, int64_t B, int64_t H,
+                                    int64_t T, int64_t Dk, int64_t Dv, void* stream);
+
 /* ---------------------------------------------------------------------------------------------------------
  * Associative carrier, DELTA write rule, chunked scan (chunk = 64, head dim D = 64 or 128), per (batch, head):
  *     S_t = a_t S_{t-1} + beta_t k_t (v_t - (a_t S_{t-1})^T k_t)^T,   o_t = S_t^T q_t,   a_t = exp(la_t).

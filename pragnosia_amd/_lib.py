@@ -41,6 +41,9 @@ SIGNATURES = {
     "pragnosia_aspin_out_bwd": [_p, _i32] + [_p] * 5 + [_i64] * 4 + [_p],
     "pragnosia_aspin_exact_fwd": [_p] * 10 + [_i64] * 5 + [_i32, _p],
     "pragnosia_aspin_exact_bwd": [_p] * 15 + [_i64] * 5 + [_i32, _p],
+    "pragnosia_aspin_exact_chunk_fwd": [_p] * 16 + [_i64] * 5 + [_p],
+    "pragnosia_aspin_exact_chunk_bwd_workspace_bytes": [_i64] * 5 + [_i32],
+    "pragnosia_aspin_exact_chunk_bwd": [_p] * 21 + [_i64] * 6 + [_p],
     "pragnosia_aspin_delta_fwd": [_p] * 11 + [_i64] * 5 + [_p],
     "pragnosia_aspin_delta_bwd_workspace_bytes": [_i64] * 5,
     "pragnosia_aspin_delta_bwd": [_p] * 17 + [_i64] * 6 + [_p],
@@ -72,7 +75,8 @@ SIGNATURES = {
 _RET_I64 = {"pragnosia_aspin_delta_bwd_workspace_bytes", "pragnosia_aspin_prep_theta_partials",
             "pragnosia_aspin_chunk_seg_workspace_bytes", "pragnosia_aspin_out_weight_partials",
             "pragnosia_aspin_prep_proj_partials", "pragnosia_aspin_chunk_wide_workspace_bytes",
-            "pragnosia_layer_norm_partials", "pragnosia_wgrad_workspace_bytes"}
+            "pragnosia_layer_norm_partials", "pragnosia_wgrad_workspace_bytes",
+            "pragnosia_aspin_exact_chunk_bwd_workspace_bytes"}
 
 _lib = None
 

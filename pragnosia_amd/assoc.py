@@ -134,13 +134,17 @@ def _dim_blocks(n: int, cap: int) -> list[tuple[int, int]]:
 
 def _exact_scan(q, k, v, logalpha, beta, S0, want):
     """The exact scan (`ops.aspin_exact`) at the reference's wide head dims (`src/model.py:636-643`: four or two
-    heads of 176-384). Value columns never mix (each is its own recurrence over the key rows), so every rule splits
+    heads of 176-384). In chunked form (`ops.exact_chunked`) it takes them as they are. Token by token, a launch's LDS
+    bounds them: value columns never mix (each is its own recurrence over the key rows), so every rule splits
     them into blocks that fit one launch's LDS (`exact_value_cap`). The plain rule's key rows evolve independently
     too and its read sums over them: with keys in blocks of at most 128, o[.., vb] = sum over key blocks kb of
     scan(q[.., kb], k[.., kb], v[.., vb]) and S[kb, vb] is that scan's state. The delta rule couples all key rows in
     every write (r = v - P^T k), so its keys stay in one launch, up to EXACT_MAX_DK = 384."""
     Dk, Dv = q.shape[-1], v.shape[-1]
     dt = torch.float64 if q.dtype == torch.float64 else torch.float32
+    if _op_mod.exact_chunked(dt, q.shape[2], Dk, beta is not None):
+        o, S, _, _ = _op.aspin_exact(q, k, v, logalpha, beta, S0, want)
+        return o, S
     if beta is not None and Dk > _op_mod.EXACT_MAX_DK:
         raise PragnosiaError(f"assoc_scan: the delta rule takes key dims up to {_op_mod.EXACT_MAX_DK} (got {Dk}): "
                              "its state does not split into key blocks")

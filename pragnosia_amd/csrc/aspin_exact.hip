@@ -5,12 +5,12 @@
 // chunked two-pass forms `_scan_twopass` / `_scan_twopass_delta` (src/assoc.py:118-165, :207-251), whose tests hold
 // it to the literal recurrence at 1e-11 in fp64 (tests/test_assoc.py:18-44). The bf16-MFMA kernels of
 // aspin_chunk.hip and aspin_delta.hip round every operand to bf16; this file computes the same function with no
-// operand rounding, per token, per (batch, head), S (Dk x Dv) with keys on rows:
+// operand rounding, token by token: in fp64, and in fp32 for sequences shorter than half a chunk (longer ones run
+// chunked on the fp32 matrix cores, aspin_exact_chunk.hip). Per (batch, head), S (Dk x Dv) with keys on rows:
 //     plain:  S_t = a_t S_{t-1} + k_t v_t^T
 //     delta:  P_t = a_t S_{t-1},  r_t = v_t - P_t^T k_t,  S_t = P_t + beta_t k_t r_t^T
 //     o_t = S_t^T q_t,   a_t = exp(la_t).
-// (The chunked form is the same function reassociated; in fp32/fp64 the recurrence itself is the accurate way to
-// evaluate it and needs no chunk inverse.)
+// (The chunked form is the same function reassociated.)
 //
 // Layout of the work: one workgroup per (batch, head), ceil(Dv / 16) waves. Lane l of wave w owns value column
 // j = 16 w + (l & 15) and the R key rows g R .. g R + R - 1 of that column (g = l >> 4, R = the smallest of 2, 4, 8,

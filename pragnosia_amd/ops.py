@@ -928,6 +928,9 @@ EXACT_CKPT = 8  # tokens per checkpointed state (PRAGNOSIA_EXACT_CKPT_TOKENS)
 EXACT_MAX_DK = 384  # key rows (kMaxDk)
 EXACT_MAX_DV = 128  # value columns (kMaxDv)
 EXACT_MAX_LDS = 160 * 1024
+# fp32 sequences of at least this many tokens run in chunked form on the fp32 matrix cores (aspin_exact_chunk.hip), whose
+# unit is a chunk of 64 tokens: below half a chunk the padding outweighs it. fp64 stays token by token.
+EXACT_CHUNK_MIN_T = 32
 
 
 def exact_rows_per_lane(Dk: int) -> int:
@@ -961,13 +964,33 @@ def _dtype_code(dt: torch.dtype) -> int:
     return 1 if dt == torch.float64 else 0
 
 
+def exact_chunked(dt: torch.dtype, T: int, Dk: int, delta: bool) -> bool:
+    """Whether the exact scan of T tokens runs in chunked form (any value width; any key width, up to 384 for the delta
+    rule), rather than token by token."""
+    return dt == torch.float32 and T >= EXACT_CHUNK_MIN_T and (Dk <= EXACT_MAX_DK or not delta)
+
+
+def _exact_parts(B: int, H: int, T: int, Dv: int, delta: bool) -> list[int]:
+    """Sizes (floats) of what the chunked form keeps in `resid`: per chunk the scores and the two decay vectors, then for
+    the delta rule M and X, R and U (multiples of 64, so each part of the buffer is 16-byte aligned)."""
+    n = B * H * ((T + CHUNK - 1) // CHUNK) * CHUNK
+    rows = (B * H * T * Dv + 63) // 64 * 64
+    return [n * CHUNK, 2 * n] + ([n * CHUNK, n * CHUNK, rows, rows] if delta else [])
+
+
+def _exact_views(buf: Tensor, sizes: list[int]) -> list[Optional[Tensor]]:
+    parts = list(buf.split(sizes))
+    return parts + [None] * (6 - len(parts))
+
+
 def _expect_exact(op: str, q: Tensor, k, v, la, beta=None, S0=None) -> None:
-    """q, k (B, H, T, Dk); v (B, H, T, Dv); la, beta (B, H, T); S0 (B, H, Dk, Dv); Dk <= 384, Dv <= 128."""
+    """q, k (B, H, T, Dk); v (B, H, T, Dv); la, beta (B, H, T); S0 (B, H, Dk, Dv); token by token Dk <= 384, Dv <= 128."""
     if q.dim() != 4 or v is None or v.dim() != 4:
         raise PragnosiaError(f"{op}: q and v must be (B, H, T, D)")
     B, H, T, Dk = q.shape
     Dv = v.shape[-1]
-    if not (0 < Dk <= EXACT_MAX_DK and 0 < Dv <= EXACT_MAX_DV):
+    if not (exact_chunked(_exact_dtype(q), T, Dk, beta is not None)
+            or (0 < Dk <= EXACT_MAX_DK and 0 < Dv <= EXACT_MAX_DV)):
         raise PragnosiaError(f"{op}: head dims Dk={Dk}, Dv={Dv} must be in 1..{EXACT_MAX_DK} x 1..{EXACT_MAX_DV}")
     _expect(op, q.device, k=(k, (B, H, T, Dk)), v=(v, (B, H, T, Dv)), la=(la, (B, H, T)), beta=(beta, (B, H, T)),
             S0=(S0, (B, H, Dk, Dv)))
@@ -977,10 +1000,13 @@ def _expect_exact(op: str, q: Tensor, k, v, la, beta=None, S0=None) -> None:
 def aspin_exact(q: Tensor, k: Tensor, v: Tensor, la: Tensor, beta: Optional[Tensor], S0: Optional[Tensor],
                 want_ckpt: bool) -> tuple[Tensor, Tensor, Tensor, Tensor]:
     """The scan with fp32 operands (fp64 when q is fp64), plain rule, or the delta rule when beta is given.
-    q, k (B, H, T, Dk), v (B, H, T, Dv), la and beta (B, H, T), S0 (B, H, Dk, Dv) or None; Dk <= 384, Dv <= 128
-    (wide keys take fewer value columns: exact_value_cap; the library refuses what does not fit its LDS). Returns
-    (o (B, H, T, Dv), S_final (B, H, Dk, Dv), ckpt, resid) in the compute dtype; ckpt (the state entering every 8
-    tokens) and resid (the delta rule's residuals) are what the backward reads, empty unless want_ckpt."""
+    q, k (B, H, T, Dk), v (B, H, T, Dv), la and beta (B, H, T), S0 (B, H, Dk, Dv) or None. Returns (o (B, H, T, Dv),
+    S_final (B, H, Dk, Dv), ckpt, resid) in the compute dtype; ckpt and resid are what the backward reads, empty unless
+    want_ckpt. fp32 sequences of EXACT_CHUNK_MIN_T tokens or more run in chunked form (`exact_chunked`; any widths, the
+    delta rule's keys up to 384): ckpt is the state entering every 64 tokens, resid one flat buffer of the chunks' scores,
+    decays and (delta) inverses and residuals. The rest runs token by token, Dk <= 384 and Dv <= 128 (wide keys take
+    fewer value columns: exact_value_cap; the library refuses what does not fit its LDS): ckpt is the state entering
+    every 8 tokens, resid the delta rule's residuals."""
     _require_gpu(q, k, v, la, beta, S0)
     _expect_exact("aspin_exact", q, k, v, la, beta, S0)
     dt = _exact_dtype(q)
@@ -991,6 +1017,18 @@ def aspin_exact(q: Tensor, k: Tensor, v: Tensor, la: Tensor, beta: Optional[Tens
     dev = q.device
     o = torch.empty(B, H, T, Dv, device=dev, dtype=dt)
     S = torch.empty(B, H, Dk, Dv, device=dev, dtype=dt)
+    if exact_chunked(dt, T, Dk, beta is not None):
+        NC = (T + CHUNK - 1) // CHUNK
+        ckpt = torch.empty(B, H, NC, Dk, Dv, device=dev, dtype=dt)
+        sizes = _exact_parts(B, H, T, Dv, beta is not None)
+        resid = torch.empty(sum(sizes), device=dev, dtype=dt)
+        scores, gates, M, X, R, U = _exact_views(resid, sizes)
+        W = torch.empty(B * H * NC * CHUNK, (Dk + 15) // 16 * 16, device=dev) if beta is not None else None
+        check(lib().pragnosia_aspin_exact_chunk_fwd(_ptr(q), _ptr(k), _ptr(v), _ptr(la), _ptr(beta), _ptr(S0), _ptr(o),
+                                                    _ptr(S), _ptr(ckpt), _ptr(scores), _ptr(gates), _ptr(M), _ptr(X),
+                                                    _ptr(R), _ptr(U), _ptr(W), B, H, T, Dk, Dv, _stream(q)),
+              "pragnosia_aspin_exact_chunk_fwd")
+        return (o, S, ckpt, resid) if want_ckpt else (o, S, q.new_empty(0), q.new_empty(0))
     NB = (T + EXACT_CKPT - 1) // EXACT_CKPT
     ckpt = torch.empty(B, H, NB, Dk, Dv, device=dev, dtype=dt) if want_ckpt else q.new_empty(0)
     resid = (torch.empty(B, H, T, Dv, device=dev, dtype=dt) if (want_ckpt and beta is not None)
@@ -1007,6 +1045,10 @@ def _(q, k, v, la, beta, S0, want_ckpt):
     B, H, T, Dk = q.shape
     Dv = v.shape[-1]
     dt = _exact_dtype(q)
+    if want_ckpt and exact_chunked(dt, T, Dk, beta is not None):
+        return (q.new_empty(B, H, T, Dv, dtype=dt), q.new_empty(B, H, Dk, Dv, dtype=dt),
+                q.new_empty(B, H, (T + CHUNK - 1) // CHUNK, Dk, Dv, dtype=dt),
+                q.new_empty(sum(_exact_parts(B, H, T, Dv, beta is not None)), dtype=dt))
     NB = (T + EXACT_CKPT - 1) // EXACT_CKPT
     ckpt = q.new_empty(B, H, NB, Dk, Dv, dtype=dt) if want_ckpt else q.new_empty(0, dtype=dt)
     resid = q.new_empty(B, H, T, Dv, dtype=dt) if (want_ckpt and beta is not None) else q.new_empty(0, dtype=dt)
@@ -1017,25 +1059,43 @@ def _(q, k, v, la, beta, S0, want_ckpt):
 def aspin_exact_bwd(q: Tensor, k: Tensor, v: Tensor, la: Tensor, beta: Optional[Tensor], ckpt: Tensor,
                     resid: Optional[Tensor], do: Tensor,
                     dS: Optional[Tensor]) -> tuple[Tensor, Tensor, Tensor, Tensor, Tensor, Tensor]:
-    """Backward of aspin_exact. Returns (dq, dk, dv, dla, dbeta (empty for the plain rule), dS0) in the compute
-    dtype."""
+    """Backward of aspin_exact, from what it kept (ckpt and resid, in the form that aspin_exact picked for these
+    sizes). Returns (dq, dk, dv, dla, dbeta (empty for the plain rule), dS0) in the compute dtype."""
     _require_gpu(q, k, v, la, beta, ckpt, resid, do, dS)
     _expect_exact("aspin_exact_bwd", q, k, v, la, beta)
     B, H, T, Dk = q.shape
     Dv = v.shape[-1]
-    NB = (T + EXACT_CKPT - 1) // EXACT_CKPT
-    _expect("aspin_exact_bwd", q.device, ckpt=(ckpt, (B, H, NB, Dk, Dv)), do=(do, (B, H, T, Dv)),
-            dS=(dS, (B, H, Dk, Dv)), resid=(resid if beta is not None else None, (B, H, T, Dv)))
     dt = _exact_dtype(q)
+    delta = beta is not None
+    chunked = exact_chunked(dt, T, Dk, delta)
+    NB = (T + CHUNK - 1) // CHUNK if chunked else (T + EXACT_CKPT - 1) // EXACT_CKPT
+    sizes = _exact_parts(B, H, T, Dv, delta) if chunked else []
+    _expect("aspin_exact_bwd", q.device, ckpt=(ckpt, (B, H, NB, Dk, Dv)), do=(do, (B, H, T, Dv)),
+            dS=(dS, (B, H, Dk, Dv)),
+            resid=(resid if (chunked or delta) else None, (sum(sizes),) if chunked else (B, H, T, Dv)))
+    if (chunked or delta) and resid is None:
+        raise PragnosiaError("aspin_exact_bwd: resid is what aspin_exact returned beside ckpt")
     cv = lambda t: None if t is None else t.to(dt).contiguous()
     q, k, v, la, beta, ckpt, do, dS = cv(q), cv(k), cv(v), cv(la), cv(beta), cv(ckpt), cv(do), cv(dS)
-    resid = cv(resid) if beta is not None else None
+    resid = cv(resid) if (chunked or delta) else None
     dev = q.device
     dq, dk = torch.empty(B, H, T, Dk, device=dev, dtype=dt), torch.empty(B, H, T, Dk, device=dev, dtype=dt)
     dv = torch.empty(B, H, T, Dv, device=dev, dtype=dt)
     dla = torch.empty(B, H, T, device=dev, dtype=dt)
     dbeta = torch.empty(B, H, T, device=dev, dtype=dt) if beta is not None else q.new_empty(0)
     dS0 = torch.empty(B, H, Dk, Dv, device=dev, dtype=dt)
+    if chunked:
+        nbytes = lib().pragnosia_aspin_exact_chunk_bwd_workspace_bytes(B, H, T, Dk, Dv, int(delta))
+        if nbytes < 0:
+            raise PragnosiaError(f"aspin_exact_bwd: shape rejected (B={B} H={H} T={T} Dk={Dk} Dv={Dv})")
+        ws = torch.empty(nbytes, device=dev, dtype=torch.uint8)
+        scores, gates, M, X, R, U = _exact_views(resid, sizes)
+        check(lib().pragnosia_aspin_exact_chunk_bwd(
+            _ptr(q), _ptr(k), _ptr(v), _ptr(la), _ptr(beta), _ptr(ckpt), _ptr(scores), _ptr(gates), _ptr(M), _ptr(X),
+            _ptr(R), _ptr(U), _ptr(do), _ptr(dS), _ptr(dq), _ptr(dk), _ptr(dv), _ptr(dla),
+            _ptr(dbeta) if delta else None, _ptr(dS0), _ptr(ws), nbytes, B, H, T, Dk, Dv, _stream(q)),
+            "pragnosia_aspin_exact_chunk_bwd")
+        return dq, dk, dv, dla, dbeta, dS0
     check(lib().pragnosia_aspin_exact_bwd(_ptr(q), _ptr(k), _ptr(v), _ptr(la), _ptr(beta), _ptr(ckpt), _ptr(resid),
                                           _ptr(do), _ptr(dS), _ptr(dq), _ptr(dk), _ptr(dv), _ptr(dla),
                                           _ptr(dbeta) if beta is not None else None, _ptr(dS0), B, H, T, Dk, Dv,
@@ -1069,7 +1129,7 @@ def _exact_backward(ctx, do, dS, _dckpt, _dresid):
     q, k, v, la, beta, ckpt, resid = ctx.saved_tensors
     if do is None:
         do = torch.zeros(*q.shape[:3], v.shape[-1], device=q.device, dtype=_exact_dtype(q))
-    dq, dk, dv, dla, dbeta, dS0 = aspin_exact_bwd(q, k, v, la, beta, ckpt, resid if ctx.has_beta else None,
+    dq, dk, dv, dla, dbeta, dS0 = aspin_exact_bwd(q, k, v, la, beta, ckpt, resid if resid.numel() else None,
                                                   do.contiguous(), dS)
     dt = ctx.dtypes
     return (dq.to(dt[0]), dk.to(dt[1]), dv.to(dt[2]), dla.to(dt[3]), dbeta.to(dt[4]) if ctx.has_beta else None,

@@ -1,0 +1,86 @@
+"""GPU parity of the exact scan's chunked form (fp32 operands on the fp32 matrix cores, `aspin_exact` from
+EXACT_CHUNK_MIN_T tokens) at the sizes where its tiles end: chunks of 64 tokens, key and value tiles of 64 in blocks of
+16, 16-byte or 4-byte loads.
+
+Tolerance: every output is a sum of fp32 products along at most T + Dk + Dv <= 1000 terms, so a relative error of a few
+times sqrt(1000) eps = 1.9e-6; 2e-5 in the maximum norm over the result's largest value leaves a factor of ten."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from oracle import aspin as O
+
+pytestmark = pytest.mark.gpu
+
+TOL = 2e-5
+
+
+def _inputs(B, H, T, Dk, Dv, delta, seed, s0, steep=False):
+    g = torch.Generator().manual_seed(seed)
+    q, v = torch.randn(B, H, T, Dk, generator=g), torch.randn(B, H, T, Dv, generator=g)
+    k = F.normalize(torch.randn(B, H, T, Dk, generator=g), dim=-1)
+    la = -torch.rand(B, H, T, generator=g) * 20 if steep else F.logsigmoid(torch.randn(B, H, T, generator=g) + 3.0)
+    x = {"q": q, "k": k, "v": v, "la": la}
+    if delta:
+        x["beta"] = torch.sigmoid(torch.randn(B, H, T, generator=g))
+    if s0:
+        x["S0"] = torch.randn(B, H, Dk, Dv, generator=g) * 0.1
+    return x, torch.randn(B, H, T, Dv, generator=g), torch.randn(B, H, Dk, Dv, generator=g)
+
+
+def _check(x, wo, wS, place=lambda t: t.cuda()):
+    from pragnosia_amd.assoc import assoc_scan
+    r = {n: t.double().requires_grad_(True) for n, t in x.items()}
+    yr, Sr = O.assoc_scan(r["q"], r["k"], r["v"], r["la"], r.get("S0"), chunk=16, beta=r.get("beta"))
+    gr = torch.autograd.grad([yr, Sr], list(r.values()), [wo.double(), wS.double()])
+    d = {n: place(t).requires_grad_(True) for n, t in x.items()}
+    y, S = assoc_scan(d["q"], d["k"], d["v"], d["la"], d.get("S0"), beta=d.get("beta"))
+    gd = torch.autograd.grad([y, S], list(d.values()), [wo.cuda(), wS.cuda()])
+    errs = {}
+    for n, a, b in zip(["o", "S"] + ["d" + n for n in x], [y, S, *gd], [yr, Sr, *gr]):
+        errs[n] = ((a.detach().double().cpu() - b).abs().max() / b.abs().max()).item()
+    assert max(errs.values()) < TOL, errs
+
+
+@pytest.mark.parametrize("delta", [False, True])
+@pytest.mark.parametrize("B,H,T,Dk,Dv,s0", [
+    (1, 1, 32, 16, 16, False),     # half a chunk, one tile
+    (1, 2, 63, 64, 64, True), (1, 2, 64, 64, 64, True), (1, 1, 65, 64, 64, False),   # a chunk's edges
+    (2, 1, 200, 17, 33, True),     # rows that start off 16 bytes: 4-byte loads, partial blocks both ways
+    (1, 1, 129, 100, 20, True),    # 16-byte loads, partial blocks
+    (1, 2, 97, 4, 130, True),      # less than one key block; value tiles past 128
+    (3, 3, 128, 80, 144, True),    # two key tiles a wave, three value tiles; groups past a multiple of 8
+    (1, 1, 70, 192, 176, True), (1, 1, 40, 256, 16, False), (1, 1, 66, 320, 48, True), (1, 1, 90, 384, 24, True),
+])
+def test_chunked_exact_scan_matches_oracle(delta, B, H, T, Dk, Dv, s0):
+    _check(*_inputs(B, H, T, Dk, Dv, delta, seed=T + Dk, s0=s0))
+
+
+def test_chunked_plain_rule_keys_past_384():
+    _check(*_inputs(1, 1, 50, 400, 24, False, seed=7, s0=True))
+
+
+@pytest.mark.parametrize("delta", [False, True])
+def test_chunked_steep_decays_and_resets(delta):
+    """Log-decays down to -20 a token, and -inf (a reset: the state is dropped, no NaN)."""
+    x, wo, wS = _inputs(1, 2, 150, 32, 32, delta, seed=11, s0=True, steep=True)
+    _check(x, wo, wS)
+    from pragnosia_amd.assoc import assoc_scan
+    dev = {n: t.cuda() for n, t in x.items()}
+    dev["la"][:, :, 100] = -float("inf")
+    y, S = assoc_scan(dev["q"], dev["k"], dev["v"], dev["la"], dev["S0"], beta=dev.get("beta"))
+    cut = {n: t[:, :, 100:] for n, t in dev.items() if n != "S0"}
+    cut["la"] = cut["la"].clone()
+    cut["la"][:, :, 0] = 0.0   # no state to decay
+    y2, S2 = assoc_scan(cut["q"], cut["k"], cut["v"], cut["la"], None, beta=cut.get("beta"))
+    assert (y[:, :, 100:] - y2).abs().max() < TOL * y2.abs().max() and (S - S2).abs().max() < TOL * S2.abs().max()
+
+
+@pytest.mark.parametrize("delta", [False, True])
+def test_chunked_off_16_byte_addresses(delta):
+    """Contiguous operands that start 4 bytes past a 16-byte address take the 4-byte loads."""
+    def shifted(t):
+        buf = torch.empty(t.numel() + 1, device="cuda")
+        buf[1:] = t.reshape(-1).cuda()
+        return buf[1:].view(t.shape).detach()
+    _check(*_inputs(1, 2, 100, 64, 48, delta, seed=13, s0=True), place=shifted)
