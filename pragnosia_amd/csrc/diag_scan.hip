@@ -4,13 +4,14 @@
 // The recurrence composes associatively: a segment of tokens acts on its incoming state as the affine map
 // h -> P h + e, P = prod lambda_t (|P| <= 1), e = the segment's own contribution from zero. One workgroup owns
 // CH channels of one sequence (a wave = CH channels x 64/CH time segments; with CH = 64 every load instruction
-// reads one 256-byte row segment of the D-fastest layout) and walks time in blocks of (64/CH) * NW * SEG tokens:
+// reads one 256-byte row segment of the D-fastest layout; fewer channels where there are few sequences, `channels_of`)
+// and walks time in blocks of (64/CH) * NW * SEG tokens:
 //   1. each lane takes its segment (SEG tokens of one channel, loaded during the previous block), forms lambda in
 //      registers, issues the loads of its segment in the next block, and scans the current one from zero, giving
 //      the segment's map (P, e);
-//   2. the maps go to LDS; after one barrier every lane folds the maps of the segments before it into the
-//      block's carry-in to get its own incoming state (reading the maps four at a time, so the LDS latency is paid
-//      once per four segments rather than once per segment);
+//   2. a wave's segments of a channel compose their maps by lane exchanges, and one map a wave goes to LDS; after one
+//      barrier every lane folds the maps of the waves before it into the block's carry-in to get its own incoming state
+//      (reading the maps four at a time, so the LDS latency is paid once per four waves rather than once per wave);
 //   3. the lane re-runs its SEG steps from that state out of registers and writes h.
 // The block carry and the map buffers are double-buffered, so each time block costs one barrier. Nothing is
 // re-read from HBM: the forward moves 20 B per (b, t, d) element, the backward 32 B.
@@ -29,25 +30,67 @@ struct SegMaps {
   float pr, pi, er, ei;
 };
 
-// segment maps folded per batch of LDS reads (swept 1-16 at B16 T512 D768: 4 is fastest, 23.5 -> 21.8 us forward)
+// wave maps folded per batch of LDS reads (swept 1-16 at B16 T512 D768: 4 is fastest, 23.5 -> 21.8 us forward)
 constexpr int kFold = 4;
+constexpr int kComputeUnits = 256;  // MI355X
+
+// `later` after `earlier` (for the backward, in its own direction of time)
+PGN_DEVICE SegMaps after(const SegMaps& later, const SegMaps& earlier) {
+  return SegMaps{later.pr * earlier.pr - later.pi * earlier.pi, later.pi * earlier.pr + later.pr * earlier.pi,
+                 later.pr * earlier.er - later.pi * earlier.ei + later.er,
+                 later.pi * earlier.er + later.pr * earlier.ei + later.ei};
+}
+PGN_DEVICE float2 apply(const SegMaps& m, float2 h) {
+  return make_float2(m.pr * h.x - m.pi * h.y + m.er, m.pi * h.x + m.pr * h.y + m.ei);
+}
+template <bool REV>
+PGN_DEVICE SegMaps shifted(const SegMaps& m, int by) {
+  auto sh = [&](float v) { return REV ? __shfl_down(v, by) : __shfl_up(v, by); };
+  return SegMaps{sh(m.pr), sh(m.pi), sh(m.er), sh(m.ei)};
+}
+
+// A wave's 64 / CH segments of one channel lie CH lanes apart. From each lane's own map: `m` becomes the map of all the
+// wave's segments up to and including the lane's (in the scan's direction), and the result is that of the ones before.
+template <int CH, bool REV>
+PGN_DEVICE SegMaps wave_maps(SegMaps& m, int lane) {
+#pragma unroll
+  for (int by = CH; by < 64; by *= 2) {
+    const SegMaps o = shifted<REV>(m, by);
+    if (REV ? lane + by < 64 : lane >= by) m = after(m, o);
+  }
+  const SegMaps x = shifted<REV>(m, CH);
+  return (REV ? lane + CH < 64 : lane >= CH) ? x : SegMaps{1.f, 0.f, 0.f, 0.f};
+}
+
+// The batch row and first channel of workgroup `idx`, in groups of the 64 / CH workgroups that share 256-byte row
+// segments, each group on one XCD (workgroup i runs on XCD i mod 8) so a line comes into its L2 once.
+struct Tile {
+  int b, d0;
+};
+template <int CH>
+PGN_DEVICE Tile tile_of(int idx, int n64) {
+  constexpr int per = 64 / CH;
+  const int r = idx >> 3, group = (r / per) * 8 + (idx & 7), b = group / n64;
+  return Tile{b, (group - b * n64) * 64 + (r % per) * CH};
+}
 
 template <int NW, int SEG, int CH>
 __global__ __launch_bounds__(NW * 64) void diag_fwd_kernel(
     const float* __restrict__ u, const float* __restrict__ lm, const float* __restrict__ an,
     const float* __restrict__ h0r, const float* __restrict__ h0i, float* __restrict__ hr,
-    float* __restrict__ hi, float* __restrict__ hr_last, float* __restrict__ hi_last, int T, int D, int n_ctile) {
+    float* __restrict__ hi, float* __restrict__ hr_last, float* __restrict__ hi_last, int B, int T, int D, int n64) {
   constexpr int SPW = 64 / CH;  // time segments per wave
   constexpr int NSEG = SPW * NW;
   constexpr int TB = NSEG * SEG;
-  __shared__ SegMaps maps[2][NSEG][CH];
+  __shared__ SegMaps maps[2][NW][CH];
   __shared__ float2 carry[2][CH];
 
-  const int lane = threadIdx.x & 63;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int c = lane % CH;
-  const int seg = SPW * (threadIdx.x >> 6) + lane / CH;
-  const int b = blockIdx.x / n_ctile;
-  const int d = (blockIdx.x - b * n_ctile) * CH + c;
+  const int seg = SPW * wave + lane / CH;
+  const Tile tile = tile_of<CH>(blockIdx.x, n64);
+  if (tile.b >= B || tile.d0 >= D) return;  // grid padding, uniform over the workgroup
+  const int b = tile.b, d = tile.d0 + c;
   const bool dok = d < D;
   const size_t base = (size_t)b * T * D + (dok ? d : 0);
 
@@ -99,26 +142,24 @@ __global__ __launch_bounds__(NW * 64) void diag_fwd_kernel(
       pr = qr;
       pi = qi;
     }
-    maps[p][seg][c] = SegMaps{pr, pi, er, ei};
+    SegMaps own{pr, pi, er, ei}, before;
+    if constexpr (SPW > 1) before = wave_maps<CH, false>(own, lane);
+    if (SPW == 1 || lane >= 64 - CH) maps[p][wave][c] = own;
     __syncthreads();
-    // incoming state: the block carry pushed through every earlier segment's map, the maps read kFold at a time
-    // (reads issued together, one wait per batch rather than one per segment)
+    // incoming state: the block carry pushed through every earlier wave's map, the maps read kFold at a time
+    // (reads issued together, one wait per batch rather than one per wave), then through the wave's own earlier segments
     float2 h = carry[p][c];
 #pragma unroll
-    for (int s0 = 0; s0 < NSEG - 1; s0 += kFold) {
-      if (s0 >= seg) break;  // seg is the wave index (64 channels a wave): a uniform branch
+    for (int s0 = 0; s0 < NW - 1; s0 += kFold) {
+      if (s0 >= wave) break;
       SegMaps m[kFold];
 #pragma unroll
-      for (int r = 0; r < kFold; ++r) m[r] = maps[p][min(s0 + r, NSEG - 1)][c];
+      for (int r = 0; r < kFold; ++r) m[r] = maps[p][min(s0 + r, NW - 1)][c];
 #pragma unroll
-      for (int r = 0; r < kFold; ++r) {
-        if (s0 + r < seg) {
-          const float nr = m[r].pr * h.x - m[r].pi * h.y + m[r].er;
-          const float ni = m[r].pi * h.x + m[r].pr * h.y + m[r].ei;
-          h = make_float2(nr, ni);
-        }
-      }
+      for (int r = 0; r < kFold; ++r)
+        if (s0 + r < wave) h = apply(m[r], h);
     }
+    if constexpr (SPW > 1) h = apply(before, h);
 #pragma unroll
     for (int j = 0; j < SEG; ++j) {
       const float nr = xr[j] * h.x - xi[j] * h.y + xu[j];
@@ -144,18 +185,19 @@ __global__ __launch_bounds__(NW * 64) void diag_bwd_kernel(
     const float* __restrict__ lm, const float* __restrict__ an, const float* __restrict__ hr,
     const float* __restrict__ hi, const float* __restrict__ h0r, const float* __restrict__ h0i,
     float* __restrict__ du, float* __restrict__ dlm, float* __restrict__ dan, float* __restrict__ dh0r,
-    float* __restrict__ dh0i, int T, int D, int n_ctile) {
+    float* __restrict__ dh0i, int B, int T, int D, int n64) {
   constexpr int SPW = 64 / CH;
   constexpr int NSEG = SPW * NW;
   constexpr int TB = NSEG * SEG;
-  __shared__ SegMaps maps[2][NSEG][CH];
+  __shared__ SegMaps maps[2][NW][CH];
   __shared__ float2 carry[2][CH];
 
-  const int lane = threadIdx.x & 63;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int c = lane % CH;
-  const int seg = SPW * (threadIdx.x >> 6) + lane / CH;
-  const int b = blockIdx.x / n_ctile;
-  const int d = (blockIdx.x - b * n_ctile) * CH + c;
+  const int seg = SPW * wave + lane / CH;
+  const Tile tile = tile_of<CH>(blockIdx.x, n64);
+  if (tile.b >= B || tile.d0 >= D) return;  // grid padding, uniform over the workgroup
+  const int b = tile.b, d = tile.d0 + c;
   const bool dok = d < D;
   const size_t base = (size_t)b * T * D + (dok ? d : 0);
   const size_t bd = (size_t)b * D + (dok ? d : 0);
@@ -226,24 +268,22 @@ __global__ __launch_bounds__(NW * 64) void diag_bwd_kernel(
       pr = qr;
       pi = qi;
     }
-    maps[p][seg][c] = SegMaps{pr, pi, er, ei};
+    SegMaps own{pr, pi, er, ei}, before;
+    if constexpr (SPW > 1) before = wave_maps<CH, true>(own, lane);
+    if (SPW == 1 || lane < CH) maps[p][wave][c] = own;
     __syncthreads();
     float2 a = carry[p][c];
 #pragma unroll
-    for (int s0 = NSEG - 1; s0 > 0; s0 -= kFold) {
-      if (s0 <= seg) break;
+    for (int s0 = NW - 1; s0 > 0; s0 -= kFold) {
+      if (s0 <= wave) break;
       SegMaps m[kFold];
 #pragma unroll
       for (int r = 0; r < kFold; ++r) m[r] = maps[p][max(s0 - r, 0)][c];
 #pragma unroll
-      for (int r = 0; r < kFold; ++r) {
-        if (s0 - r > seg) {
-          const float nr = m[r].pr * a.x - m[r].pi * a.y + m[r].er;
-          const float ni = m[r].pi * a.x + m[r].pr * a.y + m[r].ei;
-          a = make_float2(nr, ni);
-        }
-      }
+      for (int r = 0; r < kFold; ++r)
+        if (s0 - r > wave) a = apply(m[r], a);
     }
+    if constexpr (SPW > 1) a = apply(before, a);
 #pragma unroll
     for (int j = SEG - 1; j >= 0; --j) {
       const int t = t0 + j;
@@ -289,9 +329,9 @@ int launch_empty(const float* ar, const float* ai, float* xr, float* xi, int64_t
 template <int NW, int SEG, int CH>
 int launch_fwd(const float* u, const float* lm, const float* an, const float* h0r, const float* h0i, float* hr,
                float* hi, float* hrl, float* hil, int B, int T, int D, hipStream_t st) {
-  const int nct = (D + CH - 1) / CH;
-  hipLaunchKernelGGL((diag_fwd_kernel<NW, SEG, CH>), dim3(B * nct), dim3(NW * 64), 0, st, u, lm, an, h0r, h0i, hr,
-                     hi, hrl, hil, T, D, nct);
+  const int n64 = (D + 63) / 64;
+  hipLaunchKernelGGL((diag_fwd_kernel<NW, SEG, CH>), dim3((B * n64 + 7) / 8 * 8 * (64 / CH)), dim3(NW * 64), 0, st, u,
+                     lm, an, h0r, h0i, hr, hi, hrl, hil, B, T, D, n64);
   PGN_RETURN_LAUNCH();
 }
 
@@ -299,11 +339,36 @@ template <int NW, int SEG, int CH>
 int launch_bwd(const float* g, const float* glr, const float* gli, const float* lm, const float* an,
                const float* hr, const float* hi, const float* h0r, const float* h0i, float* du, float* dlm,
                float* dan, float* dh0r, float* dh0i, int B, int T, int D, hipStream_t st) {
-  const int nct = (D + CH - 1) / CH;
-  hipLaunchKernelGGL((diag_bwd_kernel<NW, SEG, CH>), dim3(B * nct), dim3(NW * 64), 0, st, g, glr, gli, lm, an, hr,
-                     hi, h0r, h0i, du, dlm, dan, dh0r, dh0i, T, D, nct);
+  const int n64 = (D + 63) / 64;
+  hipLaunchKernelGGL((diag_bwd_kernel<NW, SEG, CH>), dim3((B * n64 + 7) / 8 * 8 * (64 / CH)), dim3(NW * 64), 0, st, g,
+                     glr, gli, lm, an, hr, hi, h0r, h0i, du, dlm, dan, dh0r, dh0i, B, T, D, n64);
   PGN_RETURN_LAUNCH();
 }
+
+// Channels a workgroup owns. A time block costs a compute unit the same issue time whatever its shape (4096 elements,
+// about 3.5 us), so with fewer 64-channel tiles than compute units the tiles are narrowed, down to 8 channels, while
+// one round of workgroups still holds them and a block (4096 / CH tokens) is not mostly past the sequence's end.
+// Narrow rows cost coalescing (at 192 tiles of 64, B16 T512 D768: 25 / 34 us forward / backward, 29 / 40 with 16
+// channels), idle units more: B4 T2048 D704, 44 tiles, 64 / 32 / 16 / 8 channels: 62 / 37 / 26 / 32 us forward, 76 / 45 /
+// 34 / 45 backward; B8 T512 D768, 96 tiles: 20 / 15 / 18 / 19 and 24 / 20 / 24 / 27; B1 T8192 D704, 11 tiles: 233 / 129 /
+// 77 / 58 and 287 / 158 / 99 / 79; B12 T512 D704, 132 tiles (264 of 32): 21 / 24 and 27 / 33.
+int channels_of(int64_t B, int64_t T, int64_t D) {
+  const int64_t n64 = B * ((D + 63) / 64);
+  int ch = 64;
+  while (ch > 8 && n64 * (128 / ch) <= kComputeUnits && 8192 / ch < 2 * T) ch /= 2;
+  return ch;
+}
+
+// 16 waves, 4-token segments: swept against 4-16 waves, 32/64 channels and 2-16-token segments at B16 T512 D768; short
+// sequences use 4 waves of 64 channels
+#define PGN_DIAG_DISPATCH(GO)               \
+  if (T < 64) GO(4, 64);                    \
+  switch (channels_of(B, T, D)) {           \
+    case 64: GO(16, 64);                    \
+    case 32: GO(16, 32);                    \
+    case 16: GO(16, 16);                    \
+    default: GO(16, 8);                     \
+  }
 
 bool shape_ok(int64_t B, int64_t T, int64_t D) {
   if (B <= 0 || T < 0 || D <= 0) return false;
@@ -324,11 +389,10 @@ extern "C" int pragnosia_diag_scan_fwd(const float* u, const float* logmag, cons
   hipStream_t st = (hipStream_t)stream;
   if (T == 0) return launch_empty(h0r, h0i, hr_last, hi_last, B * D, st);
   PGN_CHECK_ARG(u && logmag && ang && hr && hi);
-  // 16 waves x 64 channels, 4-token segments (64-token time blocks): swept against 4-16 waves, 32/64 channels and
-  // 2-16-token segments at B16 T512 D768; short sequences use 4 waves
-  if (T >= 64)
-    return launch_fwd<16, 4, 64>(u, logmag, ang, h0r, h0i, hr, hi, hr_last, hi_last, (int)B, (int)T, (int)D, st);
-  return launch_fwd<4, 4, 64>(u, logmag, ang, h0r, h0i, hr, hi, hr_last, hi_last, (int)B, (int)T, (int)D, st);
+#define PGN_DIAG(NW, CH) \
+  return launch_fwd<NW, 4, CH>(u, logmag, ang, h0r, h0i, hr, hi, hr_last, hi_last, (int)B, (int)T, (int)D, st)
+  PGN_DIAG_DISPATCH(PGN_DIAG);
+#undef PGN_DIAG
 }
 
 extern "C" int pragnosia_diag_scan_bwd(const float* g, const float* g_last_r, const float* g_last_i,
@@ -341,9 +405,9 @@ extern "C" int pragnosia_diag_scan_bwd(const float* g, const float* g_last_r, co
   hipStream_t st = (hipStream_t)stream;
   if (T == 0) return launch_empty(g_last_r, g_last_i, dh0r, dh0i, B * D, st);
   PGN_CHECK_ARG(g && logmag && ang && hr && hi && du && dlogmag && dang);
-  if (T >= 64)
-    return launch_bwd<16, 4, 64>(g, g_last_r, g_last_i, logmag, ang, hr, hi, h0r, h0i, du, dlogmag, dang, dh0r, dh0i,
-                                 (int)B, (int)T, (int)D, st);
-  return launch_bwd<4, 4, 64>(g, g_last_r, g_last_i, logmag, ang, hr, hi, h0r, h0i, du, dlogmag, dang, dh0r, dh0i,
-                              (int)B, (int)T, (int)D, st);
+#define PGN_DIAG(NW, CH)                                                                                          \
+  return launch_bwd<NW, 4, CH>(g, g_last_r, g_last_i, logmag, ang, hr, hi, h0r, h0i, du, dlogmag, dang, dh0r, dh0i, \
+                               (int)B, (int)T, (int)D, st)
+  PGN_DIAG_DISPATCH(PGN_DIAG);
+#undef PGN_DIAG
 }
