@@ -310,6 +310,26 @@ int pragnosia_aspin_delta_bwd(const void* q, const void* k, const void* v, const
 int pragnosia_aspin_delta_window_prefix(const float* M, const float* R, const float* S0, const float* theta,
                                         float shift, float* S_in, int64_t BH, int64_t H, int64_t NW, void* stream);
 
+/* The same scan with only the state's recurrence along the chunks, for few heads over many chunks: everything else is
+ * formed for all chunks at once. o may be NULL (the state pass); sent, W and X are required, and everything written is
+ * what pragnosia_aspin_delta_fwd writes. With theta ((H, D / 2) fp32, else NULL) the state is rebased by -window theta
+ * (key-row pairs rotated) after every `window` tokens, a multiple of 64, but the last: carried windows (`src/model.py:
+ * 842-864` over `src/assoc.py:391-405`) in one pass, forward only. */
+int pragnosia_aspin_delta_par_fwd(const void* q, const void* k, const void* v, const float* la, const float* beta,
+                                  const float* S0, void* o, float* S_final, void* sent, void* W, void* X,
+                                  const float* theta, int64_t window, int64_t B, int64_t H, int64_t T, int64_t D,
+                                  int64_t chunk, void* stream);
+
+/* Bytes of the backward's workspace (16-byte aligned), or -1 for a shape it refuses. */
+int64_t pragnosia_aspin_delta_par_bwd_workspace_bytes(int64_t B, int64_t H, int64_t T, int64_t D, int64_t chunk);
+
+/* The backward in the same form, from either forward's sent, W and X: arguments as pragnosia_aspin_delta_bwd. */
+int pragnosia_aspin_delta_par_bwd(const void* q, const void* k, const void* v, const float* la, const float* beta,
+                                  const void* sent, const void* W, const void* X, const void* dO,
+                                  const float* dS_final, void* dq, void* dk, void* dv, float* dla, float* dbeta,
+                                  float* dS0, void* workspace, int64_t workspace_bytes, int64_t B, int64_t H, int64_t T,
+                                  int64_t D, int64_t chunk, void* stream);
+
 /* The R and M state passes above in one launch, head dim 64, chunk 64: N sequences (N = BH NW windows, each a
  * sequence of its own) of T tokens with q, k, v (N, T, 64) bf16, la and beta (N, T) fp32 as for
  * pragnosia_aspin_delta_fwd. RM (2N, 64, 64) fp32 receives R (entries 0 .. N - 1: each sequence's final state from a

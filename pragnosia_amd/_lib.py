@@ -47,6 +47,9 @@ SIGNATURES = {
     "pragnosia_aspin_delta_fwd": [_p] * 11 + [_i64] * 5 + [_p],
     "pragnosia_aspin_delta_bwd_workspace_bytes": [_i64] * 5,
     "pragnosia_aspin_delta_bwd": [_p] * 17 + [_i64] * 6 + [_p],
+    "pragnosia_aspin_delta_par_bwd_workspace_bytes": [_i64] * 5,
+    "pragnosia_aspin_delta_par_fwd": [_p] * 12 + [_i64] * 6 + [_p],
+    "pragnosia_aspin_delta_par_bwd": [_p] * 17 + [_i64] * 6 + [_p],
     "pragnosia_aspin_delta_window_prefix": [_p] * 4 + [_f32, _p] + [_i64] * 3 + [_p],
     "pragnosia_aspin_delta_window_maps": [_p] * 6 + [_i64] * 2 + [_p],
     "pragnosia_aspin_prep_fwd": [_p] * 9 + [_i64] * 5 + [_i32, _p],
@@ -76,7 +79,7 @@ _RET_I64 = {"pragnosia_aspin_delta_bwd_workspace_bytes", "pragnosia_aspin_prep_t
             "pragnosia_aspin_chunk_seg_workspace_bytes", "pragnosia_aspin_out_weight_partials",
             "pragnosia_aspin_prep_proj_partials", "pragnosia_aspin_chunk_wide_workspace_bytes",
             "pragnosia_layer_norm_partials", "pragnosia_wgrad_workspace_bytes",
-            "pragnosia_aspin_exact_chunk_bwd_workspace_bytes"}
+            "pragnosia_aspin_exact_chunk_bwd_workspace_bytes", "pragnosia_aspin_delta_par_bwd_workspace_bytes"}
 
 _lib = None
 

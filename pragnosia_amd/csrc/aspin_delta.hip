@@ -2274,6 +2274,11 @@ bool shape_ok(int64_t B, int64_t H, int64_t T, int64_t D, int64_t Cc) {
   return (D == DK || D == 2 * DK) && Cc == C;
 }
 
+// The chunk-parallel form's grids hold up to eight workgroups a head and two a (head, chunk), padded to sets of 8.
+bool par_shape_ok(int64_t B, int64_t H, int64_t T, int64_t D, int64_t Cc) {
+  return shape_ok(B, H, T, D, Cc) && 2 * B * H * ((T + C - 1) / C) + 16 < ((int64_t)1 << 31);
+}
+
 // ------------------------------------------------------------------------------------------------------------------
 // Carried windows of the delta rule in one pass: the entering state of every window from the windows' affine maps.
 // Given X (keys, decays and strengths only) the rule is independent per value column and linear in the state, so a
@@ -2359,6 +2364,8 @@ __global__ __launch_bounds__(256) void delta_window_prefix(const float* __restri
   if (w + 1 < NW) step(ma, ra, w);
 }
 
+#include "aspin_delta_par.h"
+
 int set_smem(const void* fn, size_t bytes) { return (int)pgn_lds_limit(fn, bytes); }
 
 int64_t align256(int64_t n) { return (n + 255) / 256 * 256; }
@@ -2386,6 +2393,24 @@ struct BwdWorkspace {
     total = dbe1 + B * H * T * 4;
   }
 };
+
+// dq, dk, dla and dbeta of a 128-wide head: the second scan's slots added into the first's
+int join_slots(__bf16* dq, const __bf16* dq1, __bf16* dk, const __bf16* dk1, float* dla, const float* dla1,
+               float* dbeta, const float* dbe1, int64_t rows, int64_t D, hipStream_t st) {
+  DeltaJoin j = {};
+  j.x[0] = dq;
+  j.y[0] = dq1;
+  j.x[1] = dk;
+  j.y[1] = dk1;
+  j.f[0] = dla;
+  j.e[0] = dla1;
+  j.f[1] = dbeta;
+  j.e[1] = dbe1;
+  j.n = rows * D;
+  j.m = rows;
+  hipLaunchKernelGGL(aspin_delta_join, dim3((unsigned)((j.n / 8 + 255) / 256)), dim3(256), 0, st, j);
+  PGN_RETURN_LAUNCH();
+}
 
 template <int KH>
 int delta_fwd(const void* q, const void* k, const void* v, const float* la, const float* beta, const float* S0,
@@ -2455,22 +2480,142 @@ int delta_bwd(const void* q, const void* k, const void* v, const float* la, cons
   if (KH == 1) PGN_RETURN_LAUNCH();
   e = hipGetLastError();
   if (e != hipSuccess) return (int)e;
-  DeltaJoin j = {};
-  j.x[0] = (__bf16*)dq;
-  j.y[0] = dq1;
-  j.x[1] = (__bf16*)dk;
-  j.y[1] = dk1;
-  j.f[0] = dla;
-  j.e[0] = dla1;
-  j.f[1] = dbeta;
-  j.e[1] = dbe1;
-  j.n = B * H * T * 64 * KH;
-  j.m = B * H * T;
-  hipLaunchKernelGGL(aspin_delta_join, dim3((unsigned)((j.n / 8 + 255) / 256)), dim3(256), 0, st, j);
+  return join_slots((__bf16*)dq, dq1, (__bf16*)dk, dk1, dla, dla1, dbeta, dbe1, B * H * T, 64 * KH, st);
+}
+
+// Workspace of the chunk-parallel backward (bytes): Y (drhs after the walk) and F, then what the two-kernel backward
+// passes on (as BwdWorkspace).
+struct ParWorkspace {
+  int64_t y, f, drhs, dsc, rsum, dq1, dk1, dla1, dbe1, total;
+  ParWorkspace(int64_t B, int64_t H, int64_t T, int64_t D) {
+    const int64_t NC = (T + C - 1) / C, KH = D / DK, hc = B * H * NC;
+    y = 0;
+    f = hc * KH * kParVals * 4;
+    drhs = f + hc * KH * kParVals * 4 * KH;
+    dsc = drhs + align256(B * H * T * D * 2);
+    rsum = dsc + align256(hc * D * D * 2);
+    total = rsum + align256(B * H * KH * T * 2 * 4);
+    dq1 = dk1 = dla1 = dbe1 = -1;
+    if (KH == 1) return;
+    dq1 = total;
+    dk1 = dq1 + align256(B * H * T * D * 2);
+    dla1 = dk1 + align256(B * H * T * D * 2);
+    dbe1 = dla1 + align256(B * H * T * 4);
+    total = dbe1 + align256(B * H * T * 4);
+  }
+};
+
+#define PGN_LAUNCHED()                       \
+  do {                                       \
+    const hipError_t e_ = hipGetLastError(); \
+    if (e_ != hipSuccess) return (int)e_;    \
+  } while (0)
+
+template <int KH>
+int delta_par_fwd(const __bf16* q, const __bf16* k, const __bf16* v, const float* la, const float* beta,
+                  const float* S0, __bf16* o, float* S_final, __bf16* sent, __bf16* W, __bf16* X, const float* theta,
+                  int window, int64_t B, int64_t H, int64_t T, hipStream_t st) {
+  const int NC = (int)((T + C - 1) / C), heads = (int)(B * H), hc = heads * NC;
+  constexpr size_t lds = walk_lds<KH, false>();
+  hipLaunchKernelGGL(aspin_delta_inv<KH>, dim3((unsigned)hc), dim3(256), 0, st, k, la, beta, X, (int)T, NC);
+  PGN_LAUNCHED();
+  const dim3 grid(sub_grid(heads, 4 * KH));
+  if (KH == 1 && theta != nullptr) {
+    const int rc = set_smem((const void*)delta_walk<1, true>, lds);
+    if (rc) return rc;
+    hipLaunchKernelGGL((delta_walk<1, true>), grid, dim3(320), lds, st, k, v, la, beta, X, S0, W, sent, S_final, theta,
+                       (float)window, window / C, (int)H, (int)T, NC, heads);
+  } else {
+    const int rc = set_smem((const void*)delta_walk<KH, false>, lds);
+    if (rc) return rc;
+    hipLaunchKernelGGL((delta_walk<KH, false>), grid, dim3(320), lds, st, k, v, la, beta, X, S0, W, sent, S_final,
+                       nullptr, 0.f, 1, (int)H, (int)T, NC, heads);
+  }
+  PGN_LAUNCHED();
+  if (o == nullptr) return PRAGNOSIA_OK;
+  const int rc = set_smem((const void*)delta_out<KH>, out_smem<KH>());
+  if (rc) return rc;
+  hipLaunchKernelGGL(delta_out<KH>, dim3(sub_grid(hc, KH)), dim3(256), out_smem<KH>(), st, q, k, la, W, sent, o, (int)T,
+                     NC, hc);
   PGN_RETURN_LAUNCH();
 }
 
+template <int KH>
+int delta_par_bwd(const __bf16* q, const __bf16* k, const __bf16* v, const float* la, const float* beta,
+                  const __bf16* sent, const __bf16* W, const __bf16* X, const __bf16* dO, const float* dS_final,
+                  __bf16* dq, __bf16* dk, __bf16* dv, float* dla, float* dbeta, float* dS0, unsigned char* ws, int64_t B,
+                  int64_t H, int64_t T, hipStream_t st) {
+  const int NC = (int)((T + C - 1) / C), heads = (int)(B * H), hc = heads * NC, scans = heads * KH;
+  constexpr size_t lds = walk_lds<KH, true>();
+  const ParWorkspace L(B, H, T, 64 * KH);
+  float *y = (float*)(ws + L.y), *F = (float*)(ws + L.f), *rs = (float*)(ws + L.rsum);
+  __bf16 *drhs = (__bf16*)(ws + L.drhs), *dsc = (__bf16*)(ws + L.dsc);
+  __bf16 *dq1 = KH == 2 ? (__bf16*)(ws + L.dq1) : nullptr, *dk1 = KH == 2 ? (__bf16*)(ws + L.dk1) : nullptr;
+  float *dla1 = KH == 2 ? (float*)(ws + L.dla1) : nullptr, *dbe1 = KH == 2 ? (float*)(ws + L.dbe1) : nullptr;
+  int rc = set_smem((const void*)delta_bwd_pre<KH>, bwd_pre_smem<KH>());
+  if (!rc) rc = set_smem((const void*)delta_bwd_walk<KH>, lds);
+  if (!rc) rc = set_smem((const void*)aspin_delta_bwd_local<KH>, local_smem<KH>());
+  if (rc) return rc;
+  hipLaunchKernelGGL(delta_bwd_pre<KH>, dim3((unsigned)hc), dim3(256), bwd_pre_smem<KH>(), st, q, k, la, dO, y, F, (int)T,
+                     NC);
+  PGN_LAUNCHED();
+  hipLaunchKernelGGL(delta_bwd_walk<KH>, dim3(sub_grid(heads, 4 * KH)), dim3(320), lds, st, k, la, beta, X, y, F,
+                     dS_final, dsc, dS0, (int)T, NC, heads);
+  PGN_LAUNCHED();
+  hipLaunchKernelGGL(delta_bwd_rsum<KH>, dim3(sub_grid(hc, KH)), dim3(256), 0, st, k, v, la, beta, sent, y, drhs, rs,
+                     (int)T, NC, hc);
+  PGN_LAUNCHED();
+  hipLaunchKernelGGL(aspin_delta_bwd_local<KH>, dim3((unsigned)(scans * NC)), dim3(512), local_smem<KH>(), st, q, k, la,
+                     beta, W, sent, dO, drhs, dsc, rs, dq, dq1, dk, dk1, dv, dla, dla1, dbeta, dbe1, (int)T, NC);
+  PGN_LAUNCHED();
+  if constexpr (KH == 2) return join_slots(dq, dq1, dk, dk1, dla, dla1, dbeta, dbe1, B * H * T, 64 * KH, st);
+  return PRAGNOSIA_OK;
+}
+
 }  // namespace
+
+extern "C" int64_t pragnosia_aspin_delta_par_bwd_workspace_bytes(int64_t B, int64_t H, int64_t T, int64_t D,
+                                                                 int64_t chunk) {
+  if (!par_shape_ok(B, H, T, D, chunk)) return -1;
+  return ParWorkspace(B, H, T, D).total;
+}
+
+extern "C" int pragnosia_aspin_delta_par_fwd(const void* q, const void* k, const void* v, const float* la,
+                                             const float* beta, const float* S0, void* o, float* S_final, void* sent,
+                                             void* W, void* X, const float* theta, int64_t window, int64_t B,
+                                             int64_t H, int64_t T, int64_t D, int64_t chunk, void* stream) {
+  if ((D != DK && D != 2 * DK) || chunk != C) return PRAGNOSIA_ERR_UNSUPPORTED;
+  PGN_CHECK_ARG(par_shape_ok(B, H, T, D, chunk));
+  PGN_CHECK_ARG(q && k && v && la && beta && S_final && sent && W && X);
+  PGN_CHECK_ARG(theta == nullptr || (D == DK && window > 0 && window % C == 0 && window < ((int64_t)1 << 28)));
+#define PGN_PAR(KH)                                                                                                  \
+  return delta_par_fwd<KH>((const __bf16*)q, (const __bf16*)k, (const __bf16*)v, la, beta, S0, (__bf16*)o, S_final, \
+                           (__bf16*)sent, (__bf16*)W, (__bf16*)X, theta, (int)window, B, H, T,                      \
+                           (hipStream_t)stream)
+  if (D == DK) PGN_PAR(1);
+  PGN_PAR(2);
+#undef PGN_PAR
+}
+
+extern "C" int pragnosia_aspin_delta_par_bwd(const void* q, const void* k, const void* v, const float* la,
+                                             const float* beta, const void* sent, const void* W, const void* X,
+                                             const void* dO, const float* dS_final, void* dq, void* dk, void* dv,
+                                             float* dla, float* dbeta, float* dS0, void* workspace,
+                                             int64_t workspace_bytes, int64_t B, int64_t H, int64_t T, int64_t D,
+                                             int64_t chunk, void* stream) {
+  if ((D != DK && D != 2 * DK) || chunk != C) return PRAGNOSIA_ERR_UNSUPPORTED;
+  PGN_CHECK_ARG(par_shape_ok(B, H, T, D, chunk));
+  PGN_CHECK_ARG(q && k && v && la && beta && sent && W && X && dO && dq && dk && dv && dla && dbeta && workspace);
+  PGN_CHECK_ARG(workspace_bytes >= ParWorkspace(B, H, T, D).total);
+#define PGN_PAR(KH)                                                                                               \
+  return delta_par_bwd<KH>((const __bf16*)q, (const __bf16*)k, (const __bf16*)v, la, beta, (const __bf16*)sent,   \
+                           (const __bf16*)W, (const __bf16*)X, (const __bf16*)dO, dS_final, (__bf16*)dq,          \
+                           (__bf16*)dk, (__bf16*)dv, dla, dbeta, dS0, (unsigned char*)workspace, B, H, T,         \
+                           (hipStream_t)stream)
+  if (D == DK) PGN_PAR(1);
+  PGN_PAR(2);
+#undef PGN_PAR
+}
 
 extern "C" int64_t pragnosia_aspin_delta_bwd_workspace_bytes(int64_t B, int64_t H, int64_t T, int64_t D,
                                                              int64_t chunk) {

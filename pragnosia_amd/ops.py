@@ -707,6 +707,38 @@ aspin_chunk_wide.register_autograd(_wide_backward, setup_context=_aspin_setup)
 
 # ---------------------------------------------------------------------------------------------------------------
 # aspin chunked scan, delta rule: replaces delta_scan_kernel and its ops, src/assoc_kernel.py:332-704
+def delta_parallel(heads: int, NC: int, D: int, backward: bool) -> bool:
+    """Whether the scan of `heads` sequences of NC chunks runs with only the state's recurrence along the chunks
+    (`pragnosia_aspin_delta_par_fwd` / `_bwd`: the same results) instead of one workgroup a scan. It spreads a scan's walk
+    over four workgroups and its other work over all chunks, which pays while one round of workgroups holds the walks and
+    there are chunks enough to cover its extra launches. us, one workgroup a scan / this form, forward and backward,
+    heads x chunks at head dim 64: 12 x 2 13/15, 14/19; 12 x 3 16/16, 19/20; 60 x 4 20/19, 25/27; 33 x 8 31/24, 44/33;
+    44 x 32 105/55, 161/82; 24 x 128 392/137, 627/215; past 64 heads 72 x 8 32/39, 45/51; 66 x 16 57/53, 84/76; 96 x 32
+    106/98, 163/187; 192 x 16 62/91, 87/176. At head dim 128: 6 x 4 19/20, 27/30; 6 x 6 24/21, 34/32; 30 x 8 31/31, 55/57;
+    24 x 32 94/67, 168/144; 12 x 64 173/97, 264/177; 36 x 16 55/68, 108/129."""
+    if D == 64:
+        return heads <= (96 if NC >= 16 and not backward else 64) and NC >= (5 if backward else 4)
+    return heads <= (24 if backward else 32) and NC >= (8 if backward else 6)
+
+
+def _delta_par_fwd(q: Tensor, k: Tensor, v: Tensor, la: Tensor, beta: Tensor, S0: Optional[Tensor], want_o: bool,
+                   theta: Optional[Tensor] = None,
+                   window: int = 0) -> tuple[Optional[Tensor], Tensor, Tensor, Tensor, Tensor]:
+    """The chunk-parallel delta forward (inputs already cast): (o or None, S_final, sent, W, X); with theta, the state
+    rebased by -window theta between windows of `window` tokens."""
+    B, H, T, D = q.shape
+    NC = (T + CHUNK - 1) // CHUNK
+    b = lambda *s: torch.empty(*s, device=q.device, dtype=torch.bfloat16)
+    o = b(B, H, T, D) if want_o else None
+    S = torch.empty(B, H, D, D, device=q.device, dtype=torch.float32)
+    sent, W, X = b(B, H, NC, D, D), b(B, H, T, D), b(B, H, NC, CHUNK, CHUNK)
+    check(lib().pragnosia_aspin_delta_par_fwd(_ptr(q), _ptr(k), _ptr(v), _ptr(la), _ptr(beta), _ptr(S0), _ptr(o),
+                                              _ptr(S), _ptr(sent), _ptr(W), _ptr(X), _ptr(theta), window, B, H,
+                                              T, D, CHUNK, _stream(q)),
+          "pragnosia_aspin_delta_par_fwd")
+    return o, S, sent, W, X
+
+
 @torch.library.custom_op("pragnosia::aspin_delta", mutates_args=())
 def aspin_delta(q: Tensor, k: Tensor, v: Tensor, la: Tensor, beta: Tensor, S0: Optional[Tensor],
                 want_sent: bool) -> tuple[Tensor, Tensor, Tensor, Tensor, Tensor]:
@@ -722,6 +754,9 @@ def aspin_delta(q: Tensor, k: Tensor, v: Tensor, la: Tensor, beta: Tensor, S0: O
     B, H, T, D = q.shape
     NC = (T + CHUNK - 1) // CHUNK
     dev = q.device
+    if delta_parallel(B * H, NC, D, False):
+        o, S, sent, W, X = _delta_par_fwd(q, k, v, la, beta, S0, True)
+        return o, S, (sent if want_sent else q.new_empty(0, dtype=torch.bfloat16)), W, X
     o = torch.empty(B, H, T, D, device=dev, dtype=torch.bfloat16)
     S = torch.empty(B, H, D, D, device=dev, dtype=torch.float32)
     sent = (torch.empty(B, H, NC, D, D, device=dev, dtype=torch.bfloat16) if want_sent
@@ -761,6 +796,16 @@ def aspin_delta_bwd(q: Tensor, k: Tensor, v: Tensor, la: Tensor, beta: Tensor, s
     dla = torch.empty(B, H, T, device=dev, dtype=torch.float32)
     dbeta = torch.empty(B, H, T, device=dev, dtype=torch.float32)
     dS0 = torch.empty(B, H, D, D, device=dev, dtype=torch.float32)
+    if delta_parallel(B * H, NC, D, True):
+        nbytes = lib().pragnosia_aspin_delta_par_bwd_workspace_bytes(B, H, T, D, CHUNK)
+        if nbytes < 0:
+            raise PragnosiaError(f"aspin_delta_bwd: shape {tuple(q.shape)} rejected")
+        ws = torch.empty(nbytes, device=dev, dtype=torch.uint8)
+        check(lib().pragnosia_aspin_delta_par_bwd(_ptr(q), _ptr(k), _ptr(v), _ptr(la), _ptr(beta), _ptr(sent), _ptr(W),
+                                                  _ptr(X), _ptr(do), _ptr(dS), _ptr(dq), _ptr(dk), _ptr(dv),
+                                                  _ptr(dla), _ptr(dbeta), _ptr(dS0), _ptr(ws), ws.numel(), B, H, T, D,
+                                                  CHUNK, _stream(q)), "pragnosia_aspin_delta_par_bwd")
+        return dq, dk, dv, dla, dbeta, dS0
     nbytes = lib().pragnosia_aspin_delta_bwd_workspace_bytes(B, H, T, D, CHUNK)
     if nbytes < 0:
         raise PragnosiaError(f"aspin_delta_bwd: shape {tuple(q.shape)} rejected")
@@ -811,6 +856,9 @@ def _delta_pass(q: Tensor, k: Tensor, v: Tensor, la: Tensor, beta: Tensor, S0: O
     B, H, T, D = q.shape
     NC = (T + CHUNK - 1) // CHUNK
     dev = q.device
+    if delta_parallel(B * H, NC, D, False):
+        o, S, sent, W, X = _delta_par_fwd(q, k, v, la, beta, S0, want_o)
+        return (o, S, sent, W, X) if want_saved else (o, S, None, None, None)
     o = torch.empty(B, H, T, D, device=dev, dtype=torch.bfloat16) if want_o else None
     S = torch.empty(B, H, D, D, device=dev, dtype=torch.float32)
     sent = W = X = None
@@ -852,13 +900,9 @@ def aspin_delta_windows(q: Tensor, k: Tensor, v: Tensor, la: Tensor, beta: Tenso
     """Forward only. The delta-rule scan over consecutive windows of `window` tokens (a multiple of 64) whose q and k
     were rotated with positions restarting at 0 in every window, the state carried across window boundaries and
     rebased by -window * theta there: what aspin_delta over each window in turn, with aspin_rebase between, computes
-    (the reference's carried windows, `src/model.py:842-864` over `src/assoc.py:391-405`), with every window at once.
-    Given X the rule is linear in the state and independent per value column, so each window maps its entering state
-    affinely, S_out = M S_in + R: the state passes over all windows (R from zero entering states; M from identity
-    states with zero values) in one launch (`pragnosia_aspin_delta_window_maps`), the entering states chained by
-    `pragnosia_aspin_delta_window_prefix`, then one pass with outputs from the true entering states. A partial last window runs zero-padded (zero keys, values, decay and
-    strength leave the state unchanged). Head dim 64. S0 enters the first window. Returns (o bf16, S after the last
-    window fp32, in its positions)."""
+    (the reference's carried windows, `src/model.py:842-864` over `src/assoc.py:391-405`), in one pass that rebases the
+    state as it walks past each window (`pragnosia_aspin_delta_par_fwd`). Head dim 64. S0 enters the first window. Returns
+    (o bf16, S after the last window fp32, in its positions)."""
     _require_gpu(q, k, v, la, beta, S0, theta)
     _expect_scan("aspin_delta_windows", q, k, v, la, beta=beta, S0=S0, theta=theta)
     if window <= 0 or window % CHUNK:
@@ -866,25 +910,8 @@ def aspin_delta_windows(q: Tensor, k: Tensor, v: Tensor, la: Tensor, beta: Tenso
     if q.shape[-1] != 64:
         raise PragnosiaError(f"aspin_delta_windows: head dim {q.shape[-1]}; the window maps are built for 64")
     q, k, v, la, beta, S0, theta = _bf16(q), _bf16(k), _bf16(v), _f32(la), _f32(beta), _f32(S0), _f32(theta)
-    B, H, T, D = q.shape
-    NW = (T + window - 1) // window
-    Tp = NW * window
-    if Tp != T:
-        pad = lambda t: F.pad(t, (0, 0, 0, Tp - T)) if t.dim() == 4 else F.pad(t, (0, Tp - T))
-        q, k, v, la, beta = (pad(t) for t in (q, k, v, la, beta))
-    BW = B * H * NW  # every window of every (batch, head) a sequence of its own: contiguous views
-    qw, kw, vw = (t.view(BW, 1, window, D) for t in (q, k, v))
-    lw, bw = la.view(BW, 1, window), beta.view(BW, 1, window)
-    RM = torch.empty(2, BW, D, D, device=q.device, dtype=torch.float32)  # R, then M: both state passes, one launch
-    check(lib().pragnosia_aspin_delta_window_maps(_ptr(qw), _ptr(kw), _ptr(vw), _ptr(lw), _ptr(bw), _ptr(RM), BW, window,
-                                                  _stream(q)), "pragnosia_aspin_delta_window_maps")
-    Sin = torch.empty(BW, 1, D, D, device=q.device, dtype=torch.float32)
-    check(lib().pragnosia_aspin_delta_window_prefix(_ptr(RM[1]), _ptr(RM[0]), _ptr(S0), _ptr(theta), float(window),
-                                                    _ptr(Sin), B * H, H, NW, _stream(q)),
-          "pragnosia_aspin_delta_window_prefix")
-    o, Sf, _, _, _ = _delta_pass(qw, kw, vw, lw, bw, Sin, True, False)
-    o = o.view(B, H, Tp, D)[:, :, :T]
-    return (o if Tp == T else o.contiguous()), Sf.view(B, H, NW, D, D)[:, :, -1].contiguous()
+    o, S, _, _, _ = _delta_par_fwd(q, k, v, la, beta, S0, True, theta, window)
+    return o, S
 
 
 @aspin_delta_windows.register_fake
