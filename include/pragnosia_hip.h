@@ -387,8 +387,8 @@ int pragnosia_aspin_prep_proj_fwd(const void* P, int64_t stride, int64_t la_col,
 int64_t pragnosia_aspin_prep_proj_partials(int64_t B, int64_t T, int64_t H);
 
 /* Backward of pragnosia_aspin_prep_proj_fwd: from dq, dk, dv ((B, H, T, D) bf16), dla and (with beta_col >= 0) dbeta
- * ((B, H, T) fp32) writes the q, k, v, decay and gate or strength columns of dP (P's layout, stride and dtype; other
- * columns untouched), theta's partials (as pragnosia_aspin_prep_bwd) and `part`:
+ * ((B, H, T) fp32) writes the q, k, v, decay and gate or strength columns of dP (P's layout, stride and dtype) and
+ * zeroes those past the last of them, and theta's partials (as pragnosia_aspin_prep_bwd) and `part`:
  * pragnosia_aspin_prep_proj_partials(B, T, H) rows, row (b H + h) ntb + j holding (d gate_bias[h] or
  * d beta_bias[h], d la_bias[h], dA[h]) partial sums (ntb = ceil(T / 64)); the caller sums them per head. */
 int pragnosia_aspin_prep_proj_bwd(const void* P, int64_t stride, int64_t la_col, int64_t gate_col, int64_t beta_col,

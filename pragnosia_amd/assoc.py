@@ -41,6 +41,12 @@ FUSED_PROJ = False
 FUSED_PLUMBING = True
 
 HEAD_DIM_KERNEL = 64
+# The fused projection's rows (3 d + 2 h: 2134 for d 704) padded with zero rows to a multiple of this, so its output's
+# and its gradient's rows are 128-byte aligned: off alignment the GEMMs around them slow down, and the weight gradient
+# leaves its kernel (widths a multiple of 8). us at 8192 tokens, unpadded / padded, forward, input and weight gradient:
+# d 704 (2134 / 2176) 47 / 44, 49 / 39, 74 / 49; d 384 (1164 / 1216) 22 / 22, 22 / 18, 52 / 26; d 768 (2328 / 2368) 45 /
+# 45, 42 / 36, 55 / 55.
+PROJ_ALIGN = 64
 _POS_CACHE: dict = {}
 
 
@@ -352,6 +358,8 @@ class AssocCarrier(nn.Module):
                 and getattr(self, "beta_scale", None) is None and getattr(self, "sconv", None) is None):
             gated = not (self.delta or self.write_all)
             extra = [self.wi.weight] if gated else ([self.wb.weight] if self.delta else [])
+            if extra and (pad := -(3 * self.d + 2 * self.h) % PROJ_ALIGN):
+                extra.append(self.wa.weight.new_zeros(pad, self.d))
             W = torch.cat([self.q.weight, self.k.weight, self.v.weight, self.wa.weight] + extra)
             P = _op_mod.linear_w(z, W)
             q, k, v, la, beta = _op.aspin_prep_proj(
@@ -379,6 +387,13 @@ class AssocCarrier(nn.Module):
             eps = self.on.eps if self.on.eps is not None else _op_mod.RMS_EPS
             return _op.aspin_out(o, self.on.weight, eps, dtype == torch.bfloat16)[0]
         return self.on(o.to(dtype)).transpose(1, 2).reshape(B, T, H * Dk)
+
+    def _gated_out(self, o):
+        """sigmoid(gate) W_o o without autograd: the gate on whichever is smaller, the d x d weight or the tokens' output
+        (at 16384 tokens of 768 under autocast, a pass of 40 us over the output becomes one of 5 over the weight)."""
+        if o.numel() > self.o.weight.numel():
+            return F.linear(o, self.o.weight * torch.sigmoid(self.gate))
+        return F.linear(o, self.o.weight) * torch.sigmoid(self.gate)
 
     def forward(self, x, h0=None, pos0: int = 0):
         """x (B, T, d); h0 = (S (B, H, dk, dk), p0) from a previous call, (S, p0, cache) with the short convolution, or
@@ -456,8 +471,7 @@ class AssocCarrier(nn.Module):
             Wg = self.o.weight * torch.sigmoid(self.gate)
             out = x + (_op_mod.linear_w(o, Wg) if FUSED_PLUMBING else F.linear(o, Wg))
         else:
-            # the same function without materialising a gated d x d weight on every call (decode, inference)
-            out = x + F.linear(o, self.o.weight) * torch.sigmoid(self.gate)
+            out = x + self._gated_out(o)
         # the state is now expressed in this call's positions 0..T-1: the next call rebases it by T
         p_out = p0 * 0 + T if torch.is_tensor(p0) else T
         return out, ((S, p_out, cc) if sc else (S, p_out))
@@ -498,7 +512,7 @@ class AssocCarrier(nn.Module):
             o, S, _ = _op.aspin_chunk_windows(q, k, v, la, S0, self.theta, window, False)
         self.sent = None
         o = self._epilogue(o, dtype)
-        out = x + F.linear(o, self.o.weight) * torch.sigmoid(self.gate)
+        out = x + self._gated_out(o)
         last = T - window * ((T - 1) // window)
         return out, (S, p0 * 0 + last if torch.is_tensor(p0) else last)
 

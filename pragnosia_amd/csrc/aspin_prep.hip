@@ -171,7 +171,8 @@ __global__ __launch_bounds__(256) void prep_fwd(const In* __restrict__ qp, const
 // projections' gradient (dcol = the gradient buffer, same layout and stride): dlogit_a = dla mask (-exp(A))
 // sigmoid(logit_a + b) (mask: the floor not active), dlogit_g = dsig sig (1 - sig), dlogit_b = dbeta mask sig (1 -
 // sig) (mask: bmin not active); and one partial per workgroup of the three per-head sums (d gbias or d bbias,
-// d abias, dA = sum dla mask la) to part, laid out (B, T blocks, H, 3) like the theta partials.
+// d abias, dA = sum dla mask la) to part, laid out (B, T blocks, H, 3) like the theta partials. Columns `used` .. S - 1
+// of the gradient's rows (a projection padded for aligned rows) are zeroed.
 template <typename In, int D>
 __global__ __launch_bounds__(256) void prep_bwd(
     const In* __restrict__ qp, const In* __restrict__ kp, const In* __restrict__ vp, const float* __restrict__ gl,
@@ -179,7 +180,7 @@ __global__ __launch_bounds__(256) void prep_bwd(
     const __bf16* __restrict__ dk, const __bf16* __restrict__ dv, In* __restrict__ dqp, In* __restrict__ dkp,
     In* __restrict__ dvp, float* __restrict__ dgl, float* __restrict__ dth, int T, int H, int ntb, int64_t S,
     Cols<In> cols, const float* __restrict__ dla, const float* __restrict__ dbeta, In* __restrict__ dcol,
-    float* __restrict__ part) {
+    float* __restrict__ part, int64_t used) {
   constexpr int LANES = RowSplit<D>::LANES, SLOTS = RowSplit<D>::SLOTS;
   __shared__ float red[SLOTS][D / 2];
   __shared__ float red3[SLOTS][3];
@@ -198,6 +199,8 @@ __global__ __launch_bounds__(256) void prep_bwd(
     if (t >= T) break;
     const size_t row = ((size_t)b * T + t) * S;
     const size_t in = row + h * D + 8 * j;
+    if (h == H - 1)  // the row's padding, by the last head's lanes
+      for (int64_t c = used + j; c < S; c += LANES) dcol[row + c] = (In)0.f;
     if (cols.acol && j == 0) {
       const float x = (float)cols.acol[row + h] + cols.abias[h];
       const float l = -softplusf_(x) * eA;
@@ -415,10 +418,10 @@ template <typename In, int D>
 void launch_prep_bwd(dim3 grid, hipStream_t st, const In* qp, const In* kp, const In* vp, const float* gate,
                      const float* theta, const int64_t* pos, const void* dq, const void* dk, const void* dv, In* dqp,
                      In* dkp, In* dvp, float* dgate, float* dth, int T, int H, int ntb, int64_t stride, Cols<In> cols,
-                     const float* dla, const float* dbeta, In* dcol, float* part) {
+                     const float* dla, const float* dbeta, In* dcol, float* part, int64_t used) {
   hipLaunchKernelGGL((prep_bwd<In, D>), grid, dim3(256), 0, st, qp, kp, vp, gate, theta, pos, (const __bf16*)dq,
                      (const __bf16*)dk, (const __bf16*)dv, dqp, dkp, dvp, dgate, dth, T, H, ntb, stride, cols, dla,
-                     dbeta, dcol, part);
+                     dbeta, dcol, part, used);
 }
 
 template <typename In>
@@ -435,13 +438,13 @@ template <typename In>
 void prep_bwd_any(int64_t Dh, dim3 grid, hipStream_t st, const In* qp, const In* kp, const In* vp, const float* gate,
                   const float* theta, const int64_t* pos, const void* dq, const void* dk, const void* dv, In* dqp,
                   In* dkp, In* dvp, float* dgate, float* dth, int T, int H, int ntb, int64_t stride, Cols<In> cols,
-                  const float* dla, const float* dbeta, In* dcol, float* part) {
+                  const float* dla, const float* dbeta, In* dcol, float* part, int64_t used) {
   if (Dh == 64)
     launch_prep_bwd<In, 64>(grid, st, qp, kp, vp, gate, theta, pos, dq, dk, dv, dqp, dkp, dvp, dgate, dth, T, H, ntb,
-                            stride, cols, dla, dbeta, dcol, part);
+                            stride, cols, dla, dbeta, dcol, part, used);
   else
     launch_prep_bwd<In, 128>(grid, st, qp, kp, vp, gate, theta, pos, dq, dk, dv, dqp, dkp, dvp, dgate, dth, T, H,
-                             ntb, stride, cols, dla, dbeta, dcol, part);
+                             ntb, stride, cols, dla, dbeta, dcol, part, used);
 }
 
 }  // namespace
@@ -483,11 +486,11 @@ extern "C" int pragnosia_aspin_prep_bwd(const void* qp, const void* kp, const vo
   if (in_bf16)
     prep_bwd_any<__bf16>(Dh, grid, st, (const __bf16*)qp, (const __bf16*)kp, (const __bf16*)vp, gate, theta, pos, dq,
                          dk, dv, (__bf16*)dqp, (__bf16*)dkp, (__bf16*)dvp, dgate, dtheta_partial, (int)T, (int)H, ntb,
-                         in_stride, Cols<__bf16>{}, nullptr, nullptr, nullptr, nullptr);
+                         in_stride, Cols<__bf16>{}, nullptr, nullptr, nullptr, nullptr, in_stride);
   else
     prep_bwd_any<float>(Dh, grid, st, (const float*)qp, (const float*)kp, (const float*)vp, gate, theta, pos, dq, dk,
                         dv, (float*)dqp, (float*)dkp, (float*)dvp, dgate, dtheta_partial, (int)T, (int)H, ntb,
-                        in_stride, Cols<float>{}, nullptr, nullptr, nullptr, nullptr);
+                        in_stride, Cols<float>{}, nullptr, nullptr, nullptr, nullptr, in_stride);
   PGN_RETURN_LAUNCH();
 }
 
@@ -563,6 +566,7 @@ extern "C" int pragnosia_aspin_prep_proj_bwd(const void* P, int64_t stride, int6
   PGN_CHECK_ARG(P && la_bias && A && theta && pos && dq && dk && dv && dla && dP && dtheta_partial && part);
   PGN_CHECK_ARG(beta_col < 0 || dbeta);
   PGN_CHECK_ARG(proj_cols_ok(H, Dh, stride, la_col, gate_col, beta_col) && P != dP);
+  const int64_t used = (la_col > gate_col ? (la_col > beta_col ? la_col : beta_col) : gate_col) + H;
   const int ntb = (int)((T + TB - 1) / TB);
   const dim3 grid((unsigned)(B * H * ntb));
   const int64_t hd = H * Dh;
@@ -574,7 +578,7 @@ extern "C" int pragnosia_aspin_prep_proj_bwd(const void* P, int64_t stride, int6
                          nullptr, dtheta_partial, (int)T, (int)H, ntb, stride,
                          proj_cols<__bf16>(P, la_col, gate_col, beta_col, la_bias, A, la_floor, gate_bias, beta_bias,
                                            beta_min),
-                         dla, dbeta, d, part);
+                         dla, dbeta, d, part, used);
   } else {
     const float* p = (const float*)P;
     float* d = (float*)dP;
@@ -582,7 +586,7 @@ extern "C" int pragnosia_aspin_prep_proj_bwd(const void* P, int64_t stride, int6
                         nullptr, dtheta_partial, (int)T, (int)H, ntb, stride,
                         proj_cols<float>(P, la_col, gate_col, beta_col, la_bias, A, la_floor, gate_bias, beta_bias,
                                          beta_min),
-                        dla, dbeta, d, part);
+                        dla, dbeta, d, part, used);
   }
   PGN_RETURN_LAUNCH();
 }

@@ -1348,9 +1348,7 @@ def aspin_prep_proj_bwd(P: Tensor, H: int, la_bias: Tensor, A: Tensor, la_floor:
     has_beta = not gated and W > 3 * H * D + H
     if has_beta:
         dbeta = torch.zeros(B, H, T, device=P.device) if dbeta is None else _f32(dbeta)
-    dP = torch.empty_like(P)
-    if W > 3 * H * D + (2 if (gated or has_beta) else 1) * H:
-        dP.zero_()  # columns the kernel does not write
+    dP = torch.empty_like(P)  # the kernel zeroes the columns past the last group
     rows = lib().pragnosia_aspin_prep_theta_partials(B, T)
     dth = torch.empty(rows, H, D // 2, device=P.device, dtype=torch.float32)
     part = torch.empty(lib().pragnosia_aspin_prep_proj_partials(B, T, H), 3, device=P.device, dtype=torch.float32)
