@@ -494,6 +494,16 @@ int pragnosia_decode_tail(const float* logits, int64_t B, int64_t V, const float
                           int64_t* pos_out, int64_t* out, int64_t n_rows, int64_t* tok, float* h, float* p0s,
                           int64_t L, float* logits_rec, void* stream);
 
+/* Dense layers' weights as pragnosia_decode_gemm reads them. The table has n layers of PRAGNOSIA_FOLD_ENTRIES int64: five
+ * row blocks' addresses ((rows, K) fp32), the five running row counts (a block may be empty), K, col_scale, its length G,
+ * ln_bias, bias, Wt, csum, bias_out, and the layer's first workgroup (the sum of ceil(N / 16) over the layers before). A
+ * layer's blocks are stacked to N rows and tiled into Wt (ceil(N / 16) 16 K floats, rows past N zero), the columns
+ * scaled by col_scale ((G,) repeated over K, G a multiple of 4 dividing K; or 0); if non-zero, csum (N): the scaled
+ * rows' sums, and bias_out (N): bias (or 0) plus W ln_bias (ln_bias (K) or 0), both summed in fp64. K a multiple of 16;
+ * blocks, col_scale, ln_bias and Wt 16-byte aligned. `table` is read on the host, `device_table` is its copy. */
+#define PRAGNOSIA_FOLD_ENTRIES 19
+int pragnosia_decode_fold(const int64_t* table, const int64_t* device_table, int64_t n, void* stream);
+
 /* The dense layers of the decode step on the fp32 matrix cores, for batches past the GEMV's (any B; 16 rows a
  * workgroup): y (B, N) = act(scale * (W z) + bias) + resid, with z = x (mode 0); z = (x - mean) / sqrt(var + eps) over
  * each row (mode 1: a LayerNorm whose weight is folded into W's columns, W[n][k] ln_weight[k], and whose bias into

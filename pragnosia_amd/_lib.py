@@ -68,6 +68,7 @@ SIGNATURES = {
     "pragnosia_decode_gemv": [_p, _i64, _i64, _p, _p, _f32, _p, _i64, _p, _p, _i32, _p, _p, _p],
     "pragnosia_decode_gemv_rms": [_p, _i64, _i64, _p, _i64, _f32, _p, _i64, _p, _p, _i32, _p, _p, _p],
     "pragnosia_decode_tail": [_p, _i64, _i64, _p, _p, _i64, _i64] + [_p] * 5 + [_i64, _p, _p, _p, _i64, _p, _p],
+    "pragnosia_decode_fold": [_p, _p, _i64, _p],
     "pragnosia_decode_gemm_waves": [_i64, _i32],
     "pragnosia_decode_gemm": [_p, _i64, _i64, _i32, _p, _f32, _p, _i64, _p, _p, _i32, _p, _p, _p],
     "pragnosia_decode_gemm_acc": [_p, _i64, _i64, _i32, _f32, _p, _i64, _p, _p, _p, _p],

@@ -24,7 +24,7 @@ import torch
 import torch.nn.functional as F
 
 from .assoc import AssocCarrier
-from .ops import decode_gemm_ln, decode_gemm_ok, decode_gemm_tile, decode_tail, ln_supported
+from .ops import DecodeFold, decode_gemm_ok, decode_tail, ln_supported
 
 
 # The fused step's dense layers run as the batched GEMV kernel (each weight read once a step) up to this many
@@ -128,6 +128,25 @@ class GreedyDecoder:
                 out.append(tuple(t.clone().contiguous() for t in st))
         return out
 
+    def _load_states(self, states):
+        """The prefilled states into the static buffers. The fused step reads the positions from `p0s` only; given as
+        numbers they go there in one copy."""
+        if not self.fused:
+            for dst, src in zip(self.st, states):
+                for a, b in zip(dst, src):
+                    if torch.is_tensor(b):
+                        a.copy_(b)
+                    else:
+                        a.fill_(float(b))
+            return
+        torch._foreach_copy_([st[0] for st in self.st], [st[0] for st in states])
+        pos = [st[1] for st in states]
+        if any(torch.is_tensor(p) for p in pos):
+            pos = [p if torch.is_tensor(p) else torch.tensor(float(p)) for p in pos]
+            self.p0s.copy_(torch.stack([p.reshape(()).to(self.p0s) for p in pos]))
+        else:
+            self.p0s.copy_(torch.tensor([float(p) for p in pos]))
+
     def _one_step(self, par=0):
         m = self.m
         h = m.e(self.tok) + m.p(self.pos)
@@ -155,36 +174,50 @@ class GreedyDecoder:
 
     def _fused_weights(self):
         """Per layer: the concatenated input projection (q, k, v, decay, then the gate or strength), the output gate
-        sigmoid(g) as a device scalar and the output projection pre-scaled by it (for the GEMM form), written into
-        the same buffers every time (the graph reads them). On the decode_gemm path, instead of the GEMM form: each
-        dense layer's weight tiled, its input LayerNorm's (or the carrier's RMSNorm's) weight folded into the tiled
-        columns, the LayerNorm's bias into the layer's bias, with the folded weights' row sums."""
-        m = self.m
-        fresh = []
-        for mx, mp in zip(m.mix, m.mlp):
+        sigmoid(g) as a device scalar and, where the o-projection runs as torch's GEMM, its weight pre-scaled by it,
+        written into the same buffers every time (the graph reads them). On the decode_gemm path instead: each dense
+        layer's weight tiled, its input LayerNorm's (or the carrier's RMSNorm's) weight folded into the tiled columns,
+        the LayerNorm's bias into the layer's bias, with the folded weights' row sums (DecodeFold)."""
+        m, dev = self.m, self.m.e.weight.device
+        parts = []
+        for mx in m.mix:
             gated = not (mx.delta or mx.write_all)
             extra = [mx.wi.weight] if gated else ([mx.wb.weight] if mx.delta else [])
-            sig = torch.sigmoid(mx.gate.detach().float()).reshape(1)
-            wcat = torch.cat([mx.q.weight, mx.k.weight, mx.v.weight, mx.wa.weight] + extra).detach().float()
-            if self.gemm:
-                tp, cp, bp = decode_gemm_ln(wcat, mx.ln.weight, mx.ln.bias, None)
-                ta, ca, ba = decode_gemm_ln(mp.a.weight, mp.n.weight, mp.n.bias, mp.a.bias)
-                fresh.append((tp, cp, bp, sig, decode_gemm_tile(mx.o.weight, mx.on.weight), ta, ca, ba,
-                              decode_gemm_tile(mp.b.weight)))
-            else:
-                fresh.append((wcat, sig, mx.o.weight.detach().float() * sig))
-        if self.gemm:
-            fresh.append(decode_gemm_ln(m.e.weight, m.n.weight, m.n.bias, None))
+            parts.append([mx.q.weight, mx.k.weight, mx.v.weight, mx.wa.weight] + extra)
+        rows = lambda ws: sum(w.shape[0] for w in ws)
         if getattr(self, "wbuf", None) is None:
-            self.wbuf = [tuple(t.contiguous() for t in f) for f in fresh]
-        else:
-            for dst, src in zip(self.wbuf, fresh):
-                for d, t in zip(dst, src):
-                    d.copy_(t)
+            e = lambda *s: torch.empty(*s, device=dev, dtype=torch.float32)
+            tile = lambda ws: e((rows(ws) + 15) // 16 * 16 * ws[0].shape[1])
+            ln = lambda ws: (tile(ws), e(rows(ws)), e(rows(ws)))
+            self.gates = e(len(m.mix))
+            self.sig = [self.gates[i:i + 1] for i in range(len(m.mix))]
+            if self.gemm:
+                self.wbuf = [(*ln(ws), sig, tile([mx.o.weight]), *ln([mp.a.weight]), tile([mp.b.weight]))
+                             for ws, sig, mx, mp in zip(parts, self.sig, m.mix, m.mlp)] + [ln([m.e.weight])]
+            else:
+                self.wbuf = [e(rows(ws), ws[0].shape[1]) for ws in parts]
+                self.wcat = self.wbuf
+                self.wos = [e(*mx.o.weight.shape) if self.B > GEMV_MAX_BATCH else None for mx in m.mix]
+        torch.sigmoid(torch.stack([mx.gate.detach().float().reshape(()) for mx in m.mix]), out=self.gates)
         if not self.gemm:
-            self.wcat = [f[0] for f in self.wbuf]
-            self.sig = [f[1] for f in self.wbuf]
-            self.wos = [f[2] for f in self.wbuf]
+            for ws, dst, wos, sig, mx in zip(parts, self.wbuf, self.wos, self.sig, m.mix):
+                if dst.shape != (rows(ws), ws[0].shape[1]):  # out= would move the buffer the graph reads
+                    raise ValueError("GreedyDecoder: the model's projection widths changed since the capture")
+                torch.cat([w.detach().float() for w in ws], out=dst)
+                if wos is not None:
+                    torch.mul(mx.o.weight.detach().float(), sig, out=wos)
+            return
+        src = []
+        for ws, mx, mp in zip(parts, m.mix, m.mlp):
+            src += [(ws, mx.ln.weight, mx.ln.bias, None), ([mx.o.weight], mx.on.weight, None, None),
+                    ([mp.a.weight], mp.n.weight, mp.n.bias, mp.a.bias), ([mp.b.weight], None, None, None)]
+        src.append(([m.e.weight], m.n.weight, m.n.bias, None))
+        if getattr(self, "fold", None) is None:
+            dst = []
+            for tp, cp, bp, _, to, ta, ca, ba, tb in self.wbuf[:-1]:
+                dst += [(tp, cp, bp), (to, None, None), (ta, ca, ba), (tb, None, None)]
+            self.fold = DecodeFold(src, dst + [self.wbuf[-1]])
+        self.fold.run(src)
 
     def _dense(self, x, W, ln, bias=None, scale=None, act=0, resid=None):
         """act(scale * (W LayerNorm(x)) + bias) + resid: the batched GEMV kernel up to GEMV_MAX_BATCH sequences,
@@ -329,12 +362,9 @@ class GreedyDecoder:
         """Load a prefilled state into the static buffers (capturing the graph on first use)."""
         if self.graph is None or n > self.n_max:
             self._capture(states, n)
-        for a_, b_ in zip(self.st, self._static_states(states)):
-            for a, b in zip(a_, b_):
-                a.copy_(b)
+        self._load_states(states)
         if self.fused:
             self._fused_weights()
-            self.p0s.copy_(torch.stack([st[1].reshape(()) for st in self.st]).float())
         self.pos.fill_(pw)
         first = lg.argmax(-1)
         self.out.zero_()

@@ -1584,6 +1584,58 @@ def decode_gemm_ln(W: Tensor, ln_weight: Tensor, ln_bias: Optional[Tensor], bias
     return decode_gemm_tile(Wf), csum, b.float()
 
 
+class DecodeFold:
+    """`decode_gemm_tile` / `decode_gemm_ln` of many layers in one kernel, into given buffers
+    (`pragnosia_decode_fold`). A layer's source is (row blocks, column scale or None, LayerNorm bias or None, bias or
+    None), its destination (Wt, row sums or None, folded bias or None). `run` takes the sources' tensors as they are
+    at that time; they must have the shapes that `sources` had here, on the destinations' device."""
+
+    def __init__(self, sources, dests):
+        self.dests, self.device = dests, dests[0][0].device
+        self.shapes, self.rows, wg = [], [], 0
+        for (ws, cs, lb, bias), (Wt, csum, bout) in zip(sources, dests):
+            K, N, G = ws[0].shape[1], sum(w.shape[0] for w in ws), 0 if cs is None else cs.numel()
+            _require_gpu(*ws, cs, lb, bias, Wt, csum, bout)
+            _expect("decode_fold", self.device, Wt=(Wt, ((N + 15) // 16 * 16 * K,)), csum=(csum, (N,)),
+                    bias_out=(bout, (N,)), col_scale=(cs, (None,)), ln_bias=(lb, (K,)), bias=(bias, (N,)),
+                    **{f"w{i}": (w, (None, K)) for i, w in enumerate(ws)})
+            if len(ws) > 5 or K % 16 or (G and (G % 4 or K % G)):
+                raise PragnosiaError(f"decode_fold: {len(ws)} blocks of width {K}, column scale of {G}")
+            if any(t is not None and (t.dtype != torch.float32 or not t.is_contiguous()) for t in (Wt, csum, bout)):
+                raise PragnosiaError("decode_fold: the destinations must be contiguous fp32")
+            ends = [sum(w.shape[0] for w in ws[:i + 1]) for i in range(5)]
+            self.shapes.append([None if t is None else t.shape for t in (*ws, cs, lb, bias)])
+            self.rows.append([0] * 5 + ends + [K, 0, G, 0, 0]
+                             + [0 if t is None else t.data_ptr() for t in (Wt, csum, bout)] + [wg])
+            wg += (N + 15) // 16
+
+    def _source(self, t: Optional[Tensor], shape) -> Optional[Tensor]:
+        """`t` as the kernel reads it (fp32, contiguous, 16-byte aligned), its shape and device checked."""
+        if t is None and shape is None:
+            return None
+        if t is None or t.shape != shape or t.device != self.device:
+            raise PragnosiaError(f"decode_fold: got {None if t is None else (tuple(t.shape), str(t.device))}, expected "
+                                 f"{shape and tuple(shape)} on {self.device}")
+        t = _f32(t.detach())
+        return t if t.data_ptr() % 16 == 0 else t.clone()
+
+    def run(self, sources) -> None:
+        if len(sources) != len(self.rows):
+            raise PragnosiaError(f"decode_fold: {len(sources)} layers, expected {len(self.rows)}")
+        kept, table = [], []  # the sources as read live until the launch: the table holds addresses only
+        for row, shapes, (ws, cs, lb, bias) in zip(self.rows, self.shapes, sources):
+            if len(ws) != len(shapes) - 3:
+                raise PragnosiaError(f"decode_fold: {len(ws)} row blocks, expected {len(shapes) - 3}")
+            ts = [self._source(t, shape) for t, shape in zip((*ws, cs, lb, bias), shapes)]
+            at = [0 if t is None else t.data_ptr() for t in ts]
+            n = len(ws)
+            kept.append(ts)
+            table.append(at[:n] + row[n:11] + [at[n], row[12], at[n + 1], at[n + 2]] + row[15:])
+        host = torch.tensor(table, dtype=torch.int64)
+        dev = host.to(self.device)
+        check(lib().pragnosia_decode_fold(_ptr(host), _ptr(dev), len(table), _stream(dev)), "pragnosia_decode_fold")
+
+
 def decode_gemm_ok(K: int, mode: int) -> bool:
     """Whether `decode_gemm` covers a dense layer of input width K in this mode."""
     return lib().pragnosia_decode_gemm_waves(K, mode) > 0
