@@ -46,6 +46,41 @@ struct StepIn {
 
 PGN_DEVICE float softplus_(float x) { return x > 20.f ? x : log1pf(__expf(x)); }
 
+// The step's per-head scalars as read (FROM_P form). Each is read whether it is there or not (an absent one from the
+// projection's row) and selected when used: behind branches the loads ran one after another, five to eight memory
+// round trips a step (32 sequences, 12 heads of 64: 5.98 us a layer, now 5.34; launch 1.75, the states' 12.6 MB 2.6).
+struct StepScalars {
+  float p0, la, la_b, A, fl, g, g_b, be, be_b;
+  // every load has been waited for past this point
+  PGN_DEVICE void arrived() const {
+    asm volatile("" ::"s"(p0), "s"(la), "s"(la_b), "s"(A), "s"(fl), "s"(g), "s"(g_b), "s"(be), "s"(be_b));
+  }
+  PGN_DEVICE float p0_of(const float* p0d, float p0h) const { return p0d ? p0 : p0h; }
+  PGN_DEVICE float decay(const StepIn& in) const {
+    return __expf(fmaxf(-softplus_(la + la_b) * __expf(A), in.floor ? fl : -INFINITY));
+  }
+  PGN_DEVICE float gate(const StepIn& in) const { return 1.f / (1.f + __expf(-(g + (in.gate_b ? g_b : 0.f)))); }
+  PGN_DEVICE float strength(const StepIn& in) const {
+    return fmaxf(1.f / (1.f + __expf(-(be + (in.beta_b ? be_b : 0.f)))), in.beta_min);
+  }
+};
+
+PGN_DEVICE StepScalars step_scalars(const StepIn& in, const float* prow, int h, const float* __restrict__ p0d) {
+  const float* la = prow + in.la_col + h;
+  auto at = [&](const float* p) { return p ? p + h : la; };
+  StepScalars s;
+  s.p0 = *(p0d ? p0d : la);
+  s.la = *la;
+  s.la_b = in.la_b[h];
+  s.A = in.A[h];
+  s.fl = *at(in.floor);
+  s.g = prow[(in.gate_col >= 0 ? in.gate_col : in.la_col) + h];
+  s.g_b = *at(in.gate_b);
+  s.be = prow[(in.beta_col >= 0 ? in.beta_col : in.la_col) + h];
+  s.be_b = *at(in.beta_b);
+  return s;
+}
+
 // With `on` (the per-head RMSNorm weight), the output is written normalised and token-major, o[b][h 64 + j] =
 // (o_j r) on_j with r = 1 / sqrt(mean_j o_j^2 + eps) (nn.RMSNorm(dk), eps=None: fp32 epsilon; `src/assoc.py:505`);
 // else o (B, H, 64) as computed. S and Sout may be the same array (the in-place update of the graphed decode), so
@@ -96,8 +131,7 @@ __global__ __launch_bounds__(256) void aspin_decode(const float* S, float* Sout,
     else
       x = (rg == 0 ? in.qp : (rg == 1 ? in.kp : in.vp))[voff + j];
     float n = x * x;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) n += __shfl_xor(n, off);
+    n = group_sum<64>(n);
     float inv = 1.f / fmaxf(sqrtf(n), 1e-12f);
     if (rg == 1 && has_g) inv *= 1.f / (1.f + __expf(-gl_v));
     (rg == 0 ? qs : (rg == 1 ? ks : vs))[j] = x * inv;
@@ -138,8 +172,7 @@ __global__ __launch_bounds__(256) void aspin_decode(const float* S, float* Sout,
     const float ov = red[0][j] + red[1][j] + red[2][j] + red[3][j];
     if (on) {
       float ss = ov * ov;
-#pragma unroll
-      for (int off = 1; off < 64; off <<= 1) ss += __shfl_xor(ss, off);
+      ss = group_sum<64>(ss);
       const float rr = 1.f / sqrtf(ss * (1.f / D) + on_eps);
       o[(size_t)b * H * D + h * D + j] = (ov * rr) * on[j];
     } else {
@@ -151,49 +184,47 @@ __global__ __launch_bounds__(256) void aspin_decode(const float* S, float* Sout,
 // The step for D = 64 or 128 with the work of a head split over D / 16 parts of 16 value columns (for latency: a
 // one-token step is short, and D / 16 workgroups per head fill the chip at small batches): thread (jj, rg) of part
 // `part` owns column 16 part + jj and key rows (D / 16) rg .. (D / 16) rg + D / 16 - 1 (D / 32 rotation pairs), holding
-// them in x (loaded by the caller first, so their latency overlaps what follows) and ending with the new state there.
+// them in x and ending with the new state there. Loads are counted in order, so those needed first are issued first:
+// the projections and the per-head scalars, then what `load_state` reads (x, and whatever else the caller needs).
 // `nt` is the thread's index within its part (the first 192 of a part's 256 threads normalise q, k and v; `norm`
 // selects the part that does), red the part's 16 x 17 LDS block. Returns the thread's share of output column j (the
 // sum over its rows of S_new[d][j] q[d]; the part's 16 row groups are added by the caller, red[.][jj] in order).
 // Every thread of the workgroup calls this (barriers inside).
-template <int DH>
+template <int DH, class Load>
 PGN_DEVICE float split_step(float (&x)[DH / 16], const StepIn& in, const float* __restrict__ theta,
                             const float* __restrict__ p0d, float p0h, int H, int b, int h, int part, int nt,
-                            bool norm, float* qs, float* ks, float* vs, float (*red)[17]) {
+                            bool norm, float* qs, float* ks, float* vs, float (*red)[17], Load load_state) {
   constexpr int RT = DH / 16;  // key rows per thread
   const int jj = nt & 15, rg = nt >> 4;
   const int j = 16 * part + jj;
   const float* prow = in.P + (size_t)b * in.np;
-  float th[RT / 2];
-#pragma unroll
-  for (int pr = 0; pr < RT / 2; ++pr) th[pr] = theta[h * (DH / 2) + (RT / 2) * rg + pr];
-  const float p0 = p0d ? *p0d : p0h;
-  const float la_logit = prow[in.la_col + h], la_b = in.la_b[h], Ah = in.A[h];
-  const float fl = in.floor ? in.floor[h] : -INFINITY;
-  const bool has_g = in.gate_col >= 0, has_b = in.beta_col >= 0;
-  const float gl = has_g ? prow[in.gate_col + h] + (in.gate_b ? in.gate_b[h] : 0.f) : 0.f;
-  const float bl = has_b ? prow[in.beta_col + h] + (in.beta_b ? in.beta_b[h] : 0.f) : 0.f;
   // q, k, v unit-normalised (k also gated) by waves 0, 1, 2, D / 64 channels a lane
   constexpr int CL = DH / 64;
-  float xin[CL];
+  const int vec = min(nt >> 6, 2), l = nt & 63;
+  float xin[CL], th[RT / 2];
+#pragma unroll
+  for (int e = 0; e < CL; ++e) xin[e] = prow[vec * H * DH + h * DH + 64 * e + l];
+  const StepScalars sc = step_scalars(in, prow, h, p0d);
+#pragma unroll
+  for (int pr = 0; pr < RT / 2; ++pr) th[pr] = theta[h * (DH / 2) + (RT / 2) * rg + pr];
+  load_state();
+  __builtin_amdgcn_sched_barrier(0);
+  float n = 0.f;
+#pragma unroll
+  for (int e = 0; e < CL; ++e) n += xin[e] * xin[e];
+  n = group_sum<64>(n);
+  float inv = 1.f / fmaxf(sqrtf(n), 1e-12f);
+  sc.arrived();
+  const bool has_g = in.gate_col >= 0, has_b = in.beta_col >= 0;
+  const float p0 = sc.p0_of(p0d, p0h);
+  if (vec == 1 && has_g) inv *= sc.gate(in);
   if (norm && nt < 3 * 64) {
-    const int vec = nt >> 6, l = nt & 63;
-#pragma unroll
-    for (int e = 0; e < CL; ++e) xin[e] = prow[vec * H * DH + h * DH + 64 * e + l];
-    float n = 0.f;
-#pragma unroll
-    for (int e = 0; e < CL; ++e) n += xin[e] * xin[e];
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) n += __shfl_xor(n, off);
-    float inv = 1.f / fmaxf(sqrtf(n), 1e-12f);
-    if (vec == 1 && has_g) inv *= 1.f / (1.f + __expf(-gl));
     float* dst = vec == 0 ? qs : (vec == 1 ? ks : vs);
 #pragma unroll
     for (int e = 0; e < CL; ++e) dst[64 * e + l] = xin[e] * inv;
   }
-  const float la_v = fmaxf(-softplus_(la_logit + la_b) * __expf(Ah), fl);
-  const float a = __expf(la_v);
-  const float be_v = has_b ? fmaxf(1.f / (1.f + __expf(-bl)), in.beta_min) : 0.f;
+  const float a = sc.decay(in);
+  const float be_v = has_b ? sc.strength(in) : 0.f;
 #pragma unroll
   for (int pr = 0; pr < RT / 2; ++pr) {
     float sn, cs;
@@ -246,9 +277,10 @@ __global__ __launch_bounds__(256) void aspin_decode_split(const float* S, float*
   const int j = 16 * part + jj;
   const float* Sbh = S + (size_t)bh * DH * DH;
   float x[RT];
+  const float y = split_step<DH>(x, in, theta, p0d, p0h, H, b, h, part, tid, true, qs, ks, vs, red, [&] {
 #pragma unroll
-  for (int r = 0; r < RT; ++r) x[r] = Sbh[(RT * rg + r) * DH + j];
-  const float y = split_step<DH>(x, in, theta, p0d, p0h, H, b, h, part, tid, true, qs, ks, vs, red);
+    for (int r = 0; r < RT; ++r) x[r] = Sbh[(RT * rg + r) * DH + j];
+  });
   red[rg][jj] = y;
   float* Sob = Sout + (size_t)bh * DH * DH;
 #pragma unroll
@@ -290,12 +322,18 @@ __global__ __launch_bounds__(1024) void aspin_decode_oproj(const float* __restri
   const int j = 16 * part + jj;
   const float* Sbh = S + (size_t)bh * D * D;
   float x[RT];
-#pragma unroll
-  for (int r = 0; r < RT; ++r) x[r] = Sbh[(RT * rg + r) * D + j];
   // row n0 + tid / 16 of W_o, input columns 64 h + 4 (tid & 15) .. + 3 (rows past N read row N - 1, not added)
   const int n = slice * kOprojRows + (tid >> 4), c4 = tid & 15;
-  const f32x4 w4 = *reinterpret_cast<const f32x4*>(Wo + (size_t)min(n, N - 1) * (H * D) + h * D + 4 * c4);
-  const float yp = split_step<D>(x, in, theta, p0d, p0h, H, b, h, part, nt, part == 0, qs, ks, vs, red[part]);
+  f32x4 w4;
+  float onv, so;
+  const float yp = split_step<D>(x, in, theta, p0d, p0h, H, b, h, part, nt, part == 0, qs, ks, vs, red[part], [&] {
+#pragma unroll
+    for (int r = 0; r < RT; ++r) x[r] = Sbh[(RT * rg + r) * D + j];
+    w4 = *reinterpret_cast<const f32x4*>(Wo + (size_t)min(n, N - 1) * (H * D) + h * D + 4 * c4);
+    onv = on[tid & 63];
+    so = *(scale ? scale : theta);
+  });
+  asm volatile("" ::"v"(onv), "s"(so), "s"(y));  // loaded by now, not where they are used
   red[part][rg][jj] = yp;
   if (slice == 0) {
     float* Sob = Sout + (size_t)bh * D * D;
@@ -309,17 +347,15 @@ __global__ __launch_bounds__(1024) void aspin_decode_oproj(const float* __restri
 #pragma unroll
     for (int g = 0; g < 16; ++g) ov += rp[g][tid & 15];
     float ss = ov * ov;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) ss += __shfl_xor(ss, off);
+    ss = group_sum<64>(ss);
     const float rr = 1.f / sqrtf(ss * (1.f / D) + on_eps);
-    onrm[tid] = (ov * rr) * on[tid];
+    onrm[tid] = (ov * rr) * onv;
   }
   __syncthreads();
   const f32x4 o4 = *reinterpret_cast<const f32x4*>(onrm + 4 * c4);
   float acc = (w4[0] * o4[0] + w4[1] * o4[1]) + (w4[2] * o4[2] + w4[3] * o4[3]);
-#pragma unroll
-  for (int off = 1; off < 16; off <<= 1) acc += __shfl_xor(acc, off);
-  if (c4 == 0 && n < N) atomicAdd(y + (size_t)b * N + n, (scale ? *scale : 1.f) * acc);
+  acc = group_sum<16>(acc);
+  if (c4 == 0 && n < N) atomicAdd(y + (size_t)b * N + n, (scale ? so : 1.f) * acc);
 }
 
 // The step for many heads (large batches), raw output, D = 64 or 128: one workgroup per (batch, head) and 16-byte
@@ -340,37 +376,36 @@ __global__ __launch_bounds__(256) void aspin_decode_vec(const float* S, float* S
   const int tid = threadIdx.x, cq = tid % CQ, rg = tid / CQ, w = tid >> 6, l = tid & 63;
   const float* prow = in.P + (size_t)b * in.np;
   const float* Sbh = S + (size_t)bh * DH * DH + 4 * cq;
-  f32x4 x[RPT];
-#pragma unroll
-  for (int r = 0; r < RPT; ++r) x[r] = *reinterpret_cast<const f32x4*>(Sbh + (size_t)(RPT * rg + r) * DH);
-  float th[RPT / 2];
-#pragma unroll
-  for (int pr = 0; pr < RPT / 2; ++pr) th[pr] = theta[h * (DH / 2) + (RPT / 2) * rg + pr];
-  const float p0 = p0d ? *p0d : p0h;
-  const float la_logit = prow[in.la_col + h], la_b = in.la_b[h], Ah = in.A[h];
-  const float fl = in.floor ? in.floor[h] : -INFINITY;
-  const bool has_g = in.gate_col >= 0, has_b = in.beta_col >= 0;
-  const float gl = has_g ? prow[in.gate_col + h] + (in.gate_b ? in.gate_b[h] : 0.f) : 0.f;
-  const float bl = has_b ? prow[in.beta_col + h] + (in.beta_b ? in.beta_b[h] : 0.f) : 0.f;
+  // loads are counted in order: the projections and the per-head scalars, which the step needs first, then the state.
   // q, k, v unit-normalised (k also gated) by waves 0, 1, 2, D / 64 channels a lane
   constexpr int CL = DH / 64;
+  const int vec = min(w, 2);
+  f32x4 x[RPT];
+  float xin[CL], th[RPT / 2];
+#pragma unroll
+  for (int e = 0; e < CL; ++e) xin[e] = prow[vec * H * DH + h * DH + 64 * e + l];
+  const StepScalars sc = step_scalars(in, prow, h, p0d);
+#pragma unroll
+  for (int pr = 0; pr < RPT / 2; ++pr) th[pr] = theta[h * (DH / 2) + (RPT / 2) * rg + pr];
+#pragma unroll
+  for (int r = 0; r < RPT; ++r) x[r] = *reinterpret_cast<const f32x4*>(Sbh + (size_t)(RPT * rg + r) * DH);
+  __builtin_amdgcn_sched_barrier(0);
+  float n = 0.f;
+#pragma unroll
+  for (int e = 0; e < CL; ++e) n += xin[e] * xin[e];
+  n = group_sum<64>(n);
+  float inv = 1.f / fmaxf(sqrtf(n), 1e-12f);
+  sc.arrived();
+  const bool has_g = in.gate_col >= 0, has_b = in.beta_col >= 0;
+  const float p0 = sc.p0_of(p0d, p0h);
+  if (vec == 1 && has_g) inv *= sc.gate(in);
   if (w < 3) {
-    float xin[CL];
-#pragma unroll
-    for (int e = 0; e < CL; ++e) xin[e] = prow[w * H * DH + h * DH + 64 * e + l];
-    float n = 0.f;
-#pragma unroll
-    for (int e = 0; e < CL; ++e) n += xin[e] * xin[e];
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) n += __shfl_xor(n, off);
-    float inv = 1.f / fmaxf(sqrtf(n), 1e-12f);
-    if (w == 1 && has_g) inv *= 1.f / (1.f + __expf(-gl));
     float* dst = w == 0 ? qs : (w == 1 ? ks : vs);
 #pragma unroll
     for (int e = 0; e < CL; ++e) dst[64 * e + l] = xin[e] * inv;
   }
-  const float a = __expf(fmaxf(-softplus_(la_logit + la_b) * __expf(Ah), fl));
-  const float be_v = has_b ? fmaxf(1.f / (1.f + __expf(-bl)), in.beta_min) : 0.f;
+  const float a = sc.decay(in);
+  const float be_v = has_b ? sc.strength(in) : 0.f;
 #pragma unroll
   for (int pr = 0; pr < RPT / 2; ++pr) {
     float sn, cs;
@@ -383,9 +418,10 @@ __global__ __launch_bounds__(256) void aspin_decode_vec(const float* S, float* S
   // the sum over the wave's row groups (lane bits above the column quad), then over the four waves
   auto wave_rows = [&](f32x4 v) {
 #pragma unroll
-    for (int off = CQ; off < 64; off <<= 1)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] += __shfl_xor(v[e], off);
+    for (int e = 0; e < 4; ++e) {
+      if constexpr (CQ == 16) v[e] = swap_add<16>(v[e], v[e]);
+      v[e] = swap_add<32>(v[e], v[e]);
+    }
     return v;
   };
   f32x4 wv = *reinterpret_cast<const f32x4*>(vs + 4 * cq);

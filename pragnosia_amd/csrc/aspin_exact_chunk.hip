@@ -820,10 +820,8 @@ __global__ __launch_bounds__(256) void exact_scores_bwd(const float* __restrict_
       if (DELTA) cf += F[(4 * e + m) * PR + r];
     }
     float d = row - cl;
-    d += __shfl_xor(d, 1);
-    d += __shfl_xor(d, 2);
-    cf += __shfl_xor(cf, 1);
-    cf += __shfl_xor(cf, 2);
+    d = group_sum<4>(d);
+    cf = group_sum<4>(cf);
     if (m == 0) {
       rc[ch * CT + r] = d;
       if (DELTA) db[ch * CT + r] = -cf;

@@ -21,9 +21,8 @@ constexpr int TB = 64;    // tokens per workgroup
 // sum over the L lanes that share a row (lane bits 0 .. log2 L - 1)
 template <int L>
 PGN_DEVICE float sum_lanes(float x) {
-#pragma unroll
-  for (int o = 1; o < L; o <<= 1) x += __shfl_xor(x, o);
-  return x;
+  x = group_sum<16>(x);
+  return L == 32 ? x + __shfl_xor(x, 16) : x;  // the last pass may leave half a wave, which the row swap does not take
 }
 
 PGN_DEVICE f32x4 load4(const __bf16* p) {

@@ -84,9 +84,7 @@ PGN_DEVICE void st8<__bf16>(__bf16* p, const float* x) {
 // sum over the L lanes that share a row (lane bits 0 .. log2 L - 1)
 template <int L>
 PGN_DEVICE float sum_row(float x) {
-#pragma unroll
-  for (int o = 1; o < L; o <<= 1) x += __shfl_xor(x, o);
-  return x;
+  return group_sum<L>(x);
 }
 
 template <int L>

@@ -107,25 +107,72 @@ PGN_DEVICE float pgn_exp(float x) { return __expf(x); }
 // GELU, erf form (torch's default F.gelu): 0.5 x (1 + erf(x / sqrt 2)).
 PGN_DEVICE float pgn_gelu_erf(float x) { return 0.5f * x * (1.f + erff(x * 0.70710678118654752f)); }
 
+// Lane exchanges in the vector unit: DPP row operations within a row of 16 lanes, v_permlane16_swap and
+// v_permlane32_swap across rows. __shfl_xor goes through the LDS permute unit, a wait of about 100 cycles a step where
+// these take a few cycles, and a decode layer's LayerNorm + GEMV runs three 64-lane sums in series.
+template <int CTRL>
+PGN_DEVICE float dpp_move(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true));
+}
+
+// With O = 16 or 32 and bit O of the lane number clear: a of the lane plus a of the lane O above; set: b of the lane
+// plus b of the lane O below (the swap leaves a's lower and b's lower halves in one register, the upper in the other).
+template <int O>
+PGN_DEVICE float swap_add(float a, float b) {
+  static_assert(O == 16 || O == 32, "");
+  const unsigned ua = __builtin_bit_cast(unsigned, a), ub = __builtin_bit_cast(unsigned, b);
+  const auto r = O == 16 ? __builtin_amdgcn_permlane16_swap(ua, ub, false, false)
+                         : __builtin_amdgcn_permlane32_swap(ua, ub, false, false);
+  const unsigned lo = r[0], hi = r[1];  // copied out: a bit cast of a vector's element reads its first one
+  return __builtin_bit_cast(float, lo) + __builtin_bit_cast(float, hi);
+}
+
+// Sum over each aligned group of N lanes, in every lane of it: the pairs of a butterfly over lane bits 0, 1, ... (the
+// mirrors are exchanges of bits 2 and 3 once the 4 and 8 lanes below hold equal sums). The lanes of a row of 16 must all be active, those of the wave for N > 16.
+template <int N>
+PGN_DEVICE float group_sum(float x) {
+  if constexpr (N >= 2) x += dpp_move<0xB1>(x);   // quad_perm [1, 0, 3, 2]
+  if constexpr (N >= 4) x += dpp_move<0x4E>(x);   // quad_perm [2, 3, 0, 1]
+  if constexpr (N >= 8) x += dpp_move<0x141>(x);  // row_half_mirror
+  if constexpr (N >= 16) x += dpp_move<0x140>(x);  // row_mirror
+  if constexpr (N >= 32) x = swap_add<16>(x, x);
+  if constexpr (N >= 64) x = swap_add<32>(x, x);
+  return x;
+}
+
 // Sum over the 64 lanes of a wave of NV values per lane (NV a power of two <= 16): the lanes exchange halves, so the
 // sums take 6 + NV - 1 exchanges instead of 6 NV. Lane l ends with the sum of value l >> (6 - log2 NV) in v[0].
 template <int NV>
 PGN_DEVICE void wave_sum_many(float (&v)[NV], int l) {
-  int len = NV;
+  if constexpr (NV == 1) {
+    v[0] = group_sum<64>(v[0]);
+  } else {
 #pragma unroll
-  for (int s = 32; s >= 1; s >>= 1) {
-    if (len > 1) {
-      const int half = len / 2;
-      const bool hi = (l & s) != 0;
+    for (int m = 0; m < NV / 2; ++m) v[m] = swap_add<32>(v[m], v[m + NV / 2]);
+    if constexpr (NV >= 4) {
 #pragma unroll
-      for (int m = 0; m < half; ++m) {
-        const float send = hi ? v[m] : v[m + half];
-        const float keep = hi ? v[m + half] : v[m];
-        v[m] = keep + __shfl_xor(send, s);
-      }
-      len = half;
+      for (int m = 0; m < NV / 4; ++m) v[m] = swap_add<16>(v[m], v[m + NV / 4]);
     } else {
-      v[0] += __shfl_xor(v[0], s);
+      v[0] = swap_add<16>(v[0], v[0]);
+    }
+    if constexpr (NV >= 8) {  // lane bit 3: the lane 8 away keeps the other half
+      const bool hi = (l & 8) != 0;
+#pragma unroll
+      for (int m = 0; m < NV / 8; ++m) {
+        const float send = hi ? v[m] : v[m + NV / 8], keep = hi ? v[m + NV / 8] : v[m];
+        v[m] = keep + dpp_move<0x128>(send);  // row_ror:8
+      }
+    }
+    if constexpr (NV >= 16) {
+      const bool hi = (l & 4) != 0;
+      const float send = hi ? v[0] : v[1], keep = hi ? v[1] : v[0];
+      v[0] = keep + __shfl_xor(send, 4);
+    }
+    constexpr int rest = 64 / NV;
+    if constexpr (rest == 32) {  // lane bits 0..3 left (bit 4 summed above)
+      v[0] = group_sum<16>(v[0]);
+    } else {
+      v[0] = group_sum<rest>(v[0]);
     }
   }
 }

@@ -141,8 +141,11 @@ __global__ __launch_bounds__(256) void gemv(const float* __restrict__ x, int B, 
 
 // The decode GEMV for B <= 4 sequences and K = 256 KV: one wave per RPW output rows (a one-wave workgroup, so
 // hundreds to thousands of them cover the chip and one round of loads covers the whole weight). Lane l reads the
-// 16-byte pieces 4 l + 256 u of each of its rows, so one load instruction reads 1 KiB contiguous; all RPW KV pieces
-// are issued before the inputs are read. The input is used as is (MODE 0), LayerNorm'd (MODE 1: the wave computes
+// 16-byte pieces 4 l + 256 u of each of its rows, so one load instruction reads 1 KiB contiguous. Every load of the
+// wave is issued before any is waited for, none behind a branch (an absent operand reads the weight and is not used) and
+// none left to the epilogue: at K 768 the LayerNorm form took 4.94 us a layer with its bias, LayerNorm bias and later
+// input pieces each a memory round trip of its own and its lane sums through the LDS unit, now 3.98 (launch 1.75, its
+// 8.3 MB of weights 1.7). The input is used as is (MODE 0), LayerNorm'd (MODE 1: the wave computes
 // the LayerNorm of every input row itself, the row in registers, two wave reductions), or RMS-normalised per group
 // of 64 or 128 channels (MODE 2 or 3: the carrier's per-head RMSNorm; a group's channels sit on 16 or 32 consecutive
 // lanes of one piece, so its sum of squares is a four- or five-step exchange). No LDS, no barrier. NB = 1 (B = 1) or 4 (B <= 4, rows past
@@ -154,108 +157,106 @@ __global__ __launch_bounds__(64) void gemv_wave(const float* __restrict__ x, int
                                                 const float* __restrict__ scale, int act,
                                                 const float* __restrict__ resid, float* __restrict__ y) {
   constexpr int K = 256 * KV;
+  constexpr int NV = RPW * NB, sh = 6 - log2_of<NV>();
   const int l = threadIdx.x;
   const int n0 = blockIdx.x * RPW;
-  f32x4 w[RPW][KV];
+  // the output this lane ends with, and its epilogue operands' addresses (the weight's first entry where there is none)
+  const int ob = (l >> sh) % NB, on = n0 + (l >> sh) / NB;
+  const size_t off = (size_t)min(ob, B - 1) * N + min(on, N - 1);
+  const float* sp = scale ? scale : W;
+  const float* bp = bias ? bias + min(on, N - 1) : W;
+  const float* rp = resid ? resid + off : W;
+  // the inputs first: counted in order, they are waited for (and LayerNorm'd) with the weight still in flight.
+  // Sequences past B read the last one and are not written.
+  f32x4 z[NB][KV], w[RPW][KV], g[KV], c[KV];
+#pragma unroll
+  for (int b = 0; b < NB; ++b)
+#pragma unroll
+    for (int u = 0; u < KV; ++u)
+      z[b][u] = *reinterpret_cast<const f32x4*>(x + (size_t)min(b, B - 1) * K + 4 * l + 256 * u);
+  __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int r = 0; r < RPW; ++r) {
     const float* wr = W + (size_t)min(n0 + r, N - 1) * K + 4 * l;
 #pragma unroll
     for (int u = 0; u < KV; ++u) w[r][u] = *reinterpret_cast<const f32x4*>(wr + 256 * u);
   }
-  float acc[RPW * NB];
+  constexpr int G = MODE == 3 ? 128 : 64, GL = G / 4;
+  if constexpr (MODE == 1) {
+    const float* cp = lnb ? lnb : lnw;
 #pragma unroll
-  for (int m = 0; m < RPW * NB; ++m) acc[m] = 0.f;
-  if constexpr (MODE != 0) {
-    f32x4 z[NB][KV];
+    for (int u = 0; u < KV; ++u) {
+      g[u] = *reinterpret_cast<const f32x4*>(lnw + 4 * l + 256 * u);
+      c[u] = *reinterpret_cast<const f32x4*>(cp + 4 * l + 256 * u);
+    }
+  } else if constexpr (MODE >= 2) {
+    // channels 4 (l mod GL) .. + 3 of a G-channel group: the group weight piece is the same for every u
+    g[0] = *reinterpret_cast<const f32x4*>(lnw + 4 * (l & (GL - 1)));
+  }
+  const float es = *sp, eb = *bp, er = *rp;
+  __builtin_amdgcn_sched_barrier(0);
+  float acc[NV];
+#pragma unroll
+  for (int m = 0; m < NV; ++m) acc[m] = 0.f;
+  if constexpr (MODE == 1) {
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+      float s = 0.f;
+#pragma unroll
+      for (int u = 0; u < KV; ++u) s += (z[b][u][0] + z[b][u][1]) + (z[b][u][2] + z[b][u][3]);
+      s = group_sum<64>(s);
+      const float mean = s * (1.f / K);
+      float s2 = 0.f;
+#pragma unroll
+      for (int u = 0; u < KV; ++u)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          z[b][u][e] -= mean;
+          s2 += z[b][u][e] * z[b][u][e];
+        }
+      s2 = group_sum<64>(s2);
+      const float rs = 1.f / sqrtf(s2 * (1.f / K) + eps);
+#pragma unroll
+      for (int u = 0; u < KV; ++u) z[b][u] *= rs;
+    }
+    __builtin_amdgcn_sched_barrier(0);  // up to here on the inputs alone
 #pragma unroll
     for (int b = 0; b < NB; ++b)
 #pragma unroll
       for (int u = 0; u < KV; ++u)
-        z[b][u] = b < B ? *reinterpret_cast<const f32x4*>(x + (size_t)b * K + 4 * l + 256 * u)
-                        : f32x4{0.f, 0.f, 0.f, 0.f};
-    if constexpr (MODE == 1) {
-      f32x4 g[KV], c[KV];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) z[b][u][e] = z[b][u][e] * g[u][e] + (lnb ? c[u][e] : 0.f);
+  } else if constexpr (MODE >= 2) {
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
 #pragma unroll
       for (int u = 0; u < KV; ++u) {
-        g[u] = *reinterpret_cast<const f32x4*>(lnw + 4 * l + 256 * u);
-        c[u] = lnb ? *reinterpret_cast<const f32x4*>(lnb + 4 * l + 256 * u) : f32x4{0.f, 0.f, 0.f, 0.f};
+        float s = (z[b][u][0] * z[b][u][0] + z[b][u][1] * z[b][u][1]) +
+                  (z[b][u][2] * z[b][u][2] + z[b][u][3] * z[b][u][3]);
+        s = group_sum<GL>(s);
+        z[b][u] *= 1.f / sqrtf(s * (1.f / G) + eps);
       }
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int b = 0; b < NB; ++b) {
-        float s = 0.f;
+    for (int b = 0; b < NB; ++b)
 #pragma unroll
-        for (int u = 0; u < KV; ++u) s += (z[b][u][0] + z[b][u][1]) + (z[b][u][2] + z[b][u][3]);
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
-        const float mean = s * (1.f / K);
-        float s2 = 0.f;
-#pragma unroll
-        for (int u = 0; u < KV; ++u)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const float d = z[b][u][e] - mean;
-            s2 += d * d;
-          }
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) s2 += __shfl_xor(s2, o);
-        const float rs = 1.f / sqrtf(s2 * (1.f / K) + eps);
-#pragma unroll
-        for (int u = 0; u < KV; ++u)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) z[b][u][e] = (z[b][u][e] - mean) * rs * g[u][e] + c[u][e];
-      }
-    } else {
-      // channels 4 (l mod GL) .. + 3 of a G-channel group: the group weight piece is the same for every u
-      constexpr int G = MODE == 3 ? 128 : 64, GL = G / 4;
-      const f32x4 g = *reinterpret_cast<const f32x4*>(lnw + 4 * (l & (GL - 1)));
-#pragma unroll
-      for (int b = 0; b < NB; ++b)
-#pragma unroll
-        for (int u = 0; u < KV; ++u) {
-          float s = (z[b][u][0] * z[b][u][0] + z[b][u][1] * z[b][u][1]) +
-                    (z[b][u][2] * z[b][u][2] + z[b][u][3] * z[b][u][3]);
-#pragma unroll
-          for (int o = 1; o < GL; o <<= 1) s += __shfl_xor(s, o);
-          const float rs = 1.f / sqrtf(s * (1.f / G) + eps);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) z[b][u][e] = (z[b][u][e] * rs) * g[e];
-        }
-    }
-#pragma unroll
-    for (int r = 0; r < RPW; ++r)
-#pragma unroll
-      for (int b = 0; b < NB; ++b)
-#pragma unroll
-        for (int u = 0; u < KV; ++u)
-          acc[r * NB + b] += w[r][u][0] * z[b][u][0] + w[r][u][1] * z[b][u][1] + w[r][u][2] * z[b][u][2] +
-                             w[r][u][3] * z[b][u][3];
-  } else {
-#pragma unroll
-    for (int u = 0; u < KV; ++u)
-#pragma unroll
-      for (int b = 0; b < NB; ++b) {
-        const f32x4 z = b < B ? *reinterpret_cast<const f32x4*>(x + (size_t)b * K + 4 * l + 256 * u)
-                              : f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int r = 0; r < RPW; ++r)
-          acc[r * NB + b] += w[r][u][0] * z[0] + w[r][u][1] * z[1] + w[r][u][2] * z[2] + w[r][u][3] * z[3];
-      }
+      for (int u = 0; u < KV; ++u) z[b][u] *= g[0];
   }
-  constexpr int NV = RPW * NB;
+#pragma unroll
+  for (int r = 0; r < RPW; ++r)
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+      for (int u = 0; u < KV; ++u)
+        acc[r * NB + b] += w[r][u][0] * z[b][u][0] + w[r][u][1] * z[b][u][1] + w[r][u][2] * z[b][u][2] +
+                           w[r][u][3] * z[b][u][3];
+  asm volatile("" ::"s"(es), "s"(y));  // loaded by now, not behind the sums
   wave_sum_many<NV>(acc, l);
-  constexpr int sh = 6 - log2_of<NV>();
-  if ((l & ((1 << sh) - 1)) == 0) {
-    const int m = l >> sh, r = m / NB, b = m % NB;
-    const int n = n0 + r;
-    if (n < N && b < B) {
-      float v = (scale ? *scale : 1.f) * acc[0] + (bias ? bias[n] : 0.f);
-      if (act == 1) v = pgn_gelu_erf(v);
-      const size_t off = (size_t)b * N + n;
-      if (resid) v += resid[off];
-      y[off] = v;
-    }
-  }
+  // every lane forms the value (a conditional use would take the operands' loads down here, behind the sums)
+  float v = (scale ? es : 1.f) * acc[0] + (bias ? eb : 0.f);
+  if (act == 1) v = pgn_gelu_erf(v);
+  v += resid ? er : 0.f;
+  if ((l & ((1 << sh) - 1)) == 0 && on < N && ob < B) y[off] = v;
 }
 
 // The accumulating GEMV (no normalisation) for B <= 4: y[b][n] += scale * (W x_b)[n] + bias[n], K = 256 KV split
@@ -270,26 +271,30 @@ __global__ __launch_bounds__(64) void gemv_wave_acc(const float* __restrict__ x,
   const int l = threadIdx.x;
   const int n = blockIdx.x % N, ks = blockIdx.x / N;
   const float* wr = W + (size_t)n * K + 256 * KV * ks + 4 * l;
-  f32x4 w[KV];
+  f32x4 w[KV], z[NB][KV];
 #pragma unroll
   for (int u = 0; u < KV; ++u) w[u] = *reinterpret_cast<const f32x4*>(wr + 256 * u);
+#pragma unroll
+  for (int b = 0; b < NB; ++b)  // sequences past B read the last one and are not written
+#pragma unroll
+    for (int u = 0; u < KV; ++u)
+      z[b][u] = *reinterpret_cast<const f32x4*>(x + (size_t)min(b, B - 1) * K + 256 * KV * ks + 4 * l + 256 * u);
+  const float sv = *(scale ? scale : W), bv = *(bias ? bias + n : W);
+  __builtin_amdgcn_sched_barrier(0);
   float acc[NB];
 #pragma unroll
   for (int b = 0; b < NB; ++b) acc[b] = 0.f;
 #pragma unroll
   for (int u = 0; u < KV; ++u)
 #pragma unroll
-    for (int b = 0; b < NB; ++b) {
-      const f32x4 z = b < B ? *reinterpret_cast<const f32x4*>(x + (size_t)b * K + 256 * KV * ks + 4 * l + 256 * u)
-                            : f32x4{0.f, 0.f, 0.f, 0.f};
-      acc[b] += w[u][0] * z[0] + w[u][1] * z[1] + w[u][2] * z[2] + w[u][3] * z[3];
-    }
+    for (int b = 0; b < NB; ++b)
+      acc[b] += w[u][0] * z[b][u][0] + w[u][1] * z[b][u][1] + w[u][2] * z[b][u][2] + w[u][3] * z[b][u][3];
+  asm volatile("" ::"s"(sv), "s"(bv), "s"(y));  // loaded by now, not behind the sums
   wave_sum_many<NB>(acc, l);
   constexpr int sh = 6 - log2_of<NB>();
-  if ((l & ((1 << sh) - 1)) == 0) {
-    const int b = l >> sh;
-    if (b < B) atomicAdd(y + (size_t)b * N + n, (scale ? *scale : 1.f) * acc[0] + (bias && ks == 0 ? bias[n] : 0.f));
-  }
+  const int b = l >> sh;
+  const float v = (scale ? sv : 1.f) * acc[0] + (bias && ks == 0 ? bv : 0.f);
+  if ((l & ((1 << sh) - 1)) == 0 && b < B) atomicAdd(y + (size_t)b * N + n, v);
 }
 
 template <int RPW, int NB, int KV, int MODE>

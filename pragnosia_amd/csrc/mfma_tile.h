@@ -299,19 +299,12 @@ PGN_DEVICE void put_seg(__bf16* tile, bf16x8 v, int e) {
 PGN_DEVICE float masked_decay(float x, bool keep) { return __expf(fminf(x, 0.f)) * (keep ? 1.f : 0.f); }
 
 // Sum over the 16 lanes of a lane group (same g): butterfly over lane bits 0..3.
-PGN_DEVICE float sum16(float x) {
-  x += __shfl_xor(x, 1);
-  x += __shfl_xor(x, 2);
-  x += __shfl_xor(x, 4);
-  x += __shfl_xor(x, 8);
-  return x;
-}
+PGN_DEVICE float sum16(float x) { return group_sum<16>(x); }
 
 // Sum over the 4 lane groups (same i): butterfly over lane bits 4..5.
 PGN_DEVICE float sum_groups(float x) {
-  x += __shfl_xor(x, 16);
-  x += __shfl_xor(x, 32);
-  return x;
+  x = swap_add<16>(x, x);
+  return swap_add<32>(x, x);
 }
 
 PGN_DEVICE float wave_sum(float x) { return sum_groups(sum16(x)); }
