@@ -9,9 +9,9 @@
 //
 // At 64 sequences every weight element is used 64 times a step (32 flop per byte read), so the fp32 matrix-core rate
 // matters as much as HBM, and at these sizes a workgroup's own latency (its loads, then its products, then its
-// reduction) sets the kernel's time. Work split: a workgroup owns NC column tiles of 16 output columns (NC = 1, or 3
-// where that still leaves 192 workgroups: each input piece then feeds three products, a third fewer operand bytes
-// per CU from L2) of 16 rows (one row block), all of K: its KW waves (at most 16) split K into 16-wide steps, S
+// reduction) sets the kernel's time. Work split: a workgroup owns NC = 1, 2 or 3 column tiles of 16 output columns
+// (pick_tiles: each input piece then feeds NC products) of 16 rows (one row block), all of K: its KW waves (at most 16)
+// split K into 16-wide steps, S
 // consecutive steps a chunk and C chunks a wave. So a layer at 64 rows is 4 x ceil(N / 16 NC) workgroups; those of
 // one column group are numbered 8 apart, so they run on one XCD (workgroup i goes to XCD i mod 8) and read the
 // group's weight from one L2. A wave issues its
@@ -38,6 +38,12 @@
 namespace {
 
 constexpr int MAXW = 16;  // waves per workgroup
+
+// sum over the four lanes that hold one row (lane bits 4 and 5)
+PGN_DEVICE float quarter_sum(float x) {
+  x = swap_add<16>(x, x);
+  return swap_add<32>(x, x);
+}
 
 // ACC: the K split over SK groups of workgroups (split ks over K range ks K .. ks K + K - 1 of rows of ldx = SK K
 // entries), each adding its partial products (and, for split 0, the bias) to y with atomics: y holds the residual.
@@ -108,8 +114,7 @@ __global__ __launch_bounds__(1024) void decode_gemm_k(const float* __restrict__ 
       float a = 0.f;
 #pragma unroll
       for (int s = 0; s < S; ++s) a += (z[b][s][0] + z[b][s][1]) + (z[b][s][2] + z[b][s][3]);
-      a += __shfl_xor(a, 16);
-      a += __shfl_xor(a, 32);
+      a = quarter_sum(a);
       const float mc = a * (1.f / (16 * S));
       float q = 0.f;
 #pragma unroll
@@ -119,8 +124,7 @@ __global__ __launch_bounds__(1024) void decode_gemm_k(const float* __restrict__ 
           const float d = z[b][s][e] - mc;
           q += d * d;
         }
-      q += __shfl_xor(q, 16);
-      q += __shfl_xor(q, 32);
+      q = quarter_sum(q);
       if (c == 0) {
         mw = mc;
         m2w = q;
@@ -137,8 +141,7 @@ __global__ __launch_bounds__(1024) void decode_gemm_k(const float* __restrict__ 
       for (int s = 0; s < S; ++s)
 #pragma unroll
         for (int e = 0; e < 4; ++e) a += z[b][s][e] * z[b][s][e];
-      a += __shfl_xor(a, 16);
-      a += __shfl_xor(a, 32);
+      a = quarter_sum(a);
       const float r = 1.f / sqrtf(a * (1.f / (16 * S)) + eps);
 #pragma unroll
       for (int s = 0; s < S; ++s)
@@ -245,25 +248,47 @@ int launch_nc(const Plan& p, const float* x, int B, int K, const float* csum, fl
   PGN_RETURN_LAUNCH();
 }
 
-// Workgroups of three column tiles (each x piece feeds three products: a third fewer operand bytes per CU from L2,
-// which is what bounds these layers) when that still leaves this many workgroups; else one tile a workgroup.
-constexpr int64_t kWideGroups = 192;
+// How many column tiles a workgroup takes: the count whose busiest CU has the least to do, the rounds of workgroups over
+// the CUs times a workgroup's operand pieces and products. Its x piece comes in half lines (64 bytes of a row) and costs
+// more than a contiguous weight tile: 4 for x, 3 a tile. Past three rounds of workgroups two of which fit a CU (S <= 3),
+// the last round is shared and the rounds count in fractions. us a call, cold weights, with 1 / 2 / 3 tiles: K 768, N 3072
+// (192 tiles): 16 rows 6.56 / 7.66 / 9.11, 32 rows 8.84 / 7.42 / 8.65, 64 rows 12.1 / 10.2 / 8.55; N 8192: 16 rows 9.68 /
+// 8.59 / 9.80, 32 rows 15.7 / 11.1 / 13.2, 64 rows 27.0 / 18.5 / 17.7; K 1024, N 4096: 48 rows 13.6 / 11.9 / 15.7, 64 rows
+// 17.0 / 12.1 / 17.0.
+constexpr int64_t kCUs = 256;
 
-template <int S, int C, int MODE>
-int launch(const Plan& p, const float* x, int B, int K, const float* csum, float eps, const float* Wt, int N,
-           const float* bias, const float* scale, int act, const float* resid, float* y, hipStream_t st) {
-  if constexpr (C == 1 && MODE < 2) {
-    const int64_t NT = (N + 15) / 16, ZB = (B + 15) / 16;
-    if (ZB * ((NT + 2) / 3) >= kWideGroups)
-      return launch_nc<S, C, MODE, 3>(p, x, B, K, csum, eps, Wt, N, bias, scale, act, resid, y, st);
+int pick_tiles(int S, int64_t NT, int64_t ZB, int64_t splits) {
+  int best = 1;
+  double cost = 0;
+  for (int nc : {1, 2, 3}) {
+    const int64_t wgs = (NT + nc - 1) / nc * ZB * splits;
+    const double rounds = S <= 3 && wgs > 3 * kCUs ? (double)wgs / kCUs : (double)((wgs + kCUs - 1) / kCUs);
+    const double v = rounds * (3 * nc + 4);
+    if (nc == 1 || v < cost) {
+      cost = v;
+      best = nc;
+    }
   }
-  return launch_nc<S, C, MODE, 1>(p, x, B, K, csum, eps, Wt, N, bias, scale, act, resid, y, st);
+  return best;
+}
+
+template <int S, int C, int MODE, bool ACC>
+int launch(const Plan& p, const float* x, int B, int K, const float* csum, float eps, const float* Wt, int N,
+           const float* bias, const float* scale, int act, const float* resid, float* y, hipStream_t st, int SK = 1) {
+#define PGN_NC(V) return launch_nc<S, C, MODE, V, ACC>(p, x, B, K, csum, eps, Wt, N, bias, scale, act, resid, y, st, SK)
+  if constexpr (C == 1 && MODE < 2) {
+    const int nc = pick_tiles(S, (N + 15) / 16, (B + 15) / 16, SK);
+    if (nc == 3) PGN_NC(3);
+    if (nc == 2) PGN_NC(2);
+  }
+  PGN_NC(1);
+#undef PGN_NC
 }
 
 template <int C, int MODE>
 int dispatch_s(const Plan& p, const float* x, int B, int K, const float* csum, float eps, const float* Wt, int N,
                const float* bias, const float* scale, int act, const float* resid, float* y, hipStream_t st) {
-#define PGN_S(V) return launch<V, C, MODE>(p, x, B, K, csum, eps, Wt, N, bias, scale, act, resid, y, st)
+#define PGN_S(V) return launch<V, C, MODE, false>(p, x, B, K, csum, eps, Wt, N, bias, scale, act, resid, y, st)
   if constexpr (MODE == 2) {
     if (p.S == 8) PGN_S(8);
     PGN_S(4);
@@ -279,17 +304,11 @@ int dispatch_s(const Plan& p, const float* x, int B, int K, const float* csum, f
 #undef PGN_S
 }
 
-// The split-K accumulating form: SK splits of Kp = K / SK each; mode 0 with three column tiles a workgroup where that
-// still leaves kWideGroups workgroups, the RMS mode (MODE 2, whole channel groups a split) one tile.
+// The split-K accumulating form: SK splits of Kp = K / SK each.
 template <int S, int C, int MODE>
 int launch_acc(const Plan& p, const float* x, int B, int Kp, float eps, const float* Wt, int N, const float* bias,
                const float* scale, float* y, hipStream_t st, int SK) {
-  if constexpr (C == 1 && MODE == 0) {
-    const int64_t NT = (N + 15) / 16, ZB = (B + 15) / 16;
-    if (ZB * ((NT + 2) / 3) * SK >= kWideGroups)
-      return launch_nc<S, C, 0, 3, true>(p, x, B, Kp, nullptr, 0.f, Wt, N, bias, scale, 0, nullptr, y, st, SK);
-  }
-  return launch_nc<S, C, MODE, 1, true>(p, x, B, Kp, nullptr, eps, Wt, N, bias, scale, 0, nullptr, y, st, SK);
+  return launch<S, C, MODE, true>(p, x, B, Kp, nullptr, eps, Wt, N, bias, scale, 0, nullptr, y, st, SK);
 }
 
 template <int C>
