@@ -481,8 +481,8 @@ class AssocCarrier(nn.Module):
         the same function as calling `forward` on x[:, s:s + window] for s = 0, window, ... in turn, handing each
         call the state the previous one returned (`src/model.py:842-864` drives the reference's carrier so). A
         carrier without autograd, with `window` a multiple of 64, runs every window in one pass: the projections over
-        the whole sequence, then for the plain rule one segment-parallel scan that rebases the state at window
-        boundaries, for the delta rule every window at once from its affine state map (`ops.aspin_delta_windows`);
+        the whole sequence, then one scan that rebases the state at window boundaries, for the plain rule
+        segment-parallel, for the delta rule chunk-parallel (`ops.aspin_delta_windows`);
         otherwise the windows run one call each. Returns (x + gated output, (S, length of the last window)); `sent`
         is not kept."""
         B, T, D = x.shape
