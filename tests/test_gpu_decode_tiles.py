@@ -1,5 +1,5 @@
 """The decode step's dense layers where a workgroup takes two column tiles (a partial last group, a ragged last tile, a
-partial row block) and the one-wave GEMV with operands left out, against fp64 torch.
+partial row block) and the one-wave GEMV with operands left out, against fp64 torch; the step tail's argmax at its edges.
 
 Tolerance: sums of K fp32 products in any order, each within K 2^-24 of the sum of magnitudes at the worst and about
 sqrt(K) 2^-24 as rounding errors go: 1e-5 of the largest output holds both at these K with inputs of unit size."""
@@ -64,3 +64,34 @@ def test_gemv_with_operands_left_out(given, B, K, N):
         y = torch.ops.pragnosia.decode_gemv(x, W, nw if ln else None, nb if ln else None, 1e-5, bias, scale, 0, resid)
         z = F.layer_norm(x.double(), (K,), nw.double(), None if nb is None else nb.double(), 1e-5) if ln else x.double()
         assert _rel(y, z @ W.double().t() * d(scale, 1.0) + d(bias, 0.0) + d(resid, 0.0)) < 1e-5
+
+
+@pytest.mark.parametrize("V", [1, 5, 63, 64, 1023, 1025, 8193])
+def test_decode_tail_argmax_edges(V):
+    """The tail's argmax by ordered keys is torch's: waves and threads without a logit, the maximum in every kind of
+    place, all values negative, -inf throughout, equal zeros of both signs, infinities, NaN of either sign."""
+    from pragnosia_amd.ops import decode_tail
+    g = torch.Generator(device="cuda").manual_seed(V)
+    lg = torch.randn(10, V, device="cuda", generator=g)
+    lg[0, 0] = lg[1, V - 1] = lg[2, V // 2] = 9.0
+    lg[3] = -lg[3].abs() - 1.0
+    lg[4] = -float("inf")
+    lg[5] = -0.0
+    lg[5, V // 2:] = 0.0
+    lg[6, V // 3] = float("inf")
+    lg[7, V // 2] = -float("nan")
+    lg[7, V - 1] = float("nan")
+    lg[8] = float("nan")
+    lg[9] = 1e-42  # below the normal range
+    B, d = lg.shape[0], 40
+    emb, pemb = torch.randn(V, d, device="cuda", generator=g), torch.randn(7, d, device="cuda", generator=g)
+    ctr, pos = torch.tensor([0, -1], device="cuda"), torch.tensor([3, -1], device="cuda")
+    out = torch.zeros(1, B, dtype=torch.long, device="cuda")
+    tok, h = torch.zeros(B, 1, dtype=torch.long, device="cuda"), torch.zeros(B, d, device="cuda")
+    decode_tail(lg, emb, pemb, ctr[0], ctr[1], pos[0], pos[1], out, tok, h, None, None)
+    # torch's rule from its parts: the first NaN if there is one, else the first index of the maximum
+    ref = lg.cpu()
+    best = torch.where(ref.isnan().any(1, keepdim=True), ref.isnan(), ref == ref.amax(1, keepdim=True))
+    want = best.int().argmax(1).cuda()
+    assert torch.equal(out[0], want) and torch.equal(tok.view(-1), want)
+    assert torch.equal(h, emb[want] + pemb[4])
