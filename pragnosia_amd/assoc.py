@@ -423,7 +423,8 @@ class AssocCarrier(nn.Module):
         if decode and self.dk == HEAD_DIM_KERNEL:
             # the fused fp32 step: rebase, normalise, gate, decay, write, read
             qp, kp, vp, gate, la, bt, cc = self._projections(z, cc)
-            S_prev = S0 if S0 is not None else torch.zeros(B, self.h, self.dk, self.dk, device=x.device)
+            S_prev = (S0 if S0 is not None
+                      else torch.zeros(B, self.h, self.dk, self.dk, device=x.device, dtype=torch.float32))
             S, o = _op.aspin_decode_step(S_prev, qp.reshape(B, self.h, self.dk), kp.reshape(B, self.h, self.dk),
                                          vp.reshape(B, self.h, self.dk),
                                          None if gate is None else gate.reshape(B, self.h),

@@ -120,7 +120,8 @@ class GreedyDecoder:
         out = []
         for st in states:
             if isinstance(st[1], (int, float)) or (torch.is_tensor(st[1]) and st[1].dim() == 0):
-                p0 = st[1] if torch.is_tensor(st[1]) else torch.tensor(float(st[1]), device=st[0].device)
+                p0 = (st[1] if torch.is_tensor(st[1])
+                      else torch.tensor(float(st[1]), device=st[0].device, dtype=torch.float32))
                 # (S, position) or, with a short convolution, (S, position, cache)
                 out.append((st[0].clone().contiguous(), p0.float().clone(),
                             *(t.clone().contiguous() for t in st[2:])))
@@ -142,10 +143,10 @@ class GreedyDecoder:
         torch._foreach_copy_([st[0] for st in self.st], [st[0] for st in states])
         pos = [st[1] for st in states]
         if any(torch.is_tensor(p) for p in pos):
-            pos = [p if torch.is_tensor(p) else torch.tensor(float(p)) for p in pos]
+            pos = [p if torch.is_tensor(p) else torch.tensor(float(p), dtype=torch.float32) for p in pos]
             self.p0s.copy_(torch.stack([p.reshape(()).to(self.p0s) for p in pos]))
         else:
-            self.p0s.copy_(torch.tensor([float(p) for p in pos]))
+            self.p0s.copy_(torch.tensor([float(p) for p in pos], dtype=torch.float32))
 
     def _one_step(self, par=0):
         m = self.m
@@ -339,7 +340,7 @@ class GreedyDecoder:
         self.out = torch.zeros(n_max + self.K, self.B, dtype=torch.long, device=dev)
         self.ctr = torch.zeros(1, dtype=torch.long, device=dev)
         if self.fused:  # the fused step's input and the tail kernel's alternating counter and position slots
-            self.h = torch.zeros(self.B, self.m.d, device=dev)
+            self.h = torch.zeros(self.B, self.m.d, device=dev, dtype=torch.float32)
             self.ctrb = torch.zeros(2, dtype=torch.long, device=dev)
             self.posb = torch.zeros(2, dtype=torch.long, device=dev)
         if self.record:

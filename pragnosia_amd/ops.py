@@ -201,8 +201,8 @@ def diag_scan_bwd(g: Tensor, g_last_r: Optional[Tensor], g_last_i: Optional[Tens
     logmag, ang, hr, hi, h0r, h0i = _f32(logmag), _f32(ang), _f32(hr), _f32(hi), _f32(h0r), _f32(h0i)
     du, dlm, dan = (torch.empty(B, T, D, device=g.device, dtype=torch.float32) for _ in range(3))
     has = h0r is not None
-    dh0r = torch.empty(B, D, device=g.device) if has else g.new_empty(0)
-    dh0i = torch.empty(B, D, device=g.device) if has else g.new_empty(0)
+    dh0r = torch.empty(B, D, device=g.device, dtype=torch.float32) if has else g.new_empty(0)
+    dh0i = torch.empty(B, D, device=g.device, dtype=torch.float32) if has else g.new_empty(0)
     check(lib().pragnosia_diag_scan_bwd(_ptr(g), _ptr(g_last_r), _ptr(g_last_i), _ptr(logmag), _ptr(ang), _ptr(hr),
                                         _ptr(hi), _ptr(h0r), _ptr(h0i), _ptr(du), _ptr(dlm), _ptr(dan),
                                         _ptr(dh0r) if has else None, _ptr(dh0i) if has else None,
@@ -1052,7 +1052,8 @@ def aspin_exact(q: Tensor, k: Tensor, v: Tensor, la: Tensor, beta: Optional[Tens
         sizes = _exact_parts(B, H, T, Dv, beta is not None)
         resid = torch.empty(sum(sizes), device=dev, dtype=dt)
         scores, gates, M, X, R, U = _exact_views(resid, sizes)
-        W = torch.empty(B * H * NC * CHUNK, (Dk + 15) // 16 * 16, device=dev) if beta is not None else None
+        W = (torch.empty(B * H * NC * CHUNK, (Dk + 15) // 16 * 16, device=dev, dtype=dt) if beta is not None
+             else None)
         check(lib().pragnosia_aspin_exact_chunk_fwd(_ptr(q), _ptr(k), _ptr(v), _ptr(la), _ptr(beta), _ptr(S0), _ptr(o),
                                                     _ptr(S), _ptr(ckpt), _ptr(scores), _ptr(gates), _ptr(M), _ptr(X),
                                                     _ptr(R), _ptr(U), _ptr(W), B, H, T, Dk, Dv, _stream(q)),
@@ -1221,7 +1222,8 @@ def aspin_prep_bwd(qp: Tensor, kp: Tensor, vp: Tensor, gate: Optional[Tensor], t
     dq, dk, dv = _bf16(dq), _bf16(dk), _bf16(dv)
     B, T, H, D = qp.shape
     dqp, dkp, dvp = torch.empty_like(qp), torch.empty_like(qp), torch.empty_like(qp)
-    dgate = torch.empty(B, T, H, device=qp.device) if gate is not None else qp.new_empty(0, dtype=torch.float32)
+    dgate = (torch.empty(B, T, H, device=qp.device, dtype=torch.float32) if gate is not None
+             else qp.new_empty(0, dtype=torch.float32))
     rows = lib().pragnosia_aspin_prep_theta_partials(B, T)
     dth = torch.empty(rows, H, D // 2, device=qp.device, dtype=torch.float32)
     check(lib().pragnosia_aspin_prep_bwd(_ptr(qp), _ptr(kp), _ptr(vp), _ptr(gate), _ptr(theta), _ptr(pos), _ptr(dq),
@@ -1347,7 +1349,7 @@ def aspin_prep_proj_bwd(P: Tensor, H: int, la_bias: Tensor, A: Tensor, la_floor:
     B, T, W = P.shape
     has_beta = not gated and W > 3 * H * D + H
     if has_beta:
-        dbeta = torch.zeros(B, H, T, device=P.device) if dbeta is None else _f32(dbeta)
+        dbeta = torch.zeros(B, H, T, device=P.device, dtype=torch.float32) if dbeta is None else _f32(dbeta)
     dP = torch.empty_like(P)  # the kernel zeroes the columns past the last group
     rows = lib().pragnosia_aspin_prep_theta_partials(B, T)
     dth = torch.empty(rows, H, D // 2, device=P.device, dtype=torch.float32)
@@ -1386,7 +1388,7 @@ def _prep_proj_backward(ctx, dq, dk, dv, dla, dbeta):
     P, la_bias, A, la_floor, gate_bias, beta_bias, theta, pos = ctx.saved_tensors
     B, T, _ = P.shape
     zb = lambda t: torch.zeros(B, ctx.H, T, ctx.D, device=P.device, dtype=torch.bfloat16) if t is None else t
-    dla = torch.zeros(B, ctx.H, T, device=P.device) if dla is None else dla
+    dla = torch.zeros(B, ctx.H, T, device=P.device, dtype=torch.float32) if dla is None else dla
     dP, dlb, dA, dxb, dth = aspin_prep_proj_bwd(P, ctx.H, la_bias, A, la_floor, gate_bias, beta_bias, ctx.beta_min,
                                                 ctx.gated, theta, pos, zb(dq), zb(dk), zb(dv), dla,
                                                 dbeta if (dbeta is not None and dbeta.numel()) else None, ctx.D)
