@@ -468,8 +468,11 @@ class AssocCarrier(nn.Module):
             o = self.on(o).transpose(1, 2).reshape(B, T, D)
         self.sent = sent
         if _needs_grad(x, o, self.o.weight, self.gate):
-            # gate on the weight, as the reference does for training (it keeps the backward's saved tensor small)
-            Wg = self.o.weight * torch.sigmoid(self.gate)
+            # gate on the weight, as the reference does for training (it keeps the backward's saved tensor small); one
+            # per row, so the gate's gradient is summed along the rows and then down the column of their sums. In one
+            # step, d x d values to one is a multi-block reduction, which clears its semaphores with a memset: captured
+            # in a HIP graph, a few replays in forty gave a gradient off by its own size (d 384, 6400 tokens).
+            Wg = self.o.weight * torch.sigmoid(self.gate).expand(self.d, 1)
             out = x + (_op_mod.linear_w(o, Wg) if FUSED_PLUMBING else F.linear(o, Wg))
         else:
             out = x + self._gated_out(o)

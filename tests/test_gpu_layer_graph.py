@@ -1,0 +1,45 @@
+"""GPU: one AssocCarrier's training step captured in a HIP graph, at the widths of the models trained on it."""
+import pytest
+import torch
+
+from test_gpu_training import _memset_nodes
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("d,head_dim,delta", [(384, 128, False), (704, 64, False), (768, 64, True)])
+def test_layer_step_records_no_memset(d, head_dim, delta):
+    """The step's graph holds no memset node (a reduction of the d x d gated weight to the scalar gate's gradient would
+    record one from d 384 on), and its replays, with eager steps and synchronisations between them, give the eager
+    step's gradients: the gate's to fp32 rounding of sums of d^2 terms, which cancel to some hundredths."""
+    from pragnosia_amd.assoc import AssocCarrier
+    torch.manual_seed(d)
+    with torch.device("cuda"):
+        m = AssocCarrier(d, head_dim=head_dim, delta=delta)
+    m.need_sent = False
+    x, t = torch.zeros(4, 400, d, device="cuda"), torch.randn(4, 400, d, device="cuda")
+    params = [p for n, p in m.named_parameters()]
+
+    def step():
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            y, _ = m(x)
+        return torch.autograd.grad(y, params, t, allow_unused=True)
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        for _ in range(2):
+            step()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        out = step()
+    assert _memset_nodes(graph) == 0
+    gate = [n for n, _ in m.named_parameters()].index("gate")
+    for _ in range(6):
+        x.normal_()
+        graph.replay()
+        got = out[gate].clone()
+        torch.cuda.synchronize()
+        want = step()[gate]
+        assert want.abs() > 0 and (got - want).abs() <= 1e-4 * want.abs() + 1e-3, (got.item(), want.item())
