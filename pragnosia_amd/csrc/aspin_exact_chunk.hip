@@ -14,9 +14,8 @@
 //     dQ = e^L o (dO S^T) + (dO U^T o D) K
 //     dK = (dO U^T o D)^T Q + w o (U G^T) - e^L o (dY S^T) + (P + P^T) K,   P = -strict_tril(dY R^T o D) diag(beta)
 //     dbeta_s = R_s . dU_s - sum_t (dY R^T)_ts M_ts
-//     dL_t = sum_s (dO U^T o A + P o K K^T)_ts - (the same summed over its other index) + q_t . (dQ's state term)
-//            - k_t . (w o U G^T)_t - k_t . (e^L o dY S^T)_t,   dla = the suffix sums of dL within the chunk plus
-//            e^(L_last) <G, S> + sum_s k_s . (w o U G^T)_s.
+//     dla_t = sum_{r >= t > s} (dO U^T o A + P o K K^T)_rs + sum_{r >= t} (q_r . (dQ's state term)_r
+//             - k_r . (e^L o dY S^T)_r) + sum_{s < t} k_s . (w o U G^T)_s + e^(L_last) <G, S>.
 // Only the state's recurrence runs along the chunks. The delta rule's is kept to two products a chunk by forming
 // W = X (e^L o K) (forward) and W' = X^T (beta o w o K) (backward) beforehand: R = X V - W S, dY = Y1 + W' G.
 //
@@ -31,7 +30,14 @@
 //
 // Decays: L is summed in fp64 and only differences (<= 0) are exponentiated, in fp32, so a long or steep run of decays
 // loses nothing to cancellation; log-decays below -1e4 (e^-1e4 = 0 in fp32) are taken as -1e4, which keeps the
-// differences finite for -inf. Entries above a score matrix's diagonal are selected to zero, not multiplied.
+// differences finite for -inf.
+//
+// Infinities and NaN stay in the tokens that the recurrence takes them to: outputs before such a token, and gradients
+// that do not come past it, are what they are without it. Entries above a score matrix's diagonal are selected to zero,
+// not multiplied; a product with a triangular operand, whose zeros meet the other operand's later (transposed: earlier)
+// tokens, has its non-finite results formed again over their own tokens (`own_tokens`); a log-decay of NaN or +inf is
+// left out of L and makes NaN of the differences that span it (`Decays`); and dla sums what lies on either side of its
+// token, with no term added that another takes away again.
 //
 // Products: v_mfma_f32_16x16x4f32 (A[r][k] in lane r + 16 k, B[k][c] in lane c + 16 k, D[4 g + e][c] in lane c + 16 g).
 // Four of them cover a 16-wide contraction with lane group g holding k = 4 g + e in the e-th, so an operand whose
@@ -188,6 +194,39 @@ PGN_DEVICE void store_tile(f32x4 (&acc)[2][2], float* p, int ld, int nrows, int 
   });
 }
 
+// Where acc, the 64 x 64 product of a(r, k), zero unless k <= r (LOWER) or k >= r, with b(k, c) over k < K, holds
+// anything non-finite: those entries again as sums over k's own range only, since 0 times an infinity or a NaN is NaN.
+// nc: columns that b has. Costs a comparison an entry where there is none.
+template <bool LOWER, class FA, class FB>
+PGN_DEVICE void own_tokens(f32x4 (&acc)[2][2], int K, int nc, const WaveIdx& x, FA&& a, FB&& b) {
+  bool bad = false;
+  each(acc, x, [&](int, int, float v) { bad |= !(fabsf(v) < INFINITY); });
+  if (!__any(bad)) return;
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int r = 32 * (x.w >> 1) + 16 * i + 4 * x.g, c = min(32 * (x.w & 1) + 16 * j + x.i, nc - 1);
+      f32x4 s = zero4();
+      for (int k = 0; k < K; ++k) {
+        const float bk = b(k, c);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (LOWER ? k <= r + e : k >= r + e) s[e] += a(r + e, k) * bk;
+      }
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (!(fabsf(acc[i][j][e]) < INFINITY)) acc[i][j][e] = s[e];
+    }
+}
+
+PGN_DEVICE void add(f32x4 (&a)[2][2], const f32x4 (&b)[2][2]) {
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) a[i][j] += b[i][j];
+}
+
 // out[row] = acc's row . X's row over the wave's 32 columns (X: rows of ld floats, nrows x ncols valid)
 PGN_DEVICE void row_dots(f32x4 (&acc)[2][2], const float* __restrict__ X, int ld, int nrows, int ncols, float* out,
                          const WaveIdx& x) {
@@ -206,22 +245,38 @@ PGN_DEVICE void row_dots(f32x4 (&acc)[2][2], const float* __restrict__ X, int ld
     }
 }
 
-// Cumulative log-decays of a chunk's n tokens (zero decay past them) in fp64, by the first wave
-PGN_DEVICE void decay_sums(const float* __restrict__ la, int n, double* Ls) {
+// Cumulative log-decays of a chunk's n tokens (zero decay past them) in fp64, by the first wave, without those that are
+// NaN or +inf (`bad`, a bit a token)
+struct Decays {
+  double L[CT];
+  unsigned long long bad;
+};
+PGN_DEVICE void decay_sums(const float* __restrict__ la, int n, Decays& d) {
   const int t = threadIdx.x;
   if (t < CT) {
     const float f = t < n ? la[t] : 0.f;
-    double v = (double)f < kLaMin ? kLaMin : (double)f;
+    const bool ok = f < INFINITY;
+    double v = ok ? ((double)f < kLaMin ? kLaMin : (double)f) : 0.;
 #pragma unroll
     for (int s = 1; s < CT; s <<= 1) {
       const double y = __shfl_up(v, s);
       if (t >= s) v += y;
     }
-    Ls[t] = v;
+    d.L[t] = v;
+    const unsigned long long b = __ballot(!ok);
+    if (t == 0) d.bad = b;
   }
 }
 
-PGN_DEVICE float decay(const double* Ls, int t, int s) { return expf((float)(Ls[t] - Ls[s])); }
+// The decay from after token s to token t >= s, and from the chunk's start to token t
+PGN_DEVICE float decay(const Decays& d, int t, int s) {
+  const float v = expf((float)(d.L[t] - d.L[s]));
+  return d.bad != 0 && (d.bad >> s >> 1 & ((1ull << (t - s)) - 1)) != 0 ? NAN : v;
+}
+PGN_DEVICE float decay_from_start(const Decays& d, int t) {
+  const float v = expf((float)d.L[t]);
+  return (d.bad & (~0ull >> (63 - t))) != 0 ? NAN : v;
+}
 
 struct Shape {
   int BH, T, Dk, Dv, NC, DkP, nkt, nvt;  // nkt, nvt: 64-wide key and value tiles; DkP: Dk rounded up to 16
@@ -247,7 +302,7 @@ __global__ __launch_bounds__(256) void exact_scores(const float* __restrict__ q,
                                                     float* __restrict__ wt, float* __restrict__ M,
                                                     float* __restrict__ X, Shape s) {
   __shared__ __align__(16) float lds[4 * kSlice];
-  __shared__ double Ls[CT];
+  __shared__ Decays Ls;
   __shared__ float bes[CT];
   const WaveIdx x = wave_idx();
   const int tid = threadIdx.x, bh = blockIdx.x / s.NC, c = blockIdx.x - bh * s.NC;
@@ -294,7 +349,7 @@ __global__ __launch_bounds__(256) void exact_scores(const float* __restrict__ q,
   }
   __syncthreads();
   if (tid < CT) {
-    eL[ch * CT + tid] = expf((float)Ls[tid]);
+    eL[ch * CT + tid] = decay_from_start(Ls, tid);
     wt[ch * CT + tid] = decay(Ls, CT - 1, tid);
   }
   float* Ac = A + ch * CT * CT;
@@ -305,7 +360,7 @@ __global__ __launch_bounds__(256) void exact_scores(const float* __restrict__ q,
     each(ak, x, [&](int t, int u, float v) {
       const float m = t > u ? v * decay(Ls, t, u) : 0.f;
       Mc[t * CT + u] = m;
-      Nt[t * PR + u] = m * bes[u];
+      Nt[t * PR + u] = t > u ? m * bes[u] : 0.f;
       Xt[t * PR + u] = 0.f;
     });
     __syncthreads();
@@ -321,7 +376,7 @@ __global__ __launch_bounds__(256) void exact_scores(const float* __restrict__ q,
 #pragma unroll
         for (int m = 0; 4 * m < t; ++m) nr[m] = *reinterpret_cast<const f32x4*>(Nt + (b + t) * PR + b + 4 * m);
 #pragma unroll
-        for (int u = 0; u < t; ++u) v[t] -= nr[u >> 2][u & 3] * v[u];
+        for (int u = 0; u < t; ++u) v[t] -= (u >= x.i ? nr[u >> 2][u & 3] : 0.f) * v[u];  // v[u] = 0 above the diagonal
       }
       if (x.l < 16) {
 #pragma unroll
@@ -338,7 +393,33 @@ __global__ __launch_bounds__(256) void exact_scores(const float* __restrict__ q,
       if (i < 4) {
         f32x4 t = zero4();
         for (int m = j; m < i; ++m) t = mfma16(rows16(Nt, i, m), frag<kCols>(Xt + 16 * m * PR, 16 * j, 0, x), t);
-        const f32x4 y = mfma16(rows16(Xt, i, i), t, zero4());
+        bool bad = false;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) bad |= !(fabsf(t[e]) < INFINITY);
+        const bool careful = __any(bad);  // own_tokens for the blocks' triangular operands, X_jj and X_ii
+        if (careful) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            float f = 0.f;
+            for (int u = 16 * j + x.i; u < 16 * i; ++u)
+              f += Nt[(16 * i + 4 * x.g + e) * PR + u] * Xt[u * PR + 16 * j + x.i];
+            t[e] = f;
+          }
+        }
+        f32x4 y = mfma16(rows16(Xt, i, i), t, zero4());
+        bool bady = careful;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) bady |= !(fabsf(y[e]) < INFINITY);
+        if (__any(bady)) {
+          y = zero4();
+#pragma unroll
+          for (int u = 0; u < 16; ++u) {
+            const float tu = __shfl(t[u & 3], x.i + 16 * (u >> 2));
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (u <= 4 * x.g + e) y[e] += Xt[(16 * i + 4 * x.g + e) * PR + 16 * i + u] * tu;
+          }
+        }
 #pragma unroll
         for (int e = 0; e < 4; ++e) Xt[(16 * i + 4 * x.g + e) * PR + 16 * j + x.i] = -y[e];
       }
@@ -370,6 +451,12 @@ __global__ __launch_bounds__(256) void exact_wy_fwd(const float* __restrict__ k,
   product<kRows, kCols, true, VEC>(acc, Src{X + ch * CT * CT, CT, CT, CT},
                                    Src{(val ? v : k) + row0 * D + n0, D, D - n0, n}, n, lds, buf, x,
                                    val ? nullptr : eL + ch * CT);
+  {
+    const float *Xc = X + ch * CT * CT, *vk = (val ? v : k) + row0 * D + n0, *el = eL + ch * CT;
+    own_tokens<true>(
+        acc, n, D - n0, x, [&](int r, int m) { return Xc[r * CT + m]; },
+        [&](int m, int cc) { return (val ? 1.f : el[m]) * vk[(size_t)m * D + cc]; });
+  }
   if (val)
     store_tile(acc, R + row0 * D + n0, D, n, D - n0, x);
   else
@@ -704,8 +791,14 @@ __global__ __launch_bounds__(256) void exact_out(const float* __restrict__ q, co
   product<kRows, kCols, VEC, VEC>(acc, Src{q + row0 * s.Dk, s.Dk, n, s.Dk},
                                   Src{Sc + ch * s.Dk * s.Dv + n0, s.Dv, s.Dv - n0, s.Dk}, s.Dk, lds, buf, x);
   scale_rows(acc, eL + ch * CT, x);
-  product<kRows, kCols, true, VEC>(acc, Src{A + ch * CT * CT, CT, n, CT},
-                                   Src{u + row0 * s.Dv + n0, s.Dv, s.Dv - n0, n}, n, lds, buf, x);
+  const float *Ac = A + ch * CT * CT, *uc = u + row0 * s.Dv + n0;
+  f32x4 au[2][2];
+  clear(au);
+  product<kRows, kCols, true, VEC>(au, Src{Ac, CT, n, CT}, Src{uc, s.Dv, s.Dv - n0, n}, n, lds, buf, x);
+  own_tokens<true>(
+      au, n, s.Dv - n0, x, [&](int r, int m) { return Ac[r * CT + m]; },
+      [&](int m, int cc) { return uc[(size_t)m * s.Dv + cc]; });
+  add(acc, au);
   store_tile(acc, o + row0 * s.Dv + n0, s.Dv, n, s.Dv - n0, x);
 }
 
@@ -734,13 +827,20 @@ __global__ __launch_bounds__(256) void exact_wy_bwd(const float* __restrict__ k,
   clear(acc);
   int buf = 0;
   if (!val) {
-    product<kCols, kCols, true, VEC>(acc, Xt, Src{k + row0 * s.Dk + n0, s.Dk, s.Dk - n0, n}, n, lds, buf, x, sc);
+    const float* kc = k + row0 * s.Dk + n0;
+    product<kCols, kCols, true, VEC>(acc, Xt, Src{kc, s.Dk, s.Dk - n0, n}, n, lds, buf, x, sc);
+    own_tokens<false>(
+        acc, n, s.Dk - n0, x, [&](int r, int m) { return Xt.p[m * CT + r]; },
+        [&](int m, int cc) { return sc[m] * kc[(size_t)m * s.Dk + cc]; });
     store_tile(acc, W + ch * CT * s.DkP + n0, s.DkP, CT, s.DkP - n0, x);
     return;
   }
   const int nc = s.Dv - n0;
-  product<kCols, kCols, true, VEC>(acc, Src{A + ch * CT * CT, CT, CT, n},
-                                   Src{dO + row0 * s.Dv + n0, s.Dv, nc, n}, n, lds, buf, x);
+  const float *Ac = A + ch * CT * CT, *doc = dO + row0 * s.Dv + n0;
+  product<kCols, kCols, true, VEC>(acc, Src{Ac, CT, CT, n}, Src{doc, s.Dv, nc, n}, n, lds, buf, x);
+  own_tokens<false>(
+      acc, n, nc, x, [&](int r, int m) { return Ac[m * CT + r]; },
+      [&](int m, int cc) { return doc[(size_t)m * s.Dv + cc]; });
   scale_rows(acc, sc, x);
   each(acc, x, [&](int r, int cc, float v) { tile[r * PR + cc] = v; });
   f32x4 rx[2];
@@ -763,12 +863,16 @@ __global__ __launch_bounds__(256) void exact_wy_bwd(const float* __restrict__ k,
       for (int j = 0; j < 2; ++j) acc[i][j] = mfma16(a, frag<kCols>(tile, c0 + 16 * j, kk, x), acc[i][j]);
     }
   }
+  own_tokens<false>(
+      acc, CT, nc, x, [&](int r, int m) { return Xt.p[m * CT + r]; },
+      [&](int m, int cc) { return tile[m * PR + cc]; });
   store_tile(acc, y + row0 * s.Dv + n0, s.Dv, n, nc, x);
 }
 
 // ------------------------------------------------------------------------------------------------------------------
-// Backward, per chunk: dA = tril(dO U^T o D) (before D: its products with A give the decay gradient's row and column
-// sums, into rc), and for the delta rule P + P^T, Z's sums and dbeta's second term (into db).
+// Backward, per chunk: dA = tril(dO U^T o D) (before D: its products with A give the decay gradient's sums over the
+// pairs of tokens on either side of each, into rc), and for the delta rule P + P^T, Z's sums and dbeta's second term
+// (into db).
 template <bool DELTA, bool VEC>
 __global__ __launch_bounds__(256) void exact_scores_bwd(const float* __restrict__ dO, const float* __restrict__ u,
                                                         const float* __restrict__ dY, const float* __restrict__ R,
@@ -777,7 +881,7 @@ __global__ __launch_bounds__(256) void exact_scores_bwd(const float* __restrict_
                                                         float* __restrict__ dA, float* __restrict__ Psym,
                                                         float* __restrict__ rc, float* __restrict__ db, Shape s) {
   __shared__ __align__(16) float lds[4 * kSlice];
-  __shared__ double Ls[CT];
+  __shared__ Decays Ls;
   __shared__ float bes[CT];
   const WaveIdx x = wave_idx();
   const int tid = threadIdx.x, bh = blockIdx.x / s.NC, c = blockIdx.x - bh * s.NC;
@@ -812,14 +916,33 @@ __global__ __launch_bounds__(256) void exact_scores_bwd(const float* __restrict_
   __syncthreads();
   {
     const int r = tid >> 2, m = tid & 3;
-    float row = 0.f, cl = 0.f, cf = 0.f;
+    // row r's sums up to, not including, each column: within the thread's 16, then over the four threads of the row
+    f32x4 v[4];
+    float run = 0.f, cf = 0.f;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const f32x4 w = *reinterpret_cast<const f32x4*>(E + r * PR + 16 * m + 4 * e);
+#pragma unroll
+      for (int z = 0; z < 4; ++z) {
+        v[e][z] = run;
+        run += w[z];
+      }
+    }
+    float before = 0.f;
+#pragma unroll
+    for (int z = 1; z < 4; ++z) {
+      const float y = __shfl_up(run, z);
+      if (m >= z) before += y;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) *reinterpret_cast<f32x4*>(E + r * PR + 16 * m + 4 * e) = v[e] + before;
+    __syncthreads();
+    float d = 0.f;  // column r, the rows from r on
 #pragma unroll
     for (int e = 0; e < 16; ++e) {
-      row += E[r * PR + 4 * e + m];
-      cl += E[(4 * e + m) * PR + r];
+      if (4 * e + m >= r) d += E[(4 * e + m) * PR + r];
       if (DELTA) cf += F[(4 * e + m) * PR + r];
     }
-    float d = row - cl;
     d = group_sum<4>(d);
     cf = group_sum<4>(cf);
     if (m == 0) {
@@ -842,7 +965,7 @@ __global__ __launch_bounds__(256) void exact_scores_bwd(const float* __restrict_
 // Gradients, per chunk and 64 columns, the tiles of dV (delta: dU, only for its row products with R), dQ and dK.
 // Partial sums, one a (tile, wave column): q . dQ's state term, k . (w o U G^T), k . (e^L o dY S^T), R . dU.
 template <bool DELTA, bool VEC>
-__global__ __launch_bounds__(256) void exact_grads(
+__global__ __launch_bounds__(256, DELTA ? 3 : 4) void exact_grads(
     const float* __restrict__ q, const float* __restrict__ k, const float* __restrict__ u,
     const float* __restrict__ R, const float* __restrict__ dO, const float* __restrict__ dY,
     const float* __restrict__ A, const float* __restrict__ dA, const float* __restrict__ Psym,
@@ -857,15 +980,21 @@ __global__ __launch_bounds__(256) void exact_grads(
   const size_t row0 = (size_t)bh * s.T + t0, ch = it.group, tot = (size_t)s.BH * s.NC * CT;
   const float *Sp = Sc + ch * s.Dk * s.Dv, *Gp = G + ch * s.Dk * s.Dv;
   const float *Ac = A + ch * CT * CT, *dAc = dA + ch * CT * CT;
-  f32x4 acc[2][2];
+  f32x4 acc[2][2], tri[2][2];
   clear(acc);
+  clear(tri);
   int buf = 0;
   if (it.sub >= 2 * s.nkt) {
     const int tile = it.sub - 2 * s.nkt, n0 = 64 * tile, nc = s.Dv - n0;
     product<kRows, kCols, VEC, VEC>(acc, Src{k + row0 * s.Dk, s.Dk, n, s.Dk}, Src{Gp + n0, s.Dv, nc, s.Dk}, s.Dk, lds,
                                     buf, x);
     scale_rows(acc, wt + ch * CT, x);
-    product<kCols, kCols, true, VEC>(acc, Src{Ac, CT, CT, n}, Src{dO + row0 * s.Dv + n0, s.Dv, nc, n}, n, lds, buf, x);
+    const float* doc = dO + row0 * s.Dv + n0;
+    product<kCols, kCols, true, VEC>(tri, Src{Ac, CT, CT, n}, Src{doc, s.Dv, nc, n}, n, lds, buf, x);
+    own_tokens<false>(
+        tri, n, nc, x, [&](int r, int m) { return Ac[m * CT + r]; },
+        [&](int m, int cc) { return doc[(size_t)m * s.Dv + cc]; });
+    add(acc, tri);
     if constexpr (DELTA)
       row_dots(acc, R + row0 * s.Dv + n0, s.Dv, n, nc, pb + (size_t)(2 * tile + (x.w & 1)) * tot + ch * CT, x);
     else
@@ -882,7 +1011,11 @@ __global__ __launch_bounds__(256) void exact_grads(
                                     Src{Sp + (size_t)n0 * s.Dv, s.Dv, nc, s.Dv}, s.Dv, lds, buf, x);
     scale_rows(acc, eL + ch * CT, x);
     row_dots(acc, qt, s.Dk, n, nc, pq + slot, x);
-    product<kRows, kCols, true, VEC>(acc, Src{dAc, CT, n, CT}, Src{kt, s.Dk, nc, n}, n, lds, buf, x);
+    product<kRows, kCols, true, VEC>(tri, Src{dAc, CT, n, CT}, Src{kt, s.Dk, nc, n}, n, lds, buf, x);
+    own_tokens<true>(
+        tri, n, nc, x, [&](int r, int m) { return dAc[r * CT + m]; },
+        [&](int m, int cc) { return kt[(size_t)m * s.Dk + cc]; });
+    add(acc, tri);
     store_tile(acc, dq + row0 * s.Dk + n0, s.Dk, n, nc, x);
     return;
   }
@@ -903,11 +1036,16 @@ __global__ __launch_bounds__(256) void exact_grads(
       for (int j = 0; j < 2; ++j) acc[i][j] -= ay[i][j];
     product<kRows, kCols, true, VEC>(acc, Src{Psym + ch * CT * CT, CT, CT, CT}, Src{kt, s.Dk, nc, n}, n, lds, buf, x);
   }
-  product<kCols, kCols, true, VEC>(acc, Src{dAc, CT, CT, n}, Src{q + row0 * s.Dk + n0, s.Dk, nc, n}, n, lds, buf, x);
+  const float* qt = q + row0 * s.Dk + n0;
+  product<kCols, kCols, true, VEC>(tri, Src{dAc, CT, CT, n}, Src{qt, s.Dk, nc, n}, n, lds, buf, x);
+  own_tokens<false>(
+      tri, n, nc, x, [&](int r, int m) { return dAc[m * CT + r]; },
+      [&](int m, int cc) { return qt[(size_t)m * s.Dk + cc]; });
+  add(acc, tri);
   store_tile(acc, dk + row0 * s.Dk + n0, s.Dk, n, nc, x);
 }
 
-// dla and dbeta from the partial sums, one wave a chunk; the suffix sums in fp64.
+// dla and dbeta from the partial sums, one wave a chunk; the sums from each token on and before it in fp64.
 template <bool DELTA>
 __global__ __launch_bounds__(64) void exact_gates_bwd(const float* __restrict__ rc, const float* __restrict__ db,
                                                       const float* __restrict__ pq, const float* __restrict__ pk,
@@ -916,27 +1054,28 @@ __global__ __launch_bounds__(64) void exact_gates_bwd(const float* __restrict__ 
                                                       float* __restrict__ dbeta, Shape s) {
   const int t = threadIdx.x, bh = blockIdx.x / s.NC, c = blockIdx.x - bh * s.NC, n = min(CT, s.T - c * CT);
   const size_t ch = blockIdx.x, tot = (size_t)s.BH * s.NC * CT, at = ch * CT + t;
-  double d = rc[at], kg = 0., b = DELTA ? db[at] : 0.;
+  double from = 0., before = 0., b = DELTA ? db[at] : 0., end = 0.;
   for (int m = 0; m < 2 * s.nkt; ++m) {
-    d += pq[m * tot + at];
-    kg += pk[m * tot + at];
-    if (DELTA) d -= py[m * tot + at];
+    from += pq[m * tot + at];
+    before += pk[m * tot + at];
+    if (DELTA) from -= py[m * tot + at];
   }
   if (DELTA)
     for (int m = 0; m < 2 * s.nvt; ++m) b += pb[m * tot + at];
-  d -= kg;
-  double end = kg;
   for (int m = t; m < nhs; m += 64) end += hs[ch * nhs + m];
 #pragma unroll
   for (int m = 1; m < 64; m <<= 1) end += __shfl_xor(end, m);
 #pragma unroll
   for (int m = 1; m < 64; m <<= 1) {
-    const double y = __shfl_down(d, m);
-    if (t + m < 64) d += y;
+    const double y = __shfl_down(from, m), z = __shfl_up(before, m);
+    if (t + m < 64) from += y;
+    if (t >= m) before += z;
   }
+  before = __shfl_up(before, 1);
+  if (t == 0) before = 0.;
   if (t < n) {
     const size_t row = (size_t)bh * s.T + c * CT + t;
-    dla[row] = (float)(d + end);
+    dla[row] = (float)((double)rc[at] + (from + before) + end);
     if (DELTA) dbeta[row] = (float)b;
   }
 }

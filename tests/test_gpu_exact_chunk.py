@@ -84,3 +84,28 @@ def test_chunked_off_16_byte_addresses(delta):
         buf[1:] = t.reshape(-1).cuda()
         return buf[1:].view(t.shape).detach()
     _check(*_inputs(1, 2, 100, 64, 48, delta, seed=13, s0=True), place=shifted)
+
+
+@pytest.mark.parametrize("delta,name", [(r, n) for r in (False, True) for n in "q k v la beta S0 do dS".split()
+                                        if r or n != "beta"])
+def test_chunked_non_finite_values_stay_where_the_recurrence_takes_them(delta, name, monkeypatch):
+    """An infinity or a NaN in one place of one operand: every output that is finite token by token is finite here, and
+    the same, and no other one is (ragged rows and tiles; tokens at a chunk's start, inside blocks and at the end)."""
+    from pragnosia_amd import ops
+    B, H, T, Dk, Dv = 1, 2, 150, 34, 70
+    x, do, dS = _inputs(B, H, T, Dk, Dv, delta, seed=17, s0=True)
+
+    def run(a, min_t):
+        monkeypatch.setattr(ops, "EXACT_CHUNK_MIN_T", min_t)
+        args = (a["q"], a["k"], a["v"], a["la"], a.get("beta"))
+        o, S, ckpt, resid = ops.aspin_exact(*args, a["S0"], True)
+        return o, S, *ops.aspin_exact_bwd(*args, ckpt, resid if resid.numel() else None, a["do"], a["dS"])
+
+    for val in (float("inf"), float("nan")):
+        for s in (64, 90, 149) if name not in ("S0", "dS") else (3,):
+            a = {n: t.clone().cuda() for n, t in {**x, "do": do, "dS": dS}.items()}
+            a[name][(0, 1, s) if name in ("la", "beta") else (0, 1, s, 7)] = val
+            for n, got, want in zip("o S dq dk dv dla dbeta dS0".split(), run(a, 32), run(a, 1 << 30)):
+                fine = want.isfinite()
+                assert torch.equal(got.isfinite(), fine), (val, s, n, (got.isfinite() != fine).nonzero()[:4])
+                assert not fine.any() or (got - want)[fine].abs().max() < TOL * want[fine].abs().max(), (val, s, n)
