@@ -237,16 +237,19 @@ int pragnosia_aspin_exact_bwd(const void* q, const void* k, const void* v, const
                               int64_t Dk, int64_t Dv, int dtype, void* stream);
 
 /* The exact scan's function in chunked form (64-token chunks, fp32 matrix cores), fp32 only: the plain rule when beta
- * is NULL (any Dk, Dv), the delta rule when given (Dk <= 384). Layouts as pragnosia_aspin_exact_fwd. With NC =
- * ceil(T / 64), the forward also writes, for the backward and for itself (all required): states (B, H, NC, Dk, Dv), the
- * state entering every chunk; scores (B, H, NC, 64, 64); gates (2, B, H, NC, 64), the decays from a chunk's start and to
- * its end; and for the delta rule M and X (B, H, NC, 64, 64), R and U (B, H, T, Dv) and the scratch W (B, H, NC, 64, Dk
- * rounded up to 16). scores, gates, M, X and W are 16-byte aligned; the other arrays need no more than a float's
- * alignment (16-byte loads are used when all of them have it and Dk and Dv are multiples of 4). */
+ * is NULL (any Dk, Dv), the delta rule when given (Dk <= 384). Layouts as pragnosia_aspin_exact_fwd. Runs the N chunks
+ * (`chunks`) of every sequence from chunk `first` on: S0 enters the first of them and S_final leaves the last (the two
+ * may be one array), so a sequence can be run in pieces. It also writes (all required) states (B, H, N, Dk, Dv), the
+ * state entering every chunk; scores (B, H, N, 64, 64); gates (2, B, H, N, 64), the decays from a chunk's start and to
+ * its end; and for the delta rule M and X (B, H, N, 64, 64), R and U (B, H, N, 64, Dv) and the scratch W (B, H, N, 64,
+ * Dk rounded up to 16); the backward reads those of all chunks. scores, gates, M, X and W are 16-byte aligned; the other
+ * arrays need no more than a float's alignment (16-byte loads are used when all of them have it and Dk and Dv are
+ * multiples of 4). */
 int pragnosia_aspin_exact_chunk_fwd(const float* q, const float* k, const float* v, const float* la, const float* beta,
                                     const float* S0, float* o, float* S_final, float* states, float* scores,
                                     float* gates, float* M, float* X, float* R, float* U, float* W, int64_t B,
-                                    int64_t H, int64_t T, int64_t Dk, int64_t Dv, void* stream);
+                                    int64_t H, int64_t T, int64_t Dk, int64_t Dv, int64_t first, int64_t chunks,
+                                    void* stream);
 
 /* Bytes of the backward's workspace (16-byte aligned), or -1 for a shape it refuses; delta != 0 for the delta rule. */
 int64_t pragnosia_aspin_exact_chunk_bwd_workspace_bytes(int64_t B, int64_t H, int64_t T, int64_t Dk, int64_t Dv,

@@ -41,7 +41,7 @@ SIGNATURES = {
     "pragnosia_aspin_out_bwd": [_p, _i32] + [_p] * 5 + [_i64] * 4 + [_p],
     "pragnosia_aspin_exact_fwd": [_p] * 10 + [_i64] * 5 + [_i32, _p],
     "pragnosia_aspin_exact_bwd": [_p] * 15 + [_i64] * 5 + [_i32, _p],
-    "pragnosia_aspin_exact_chunk_fwd": [_p] * 16 + [_i64] * 5 + [_p],
+    "pragnosia_aspin_exact_chunk_fwd": [_p] * 16 + [_i64] * 7 + [_p],
     "pragnosia_aspin_exact_chunk_bwd_workspace_bytes": [_i64] * 5 + [_i32],
     "pragnosia_aspin_exact_chunk_bwd": [_p] * 21 + [_i64] * 6 + [_p],
     "pragnosia_aspin_delta_fwd": [_p] * 11 + [_i64] * 5 + [_p],

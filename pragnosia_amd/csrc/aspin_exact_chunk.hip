@@ -279,7 +279,9 @@ PGN_DEVICE float decay_from_start(const Decays& d, int t) {
 }
 
 struct Shape {
-  int BH, T, Dk, Dv, NC, DkP, nkt, nvt;  // nkt, nvt: 64-wide key and value tiles; DkP: Dk rounded up to 16
+  // NC chunks of each sequence, from chunk c0 on; nkt, nvt: 64-wide key and value tiles; DkP: Dk rounded up to 16
+  int BH, T, Dk, Dv, NC, DkP, nkt, nvt, c0;
+  PGN_DEVICE int token(int c) const { return (c0 + c) * CT; }  // the first of the c-th chunk
 };
 
 // Work items numbered so that a group's items run on one XCD (workgroup i runs on XCD i mod 8) and share its L2:
@@ -306,7 +308,7 @@ __global__ __launch_bounds__(256) void exact_scores(const float* __restrict__ q,
   __shared__ float bes[CT];
   const WaveIdx x = wave_idx();
   const int tid = threadIdx.x, bh = blockIdx.x / s.NC, c = blockIdx.x - bh * s.NC;
-  const int t0 = c * CT, n = min(CT, s.T - t0);
+  const int t0 = s.token(c), n = min(CT, s.T - t0);
   const size_t row0 = (size_t)bh * s.T + t0, ch = (size_t)bh * s.NC + c;
   decay_sums(la + row0, n, Ls);
   if (DELTA && tid < CT) bes[tid] = tid < n ? beta[row0 + tid] : 0.f;
@@ -441,7 +443,7 @@ __global__ __launch_bounds__(256) void exact_wy_fwd(const float* __restrict__ k,
   const WaveIdx x = wave_idx();
   const Item it = item_of(blockIdx.x, s.nvt + s.nkt);
   if (it.group >= s.BH * s.NC) return;
-  const int bh = it.group / s.NC, c = it.group - bh * s.NC, t0 = c * CT, n = min(CT, s.T - t0);
+  const int bh = it.group / s.NC, c = it.group - bh * s.NC, t0 = s.token(c), n = min(CT, s.T - t0);
   const size_t row0 = (size_t)bh * s.T + t0, ch = it.group;
   const bool val = it.sub < s.nvt;
   const int n0 = 64 * (val ? it.sub : it.sub - s.nvt), D = val ? s.Dv : s.Dk;
@@ -458,7 +460,7 @@ __global__ __launch_bounds__(256) void exact_wy_fwd(const float* __restrict__ k,
         [&](int m, int cc) { return (val ? 1.f : el[m]) * vk[(size_t)m * D + cc]; });
   }
   if (val)
-    store_tile(acc, R + row0 * D + n0, D, n, D - n0, x);
+    store_tile(acc, R + ch * CT * D + n0, D, n, D - n0, x);
   else
     store_tile(acc, W + ch * CT * s.DkP + n0, s.DkP, CT, s.DkP - n0, x);
 }
@@ -496,8 +498,8 @@ PGN_DEVICE unsigned row_step(int p, int ld4) { return (unsigned)((16 * (p >> 2) 
 template <int KT, bool BWD>
 __global__ __launch_bounds__(256) void exact_chain_plain(const float* __restrict__ xk, const float* __restrict__ yv,
                                                          const float* __restrict__ f, const float* __restrict__ eL,
-                                                         const float* __restrict__ init, float* __restrict__ states,
-                                                         float* __restrict__ last, const float* __restrict__ Sc,
+                                                         const float* init, float* __restrict__ states,
+                                                         float* last, const float* __restrict__ Sc,
                                                          float* __restrict__ hs, int nvb, int nkb, Shape s) {
   const WaveIdx x = wave_idx();
   const Item it = item_of(blockIdx.x, nvb * nkb);
@@ -528,7 +530,7 @@ __global__ __launch_bounds__(256) void exact_chain_plain(const float* __restrict
   };
   auto load = [&](Set& u, int c) {
     if (c < 0 || c >= s.NC) return;
-    const int t0 = c * CT, n = min(CT, s.T - t0);
+    const int t0 = s.token(c), n = min(CT, s.T - t0);
     const size_t row0 = (size_t)bh * s.T + t0, ch = (size_t)bh * s.NC + c;
     const __amdgpu_buffer_rsrc_t kr = view(xk + row0 * s.Dk, n * s.Dk), vr = view(yv + row0 * s.Dv, n * s.Dv);
     const unsigned vo = fresh(vbase);
@@ -610,8 +612,8 @@ template <int KT, bool BWD>
 __global__ __launch_bounds__(256, KT == 1 || (KT <= 3 && !BWD) ? 2 : 1) void exact_chain_delta(
     const float* __restrict__ k, const float* __restrict__ q, const float* __restrict__ dO,
     const float* __restrict__ beta, const float* __restrict__ eL, const float* __restrict__ wt,
-    const float* __restrict__ W, float* __restrict__ y, float* __restrict__ U, const float* __restrict__ init,
-    float* __restrict__ states, float* __restrict__ last, const float* __restrict__ Sc, float* __restrict__ hs,
+    const float* __restrict__ W, float* __restrict__ y, float* __restrict__ U, const float* init,
+    float* __restrict__ states, float* last, const float* __restrict__ Sc, float* __restrict__ hs,
     int nvb, Shape s) {
   __shared__ f32x4 part[4][4][64];
   __shared__ f32x4 us[4][64];
@@ -651,9 +653,9 @@ __global__ __launch_bounds__(256, KT == 1 || (KT <= 3 && !BWD) ? 2 : 1) void exa
     }
   };
   auto load_y = [&](int c) {
-    const int t0 = c * CT, n = min(CT, s.T - t0);
-    const size_t row0 = (size_t)bh * s.T + t0;
-    const __amdgpu_buffer_rsrc_t r = view(y + row0 * s.Dv, n * s.Dv), br = view(BWD ? wt : beta + row0, BWD ? 0 : n);
+    const int t0 = s.token(c), n = min(CT, s.T - t0);
+    const size_t row0 = (size_t)bh * s.T + t0, yrow = BWD ? row0 : ((size_t)bh * s.NC + c) * CT;
+    const __amdgpu_buffer_rsrc_t r = view(y + yrow * s.Dv, n * s.Dv), br = view(BWD ? wt : beta + row0, BWD ? 0 : n);
     const unsigned o = fresh(ybase);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -662,7 +664,7 @@ __global__ __launch_bounds__(256, KT == 1 || (KT <= 3 && !BWD) ? 2 : 1) void exa
     }
   };
   auto load_k = [&](int c) {
-    const int t0 = c * CT, n = min(CT, s.T - t0);
+    const int t0 = s.token(c), n = min(CT, s.T - t0);
     const size_t row0 = (size_t)bh * s.T + t0, ch = (size_t)bh * s.NC + c;
     const __amdgpu_buffer_rsrc_t kr = view(k + row0 * s.Dk, n * s.Dk);
 #pragma unroll
@@ -698,7 +700,7 @@ __global__ __launch_bounds__(256, KT == 1 || (KT <= 3 && !BWD) ? 2 : 1) void exa
   for (int i = 0; i < s.NC; ++i) {
     const int c = first + dir * i;
     const bool more = i + 1 < s.NC;
-    const int t0 = c * CT, n = min(CT, s.T - t0);
+    const int t0 = s.token(c), n = min(CT, s.T - t0);
     const size_t row0 = (size_t)bh * s.T + t0, ch = (size_t)bh * s.NC + c;
     f32x4 P[4] = {zero4(), zero4(), zero4(), zero4()};
 #pragma unroll
@@ -719,7 +721,7 @@ __global__ __launch_bounds__(256, KT == 1 || (KT <= 3 && !BWD) ? 2 : 1) void exa
     {
       const f32x4 sum = (part[0][x.w][x.l] + part[1][x.w][x.l]) + (part[2][x.w][x.l] + part[3][x.w][x.l]);
       const f32x4 v = BWD ? yo + sum : yo - sum;
-      const __amdgpu_buffer_rsrc_t yr = view(y + row0 * s.Dv, n * s.Dv);
+      const __amdgpu_buffer_rsrc_t yr = view(y + (BWD ? row0 : ch * CT) * s.Dv, n * s.Dv);
       const unsigned o = fresh(ybase);
 #pragma unroll
       for (int e = 0; e < 4; ++e) bstore(yr, o + e * vd4, v[e]);
@@ -727,7 +729,7 @@ __global__ __launch_bounds__(256, KT == 1 || (KT <= 3 && !BWD) ? 2 : 1) void exa
         us[x.w][x.l] = v;
       } else {
         const f32x4 u = v * bo;
-        const __amdgpu_buffer_rsrc_t ur = view(U + row0 * s.Dv, n * s.Dv);
+        const __amdgpu_buffer_rsrc_t ur = view(U + ch * CT * s.Dv, n * s.Dv);
 #pragma unroll
         for (int e = 0; e < 4; ++e) bstore(ur, o + e * vd4, u[e]);
         us[x.w][x.l] = u;
@@ -774,16 +776,17 @@ __global__ __launch_bounds__(256, KT == 1 || (KT <= 3 && !BWD) ? 2 : 1) void exa
 }
 
 // ------------------------------------------------------------------------------------------------------------------
-// Outputs, per chunk and 64 value columns: O = e^L o (Q S) + A U.
+// Outputs, per chunk and 64 value columns: O = e^L o (Q S) + A U (delta: u = U, a chunk's rows together; else V).
 template <bool VEC>
 __global__ __launch_bounds__(256) void exact_out(const float* __restrict__ q, const float* __restrict__ u,
                                                  const float* __restrict__ A, const float* __restrict__ eL,
-                                                 const float* __restrict__ Sc, float* __restrict__ o, Shape s) {
+                                                 const float* __restrict__ Sc, float* __restrict__ o, bool delta,
+                                                 Shape s) {
   __shared__ __align__(16) float lds[4 * kSlice];
   const WaveIdx x = wave_idx();
   const Item it = item_of(blockIdx.x, s.nvt);
   if (it.group >= s.BH * s.NC) return;
-  const int bh = it.group / s.NC, c = it.group - bh * s.NC, t0 = c * CT, n = min(CT, s.T - t0), n0 = 64 * it.sub;
+  const int bh = it.group / s.NC, c = it.group - bh * s.NC, t0 = s.token(c), n = min(CT, s.T - t0), n0 = 64 * it.sub;
   const size_t row0 = (size_t)bh * s.T + t0, ch = it.group;
   f32x4 acc[2][2];
   clear(acc);
@@ -791,7 +794,7 @@ __global__ __launch_bounds__(256) void exact_out(const float* __restrict__ q, co
   product<kRows, kCols, VEC, VEC>(acc, Src{q + row0 * s.Dk, s.Dk, n, s.Dk},
                                   Src{Sc + ch * s.Dk * s.Dv + n0, s.Dv, s.Dv - n0, s.Dk}, s.Dk, lds, buf, x);
   scale_rows(acc, eL + ch * CT, x);
-  const float *Ac = A + ch * CT * CT, *uc = u + row0 * s.Dv + n0;
+  const float *Ac = A + ch * CT * CT, *uc = u + (delta ? ch * CT : row0) * s.Dv + n0;
   f32x4 au[2][2];
   clear(au);
   product<kRows, kCols, true, VEC>(au, Src{Ac, CT, n, CT}, Src{uc, s.Dv, s.Dv - n0, n}, n, lds, buf, x);
@@ -886,17 +889,17 @@ __global__ __launch_bounds__(256) void exact_scores_bwd(const float* __restrict_
   const WaveIdx x = wave_idx();
   const int tid = threadIdx.x, bh = blockIdx.x / s.NC, c = blockIdx.x - bh * s.NC;
   const int t0 = c * CT, n = min(CT, s.T - t0);
-  const size_t row0 = (size_t)bh * s.T + t0, ch = (size_t)bh * s.NC + c;
+  const size_t row0 = (size_t)bh * s.T + t0, ch = (size_t)bh * s.NC + c, urow = DELTA ? ch * CT : row0;
   decay_sums(la + row0, n, Ls);
   if (DELTA && tid < CT) bes[tid] = tid < n ? beta[row0 + tid] : 0.f;
   f32x4 a1[2][2], a2[2][2];
   clear(a1);
   clear(a2);
   int buf = 0;
-  product<kRows, kRows, VEC, VEC>(a1, Src{dO + row0 * s.Dv, s.Dv, n, s.Dv}, Src{u + row0 * s.Dv, s.Dv, n, s.Dv}, s.Dv,
+  product<kRows, kRows, VEC, VEC>(a1, Src{dO + row0 * s.Dv, s.Dv, n, s.Dv}, Src{u + urow * s.Dv, s.Dv, n, s.Dv}, s.Dv,
                                   lds, buf, x);
   if constexpr (DELTA)
-    product<kRows, kRows, VEC, VEC>(a2, Src{dY + row0 * s.Dv, s.Dv, n, s.Dv}, Src{R + row0 * s.Dv, s.Dv, n, s.Dv},
+    product<kRows, kRows, VEC, VEC>(a2, Src{dY + row0 * s.Dv, s.Dv, n, s.Dv}, Src{R + urow * s.Dv, s.Dv, n, s.Dv},
                                     s.Dv, lds, buf, x);
   __syncthreads();
   float *E = lds, *F = lds + CT * PR;  // the decay gradient's matrix; dY R^T o M
@@ -978,6 +981,7 @@ __global__ __launch_bounds__(256, DELTA ? 3 : 4) void exact_grads(
   if (it.group >= s.BH * s.NC) return;
   const int bh = it.group / s.NC, c = it.group - bh * s.NC, t0 = c * CT, n = min(CT, s.T - t0);
   const size_t row0 = (size_t)bh * s.T + t0, ch = it.group, tot = (size_t)s.BH * s.NC * CT;
+  const size_t urow = DELTA ? ch * CT : row0;
   const float *Sp = Sc + ch * s.Dk * s.Dv, *Gp = G + ch * s.Dk * s.Dv;
   const float *Ac = A + ch * CT * CT, *dAc = dA + ch * CT * CT;
   f32x4 acc[2][2], tri[2][2];
@@ -996,7 +1000,7 @@ __global__ __launch_bounds__(256, DELTA ? 3 : 4) void exact_grads(
         [&](int m, int cc) { return doc[(size_t)m * s.Dv + cc]; });
     add(acc, tri);
     if constexpr (DELTA)
-      row_dots(acc, R + row0 * s.Dv + n0, s.Dv, n, nc, pb + (size_t)(2 * tile + (x.w & 1)) * tot + ch * CT, x);
+      row_dots(acc, R + urow * s.Dv + n0, s.Dv, n, nc, pb + (size_t)(2 * tile + (x.w & 1)) * tot + ch * CT, x);
     else
       store_tile(acc, dv + row0 * s.Dv + n0, s.Dv, n, nc, x);
     return;
@@ -1019,7 +1023,7 @@ __global__ __launch_bounds__(256, DELTA ? 3 : 4) void exact_grads(
     store_tile(acc, dq + row0 * s.Dk + n0, s.Dk, n, nc, x);
     return;
   }
-  product<kRows, kRows, VEC, VEC>(acc, Src{u + row0 * s.Dv, s.Dv, n, s.Dv},
+  product<kRows, kRows, VEC, VEC>(acc, Src{u + urow * s.Dv, s.Dv, n, s.Dv},
                                   Src{Gp + (size_t)n0 * s.Dv, s.Dv, nc, s.Dv}, s.Dv, lds, buf, x);
   scale_rows(acc, wt + ch * CT, x);
   row_dots(acc, kt, s.Dk, n, nc, pk + slot, x);
@@ -1100,6 +1104,7 @@ Shape shape_of(int64_t B, int64_t H, int64_t T, int64_t Dk, int64_t Dv) {
   s.DkP = (int)((Dk + 15) / 16 * 16);
   s.nkt = (int)((Dk + 63) / 64);
   s.nvt = (int)((Dv + 63) / 64);
+  s.c0 = 0;
   return s;
 }
 
@@ -1190,7 +1195,8 @@ int chunk_fwd(const float* q, const float* k, const float* v, const float* la, c
                        S0, Sc, Sfin, nullptr, nullptr, nvb, s.nkt, s);
     PGN_LAUNCHED();
   }
-  hipLaunchKernelGGL((exact_out<VEC>), dim3(items(chunks, s.nvt)), dim3(256), 0, st, q, DELTA ? U : v, A, eL, Sc, o, s);
+  hipLaunchKernelGGL((exact_out<VEC>), dim3(items(chunks, s.nvt)), dim3(256), 0, st, q, DELTA ? U : v, A, eL, Sc, o,
+                     DELTA, s);
   PGN_LAUNCHED();
   return PRAGNOSIA_OK;
 }
@@ -1242,13 +1248,16 @@ extern "C" int pragnosia_aspin_exact_chunk_fwd(const float* q, const float* k, c
                                                const float* beta, const float* S0, float* o, float* S_final,
                                                float* states, float* scores, float* gates, float* M, float* X,
                                                float* R, float* U, float* W, int64_t B, int64_t H, int64_t T,
-                                               int64_t Dk, int64_t Dv, void* stream) {
+                                               int64_t Dk, int64_t Dv, int64_t first, int64_t chunks, void* stream) {
   const bool delta = beta != nullptr;
   PGN_CHECK_ARG(chunk_shape_ok(B, H, T, Dk, Dv, delta));
+  PGN_CHECK_ARG(first >= 0 && chunks > 0 && first <= (T + CT - 1) / CT - chunks);
   PGN_CHECK_ARG(q && k && v && la && o && S_final && states && scores && gates);
   PGN_CHECK_ARG(aligned16({scores, gates}));
   if (delta) PGN_CHECK_ARG(M && X && R && U && W && aligned16({M, X, W}));
-  const Shape s = shape_of(B, H, T, Dk, Dv);
+  Shape s = shape_of(B, H, T, Dk, Dv);
+  s.c0 = (int)first;
+  s.NC = (int)chunks;
   hipStream_t st = (hipStream_t)stream;
   // 16-byte loads where every row starts on one
   const bool vec = Dk % 4 == 0 && Dv % 4 == 0 && aligned16({q, k, v, states, U});

@@ -1003,13 +1003,50 @@ def _exact_parts(B: int, H: int, T: int, Dv: int, delta: bool) -> list[int]:
     """Sizes (floats) of what the chunked form keeps in `resid`: per chunk the scores and the two decay vectors, then for
     the delta rule M and X, R and U (multiples of 64, so each part of the buffer is 16-byte aligned)."""
     n = B * H * ((T + CHUNK - 1) // CHUNK) * CHUNK
-    rows = (B * H * T * Dv + 63) // 64 * 64
-    return [n * CHUNK, 2 * n] + ([n * CHUNK, n * CHUNK, rows, rows] if delta else [])
+    return [n * CHUNK, 2 * n] + ([n * CHUNK, n * CHUNK, n * Dv, n * Dv] if delta else [])
 
 
 def _exact_views(buf: Tensor, sizes: list[int]) -> list[Optional[Tensor]]:
     parts = list(buf.split(sizes))
     return parts + [None] * (6 - len(parts))
+
+
+# Without a backward to keep them for, the chunked form's states and scores are scratch, and the sequences run in pieces
+# whose scratch stays within this: 2^20 tokens of four heads of 176 take 10 GB whole (plain; 21 delta). ms whole / in
+# pieces of 512 MiB: 2^18 tokens of four heads of 176 9.5 / 7.2 plain, 19.8 / 19.7 delta; 131072 tokens of twelve heads of
+# 64 2.8 / 2.9, 6.3 / 6.4; cutting heads costs more, 64 x 1024 tokens of twelve heads of 64 (1.4 GiB) 1.03 / 1.17 delta,
+# so the bound is above what such calls take.
+EXACT_SCRATCH_BYTES = 2 << 30
+
+
+def _exact_pieces(heads: int, T: int, Dk: int, Dv: int, delta: bool) -> tuple[int, int]:
+    """(heads, chunks) of a piece: sequences are cut first (their heads walk side by side), down to 16 chunks, then
+    the heads are taken in groups."""
+    NC = (T + CHUNK - 1) // CHUNK
+    per = 4 * (Dk * Dv + CHUNK * CHUNK + 2 * CHUNK)
+    if delta:
+        per += 4 * (2 * CHUNK * CHUNK + CHUNK * (2 * Dv + (Dk + 15) // 16 * 16))
+    chunks = min(NC, max(16, EXACT_SCRATCH_BYTES // (heads * per)))
+    return max(1, min(heads, EXACT_SCRATCH_BYTES // (chunks * per))), chunks
+
+
+def _exact_chunk_fwd(q: Tensor, k: Tensor, v: Tensor, la: Tensor, beta: Optional[Tensor], S0: Optional[Tensor], o: Tensor,
+                     S: Tensor, first: int, chunks: int) -> tuple[Tensor, Tensor]:
+    """The chunked exact forward of (at most) `chunks` chunks from the chunk `first` on, into o and S (inputs already
+    cast, all contiguous): (ckpt, resid) of these chunks."""
+    B, H, T, Dk = q.shape
+    Dv, delta = v.shape[-1], beta is not None
+    N = min(chunks, (T + CHUNK - 1) // CHUNK - first)
+    e = lambda *s: torch.empty(*s, device=q.device, dtype=torch.float32)
+    sizes = _exact_parts(B, H, N * CHUNK, Dv, delta)
+    ckpt, resid = e(B, H, N, Dk, Dv), e(sum(sizes))
+    scores, gates, M, X, R, U = _exact_views(resid, sizes)
+    W = e(B * H * N * CHUNK, (Dk + 15) // 16 * 16) if delta else None
+    check(lib().pragnosia_aspin_exact_chunk_fwd(_ptr(q), _ptr(k), _ptr(v), _ptr(la), _ptr(beta), _ptr(S0), _ptr(o),
+                                                _ptr(S), _ptr(ckpt), _ptr(scores), _ptr(gates), _ptr(M), _ptr(X),
+                                                _ptr(R), _ptr(U), _ptr(W), B, H, T, Dk, Dv, first, N, _stream(q)),
+          "pragnosia_aspin_exact_chunk_fwd")
+    return ckpt, resid
 
 
 def _expect_exact(op: str, q: Tensor, k, v, la, beta=None, S0=None) -> None:
@@ -1031,11 +1068,12 @@ def aspin_exact(q: Tensor, k: Tensor, v: Tensor, la: Tensor, beta: Optional[Tens
     """The scan with fp32 operands (fp64 when q is fp64), plain rule, or the delta rule when beta is given.
     q, k (B, H, T, Dk), v (B, H, T, Dv), la and beta (B, H, T), S0 (B, H, Dk, Dv) or None. Returns (o (B, H, T, Dv),
     S_final (B, H, Dk, Dv), ckpt, resid) in the compute dtype; ckpt and resid are what the backward reads, empty unless
-    want_ckpt. fp32 sequences of EXACT_CHUNK_MIN_T tokens or more run in chunked form (`exact_chunked`; any widths, the
-    delta rule's keys up to 384): ckpt is the state entering every 64 tokens, resid one flat buffer of the chunks' scores,
-    decays and (delta) inverses and residuals. The rest runs token by token, Dk <= 384 and Dv <= 128 (wide keys take
-    fewer value columns: exact_value_cap; the library refuses what does not fit its LDS): ckpt is the state entering
-    every 8 tokens, resid the delta rule's residuals."""
+    want_ckpt (else they are scratch, of about EXACT_SCRATCH_BYTES at the most). fp32 sequences of EXACT_CHUNK_MIN_T
+    tokens or more run in chunked form (`exact_chunked`; any widths, the delta rule's keys up to 384): ckpt is the state
+    entering every 64 tokens, resid one flat buffer of the chunks' scores, decays and (delta) inverses and residuals.
+    The rest runs token by token, Dk <= 384 and Dv <= 128 (wide keys take fewer value columns: exact_value_cap; the
+    library refuses what does not fit its LDS): ckpt is the state entering every 8 tokens, resid the delta rule's
+    residuals."""
     _require_gpu(q, k, v, la, beta, S0)
     _expect_exact("aspin_exact", q, k, v, la, beta, S0)
     dt = _exact_dtype(q)
@@ -1047,18 +1085,17 @@ def aspin_exact(q: Tensor, k: Tensor, v: Tensor, la: Tensor, beta: Optional[Tens
     o = torch.empty(B, H, T, Dv, device=dev, dtype=dt)
     S = torch.empty(B, H, Dk, Dv, device=dev, dtype=dt)
     if exact_chunked(dt, T, Dk, Dv, beta is not None):
-        NC = (T + CHUNK - 1) // CHUNK
-        ckpt = torch.empty(B, H, NC, Dk, Dv, device=dev, dtype=dt)
-        sizes = _exact_parts(B, H, T, Dv, beta is not None)
-        resid = torch.empty(sum(sizes), device=dev, dtype=dt)
-        scores, gates, M, X, R, U = _exact_views(resid, sizes)
-        W = (torch.empty(B * H * NC * CHUNK, (Dk + 15) // 16 * 16, device=dev, dtype=dt) if beta is not None
-             else None)
-        check(lib().pragnosia_aspin_exact_chunk_fwd(_ptr(q), _ptr(k), _ptr(v), _ptr(la), _ptr(beta), _ptr(S0), _ptr(o),
-                                                    _ptr(S), _ptr(ckpt), _ptr(scores), _ptr(gates), _ptr(M), _ptr(X),
-                                                    _ptr(R), _ptr(U), _ptr(W), B, H, T, Dk, Dv, _stream(q)),
-              "pragnosia_aspin_exact_chunk_fwd")
-        return (o, S, ckpt, resid) if want_ckpt else (o, S, q.new_empty(0), q.new_empty(0))
+        if want_ckpt:
+            return (o, S, *_exact_chunk_fwd(q, k, v, la, beta, S0, o, S, 0, (T + CHUNK - 1) // CHUNK))
+        heads, chunks = _exact_pieces(B * H, T, Dk, Dv, beta is not None)
+        flat = lambda t: None if t is None else t.view(B * H, 1, *t.shape[2:])
+        whole = [flat(t) for t in (q, k, v, la, beta, S0, o, S)]
+        for h in range(0, B * H, heads):
+            part = [None if t is None else t[h:h + heads] for t in whole]
+            for c in range(0, (T + CHUNK - 1) // CHUNK, chunks):
+                _exact_chunk_fwd(*part, c, chunks)
+                part[5] = part[7]  # the next piece starts from the state that this one left in S
+        return o, S, q.new_empty(0), q.new_empty(0)
     NB = (T + EXACT_CKPT - 1) // EXACT_CKPT
     ckpt = torch.empty(B, H, NB, Dk, Dv, device=dev, dtype=dt) if want_ckpt else q.new_empty(0)
     resid = (torch.empty(B, H, T, Dv, device=dev, dtype=dt) if (want_ckpt and beta is not None)

@@ -109,3 +109,27 @@ def test_chunked_non_finite_values_stay_where_the_recurrence_takes_them(delta, n
                 fine = want.isfinite()
                 assert torch.equal(got.isfinite(), fine), (val, s, n, (got.isfinite() != fine).nonzero()[:4])
                 assert not fine.any() or (got - want)[fine].abs().max() < TOL * want[fine].abs().max(), (val, s, n)
+
+
+@pytest.mark.parametrize("delta", [False, True])
+@pytest.mark.parametrize("B,H,T,Dk,Dv,mib", [(1, 2, 12000, 48, 32, 1), (3, 5, 4400, 32, 64, 4), (20, 9, 130, 64, 64, 1)])
+def test_chunked_without_a_backward_bounds_its_scratch(delta, B, H, T, Dk, Dv, mib, monkeypatch):
+    """Without gradients the states, scores and inverses are scratch of a piece of the sequences (or of a group of heads)
+    at a time: the same outputs bit for bit, and no more memory than the bound (or 16 chunks of a head, a piece's least)
+    beside the outputs. The allocator may hand out up to 1 MiB more than asked for, in five arrays; whole, the scratch is
+    8 MiB and more."""
+    from pragnosia_amd import ops
+    x, _, _ = _inputs(B, H, T, Dk, Dv, delta, seed=19, s0=True)
+    a = [x[n].cuda() if n in x else None for n in ("q", "k", "v", "la", "beta", "S0")]
+    o, S, _, _ = ops.aspin_exact(*a, True)
+    monkeypatch.setattr(ops, "EXACT_SCRATCH_BYTES", mib << 20)
+    heads, chunks = ops._exact_pieces(B * H, T, Dk, Dv, delta)
+    assert heads < B * H or 64 * chunks < T
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    o2, S2, _, _ = ops.aspin_exact(*a, False)
+    peak = torch.cuda.max_memory_allocated() - before
+    assert torch.equal(o, o2) and torch.equal(S, S2)
+    per = 4 * (Dk * Dv + 64 * 66 + (2 * 64 * 64 + 64 * (2 * Dv + (Dk + 15) // 16 * 16) if delta else 0))
+    assert peak <= max(mib << 20, 16 * per) + 4 * (o.numel() + S.numel()) + (5 << 20), peak
