@@ -992,11 +992,15 @@ def _dtype_code(dt: torch.dtype) -> int:
     return 1 if dt == torch.float64 else 0
 
 
-def exact_chunked(dt: torch.dtype, T: int, Dk: int, Dv: int, delta: bool) -> bool:
-    """Whether the exact scan of T tokens runs in chunked form (key and value widths up to 4096, the delta rule's keys up
-    to 384) rather than token by token."""
-    return (dt == torch.float32 and T >= EXACT_CHUNK_MIN_T and 0 < Dk <= (EXACT_MAX_DK if delta else EXACT_CHUNK_MAX_D)
-            and 0 < Dv <= EXACT_CHUNK_MAX_D)
+def exact_chunked(dt: torch.dtype, heads: int, T: int, Dk: int, Dv: int, delta: bool) -> bool:
+    """Whether the exact scan of `heads` sequences of T tokens runs in chunked form (key and value widths up to 4096, the
+    delta rule's keys up to 384) rather than token by token. Its grids count tiles of chunks in 31 bits (chunk_shape_ok
+    of the kernels); what is past that stays token by token too."""
+    if not (dt == torch.float32 and EXACT_CHUNK_MIN_T <= T < 1 << 28 and 0 < heads < 1 << 24
+            and 0 < Dk <= (EXACT_MAX_DK if delta else EXACT_CHUNK_MAX_D) and 0 < Dv <= EXACT_CHUNK_MAX_D):
+        return False
+    nkt, nvt, chunks = (Dk + 63) // 64, (Dv + 63) // 64, heads * ((T + CHUNK - 1) // CHUNK)
+    return (chunks + 8) * (2 * nkt + nvt) < 1 << 31 and (heads + 8) * ((Dv + 15) // 16) * nkt < 1 << 31
 
 
 def _exact_parts(B: int, H: int, T: int, Dv: int, delta: bool) -> list[int]:
@@ -1055,7 +1059,7 @@ def _expect_exact(op: str, q: Tensor, k, v, la, beta=None, S0=None) -> None:
         raise PragnosiaError(f"{op}: q and v must be (B, H, T, D)")
     B, H, T, Dk = q.shape
     Dv = v.shape[-1]
-    if not (exact_chunked(_exact_dtype(q), T, Dk, Dv, beta is not None)
+    if not (exact_chunked(_exact_dtype(q), B * H, T, Dk, Dv, beta is not None)
             or (0 < Dk <= EXACT_MAX_DK and 0 < Dv <= EXACT_MAX_DV)):
         raise PragnosiaError(f"{op}: head dims Dk={Dk}, Dv={Dv} must be in 1..{EXACT_MAX_DK} x 1..{EXACT_MAX_DV}")
     _expect(op, q.device, k=(k, (B, H, T, Dk)), v=(v, (B, H, T, Dv)), la=(la, (B, H, T)), beta=(beta, (B, H, T)),
@@ -1084,7 +1088,7 @@ def aspin_exact(q: Tensor, k: Tensor, v: Tensor, la: Tensor, beta: Optional[Tens
     dev = q.device
     o = torch.empty(B, H, T, Dv, device=dev, dtype=dt)
     S = torch.empty(B, H, Dk, Dv, device=dev, dtype=dt)
-    if exact_chunked(dt, T, Dk, Dv, beta is not None):
+    if exact_chunked(dt, B * H, T, Dk, Dv, beta is not None):
         if want_ckpt:
             return (o, S, *_exact_chunk_fwd(q, k, v, la, beta, S0, o, S, 0, (T + CHUNK - 1) // CHUNK))
         heads, chunks = _exact_pieces(B * H, T, Dk, Dv, beta is not None)
@@ -1112,7 +1116,7 @@ def _(q, k, v, la, beta, S0, want_ckpt):
     B, H, T, Dk = q.shape
     Dv = v.shape[-1]
     dt = _exact_dtype(q)
-    if want_ckpt and exact_chunked(dt, T, Dk, Dv, beta is not None):
+    if want_ckpt and exact_chunked(dt, B * H, T, Dk, Dv, beta is not None):
         return (q.new_empty(B, H, T, Dv, dtype=dt), q.new_empty(B, H, Dk, Dv, dtype=dt),
                 q.new_empty(B, H, (T + CHUNK - 1) // CHUNK, Dk, Dv, dtype=dt),
                 q.new_empty(sum(_exact_parts(B, H, T, Dv, beta is not None)), dtype=dt))
@@ -1134,7 +1138,7 @@ def aspin_exact_bwd(q: Tensor, k: Tensor, v: Tensor, la: Tensor, beta: Optional[
     Dv = v.shape[-1]
     dt = _exact_dtype(q)
     delta = beta is not None
-    chunked = exact_chunked(dt, T, Dk, Dv, delta)
+    chunked = exact_chunked(dt, B * H, T, Dk, Dv, delta)
     NB = (T + CHUNK - 1) // CHUNK if chunked else (T + EXACT_CKPT - 1) // EXACT_CKPT
     sizes = _exact_parts(B, H, T, Dv, delta) if chunked else []
     _expect("aspin_exact_bwd", q.device, ckpt=(ckpt, (B, H, NB, Dk, Dv)), do=(do, (B, H, T, Dv)),

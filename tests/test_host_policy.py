@@ -34,3 +34,20 @@ def test_backward_splits_sooner():
     assert seg_chunks(96, 16, range(1, 17), "fwd") == 16
     assert seg_chunks(128, 8, range(1, 9), "bwd") == 8
     assert seg_chunks(192, 8, range(1, 9), "bwd") == 8
+
+
+def test_exact_chunked_is_what_the_library_takes():
+    """The exact scan runs in chunked form only where the library's chunked entry points take the sizes; the rest stays
+    with the token-by-token form, which takes more sequences."""
+    import torch
+
+    from pragnosia_amd._lib import lib
+    from pragnosia_amd.ops import exact_chunked
+    cases = [(1, 32, 1, 1), (4, 2048, 176, 176), (1, 1 << 20, 352, 352), ((1 << 24) - 1, 32, 1, 1), (1 << 24, 32, 1, 1),
+             (1, (1 << 28) - 1, 16, 16), (1, 1 << 28, 16, 16), (1 << 20, 65536, 64, 64), (1 << 20, 16384, 4, 4),
+             ((1 << 24) - 1, 64, 8, 4096), (2, 100, 400, 16), (2, 100, 4097, 16), (2, 100, 16, 4097)]
+    for delta in (False, True):
+        for heads, T, Dk, Dv in cases:
+            takes = lib().pragnosia_aspin_exact_chunk_bwd_workspace_bytes(heads, 1, T, Dk, Dv, int(delta)) >= 0
+            assert exact_chunked(torch.float32, heads, T, Dk, Dv, delta) == takes, (heads, T, Dk, Dv, delta)
+    assert not exact_chunked(torch.float32, 4, 31, 64, 64, False) and not exact_chunked(torch.float64, 4, 64, 64, 64, False)
