@@ -460,7 +460,7 @@ __global__ __launch_bounds__(256) void exact_wy_fwd(const float* __restrict__ k,
         [&](int m, int cc) { return (val ? 1.f : el[m]) * vk[(size_t)m * D + cc]; });
   }
   if (val)
-    store_tile(acc, R + ch * CT * D + n0, D, n, D - n0, x);
+    store_tile(acc, R + ch * CT * D + n0, D, CT, D - n0, x);  // a short last chunk's rows end in zeros
   else
     store_tile(acc, W + ch * CT * s.DkP + n0, s.DkP, CT, s.DkP - n0, x);
 }
@@ -655,7 +655,7 @@ __global__ __launch_bounds__(256, KT == 1 || (KT <= 3 && !BWD) ? 2 : 1) void exa
   auto load_y = [&](int c) {
     const int t0 = s.token(c), n = min(CT, s.T - t0);
     const size_t row0 = (size_t)bh * s.T + t0, yrow = BWD ? row0 : ((size_t)bh * s.NC + c) * CT;
-    const __amdgpu_buffer_rsrc_t r = view(y + yrow * s.Dv, n * s.Dv), br = view(BWD ? wt : beta + row0, BWD ? 0 : n);
+    const __amdgpu_buffer_rsrc_t r = view(y + yrow * s.Dv, (BWD ? n : CT) * s.Dv), br = view(BWD ? wt : beta + row0, BWD ? 0 : n);
     const unsigned o = fresh(ybase);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -721,7 +721,7 @@ __global__ __launch_bounds__(256, KT == 1 || (KT <= 3 && !BWD) ? 2 : 1) void exa
     {
       const f32x4 sum = (part[0][x.w][x.l] + part[1][x.w][x.l]) + (part[2][x.w][x.l] + part[3][x.w][x.l]);
       const f32x4 v = BWD ? yo + sum : yo - sum;
-      const __amdgpu_buffer_rsrc_t yr = view(y + (BWD ? row0 : ch * CT) * s.Dv, n * s.Dv);
+      const __amdgpu_buffer_rsrc_t yr = view(y + (BWD ? row0 : ch * CT) * s.Dv, (BWD ? n : CT) * s.Dv);
       const unsigned o = fresh(ybase);
 #pragma unroll
       for (int e = 0; e < 4; ++e) bstore(yr, o + e * vd4, v[e]);
@@ -729,7 +729,7 @@ __global__ __launch_bounds__(256, KT == 1 || (KT <= 3 && !BWD) ? 2 : 1) void exa
         us[x.w][x.l] = v;
       } else {
         const f32x4 u = v * bo;
-        const __amdgpu_buffer_rsrc_t ur = view(U + ch * CT * s.Dv, n * s.Dv);
+        const __amdgpu_buffer_rsrc_t ur = view(U + ch * CT * s.Dv, CT * s.Dv);
 #pragma unroll
         for (int e = 0; e < 4; ++e) bstore(ur, o + e * vd4, u[e]);
         us[x.w][x.l] = u;
