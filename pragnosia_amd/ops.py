@@ -852,13 +852,13 @@ def _delta_pass(q: Tensor, k: Tensor, v: Tensor, la: Tensor, beta: Tensor, S0: O
                                             Optional[Tensor]]:
     """One 64-wide delta forward through the C ABI writing only what is asked for: o when want_o; the entering
     states, W and X when want_saved (the state pass of a recomputing backward, want_o False, skips the output
-    products). Returns (o, S_final, sent, W, X), None for what was not written. Inputs already cast."""
+    products). Returns (o, S_final, sent, W, X), None for what was not written. Inputs already cast. The chunk-parallel
+    form writes the states, W and X in any case, so it is taken only where they are wanted."""
     B, H, T, D = q.shape
     NC = (T + CHUNK - 1) // CHUNK
     dev = q.device
-    if delta_parallel(B * H, NC, D, False):
-        o, S, sent, W, X = _delta_par_fwd(q, k, v, la, beta, S0, want_o)
-        return (o, S, sent, W, X) if want_saved else (o, S, None, None, None)
+    if want_saved and delta_parallel(B * H, NC, D, False):
+        return _delta_par_fwd(q, k, v, la, beta, S0, want_o)
     o = torch.empty(B, H, T, D, device=dev, dtype=torch.bfloat16) if want_o else None
     S = torch.empty(B, H, D, D, device=dev, dtype=torch.float32)
     sent = W = X = None

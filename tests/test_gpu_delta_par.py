@@ -66,3 +66,20 @@ def test_windows_match_the_window_loop(B, H, T, window, s0, monkeypatch):
     ref = torch.cat(outs, 2).float()
     assert (o.float() - ref).abs().max() <= 2.0 ** -7 * ref.abs().max()
     assert (S - st).abs().max() <= 2.0 ** -8 * st.abs().max()
+
+
+def test_fused_forward_keeps_states_on_chip():
+    """The scan that keeps nothing for its backward takes no memory beside o and S either, at a size whose plain forward
+    runs chunk-parallel and writes 22 MiB of states, W and X (the allocator may hand out up to 1 MiB more than asked for,
+    in two arrays), and gives the plain forward's outputs."""
+    from pragnosia_amd import ops
+    x, _, _ = _inputs(2, 12, 2560, 64, True, seed=3)
+    assert ops.delta_parallel(24, 40, 64, False)
+    o, S, _, _, _ = ops.aspin_delta(*x, True)
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    of, Sf = ops.aspin_delta_fused(*x)
+    peak = torch.cuda.max_memory_allocated() - before
+    assert torch.equal(o, of) and torch.equal(S, Sf)
+    assert peak <= 2 * o.numel() + 4 * S.numel() + (2 << 20), peak
