@@ -894,6 +894,54 @@ def aspin_delta_fused(q: Tensor, k: Tensor, v: Tensor, la: Tensor, beta: Tensor,
     return o, S
 
 
+def delta_window_maps(heads: int, T: int, window: int) -> bool:
+    """Whether the carried windows of `heads` sequences of T tokens run as the windows' affine maps (every window at once,
+    twice, and a chain of one step a window) instead of one chunk-parallel walk over all chunks. The walk does less in
+    all but takes every chunk of a sequence in turn, so a long sequence of few heads is faster as maps. From the cost of
+    each, in us: a round of window workgroups over the compute units takes 3.5 and 2.9 a chunk, the chain 0.9 a window,
+    padding a partial last window five copies; the walk 0.72 a chunk and round of its four workgroups a head, the rest
+    0.0155 a chunk and head. Measured, maps / walk: 12 heads, 32768 tokens in windows of 1024 272 / 431, of 256 388 /
+    442, of 64 977 / 478; 12 heads of 8192 in 512 100 / 121; 4 heads of 131072 in 2048 335 / 1502; 24 heads of 32768 in
+    1024 493 / 541; 24 heads of 8192 in 512 156 / 136; 96 heads of 16384 in 2048 929 / 745; with a partial last window,
+    12 heads of 30000 in 1024 383 / 399, of 20000 in 512 286 / 273. Over 4 to 384 heads, 1024 to 131072 tokens and
+    windows of 64 to 2048 (246 sizes) the choice is the faster one or within 5% of it."""
+    up = lambda a, b: -(-a // b)
+    NW, NC = up(T, window), up(T, CHUNK)
+    rounds = up(2 * heads * NW, COMPUTE_UNITS) + up(heads * NW, COMPUTE_UNITS)
+    maps = 8 + rounds * (3.5 + 2.9 * window / CHUNK) + 0.9 * NW + (25 + 2.5e-4 * heads * T if T % window else 0)
+    walk = 12 + NC * (0.72 * up(4 * heads, COMPUTE_UNITS) + 0.0155 * heads)
+    return maps < 0.95 * walk
+
+
+def _delta_windows_maps(q: Tensor, k: Tensor, v: Tensor, la: Tensor, beta: Tensor, S0: Optional[Tensor], theta: Tensor,
+                        window: int) -> tuple[Tensor, Tensor]:
+    """The windows as affine maps (inputs already cast): given the chunk inverses the rule is linear in the state and
+    independent per value column, so a window takes its entering state to S_out = M S_in + R. The state passes over all
+    windows (R from zero entering states; M from identity states with zero values) in one launch
+    (`pragnosia_aspin_delta_window_maps`), the entering states chained by `pragnosia_aspin_delta_window_prefix`, then one
+    pass with outputs from them. A partial last window is zero-padded (zero keys, values, decay and strength leave the
+    state unchanged)."""
+    B, H, T, D = q.shape
+    NW = (T + window - 1) // window
+    Tp = NW * window
+    if Tp != T:
+        pad = lambda t: F.pad(t, (0, 0, 0, Tp - T)) if t.dim() == 4 else F.pad(t, (0, Tp - T))
+        q, k, v, la, beta = (pad(t) for t in (q, k, v, la, beta))
+    BW = B * H * NW  # every window of every (batch, head) a sequence of its own: contiguous views
+    qw, kw, vw = (t.view(BW, 1, window, D) for t in (q, k, v))
+    lw, bw = la.view(BW, 1, window), beta.view(BW, 1, window)
+    RM = torch.empty(2, BW, D, D, device=q.device, dtype=torch.float32)  # R, then M: both state passes, one launch
+    check(lib().pragnosia_aspin_delta_window_maps(_ptr(qw), _ptr(kw), _ptr(vw), _ptr(lw), _ptr(bw), _ptr(RM), BW, window,
+                                                  _stream(q)), "pragnosia_aspin_delta_window_maps")
+    Sin = torch.empty(BW, 1, D, D, device=q.device, dtype=torch.float32)
+    check(lib().pragnosia_aspin_delta_window_prefix(_ptr(RM[1]), _ptr(RM[0]), _ptr(S0), _ptr(theta), float(window),
+                                                    _ptr(Sin), B * H, H, NW, _stream(q)),
+          "pragnosia_aspin_delta_window_prefix")
+    o, S, _, _, _ = _delta_pass(qw, kw, vw, lw, bw, Sin, True, False)
+    o = o.view(B, H, Tp, D)[:, :, :T]
+    return (o if Tp == T else o.contiguous()), S.view(B, H, NW, D, D)[:, :, -1].contiguous()
+
+
 @torch.library.custom_op("pragnosia::aspin_delta_windows", mutates_args=())
 def aspin_delta_windows(q: Tensor, k: Tensor, v: Tensor, la: Tensor, beta: Tensor, S0: Optional[Tensor],
                         theta: Tensor, window: int) -> tuple[Tensor, Tensor]:
@@ -901,15 +949,18 @@ def aspin_delta_windows(q: Tensor, k: Tensor, v: Tensor, la: Tensor, beta: Tenso
     were rotated with positions restarting at 0 in every window, the state carried across window boundaries and
     rebased by -window * theta there: what aspin_delta over each window in turn, with aspin_rebase between, computes
     (the reference's carried windows, `src/model.py:842-864` over `src/assoc.py:391-405`), in one pass that rebases the
-    state as it walks past each window (`pragnosia_aspin_delta_par_fwd`). Head dim 64. S0 enters the first window. Returns
-    (o bf16, S after the last window fp32, in its positions)."""
+    state as it walks past each window (`pragnosia_aspin_delta_par_fwd`), or, a long sequence of few heads, from the
+    windows' affine maps (`delta_window_maps`). Head dim 64. S0 enters the first window. Returns (o bf16, S after the
+    last window fp32, in its positions)."""
     _require_gpu(q, k, v, la, beta, S0, theta)
     _expect_scan("aspin_delta_windows", q, k, v, la, beta=beta, S0=S0, theta=theta)
     if window <= 0 or window % CHUNK:
         raise PragnosiaError(f"aspin_delta_windows: window {window} must be a positive multiple of {CHUNK}")
     if q.shape[-1] != 64:
-        raise PragnosiaError(f"aspin_delta_windows: head dim {q.shape[-1]}; the window maps are built for 64")
+        raise PragnosiaError(f"aspin_delta_windows: head dim {q.shape[-1]}; the windowed scan is built for 64")
     q, k, v, la, beta, S0, theta = _bf16(q), _bf16(k), _bf16(v), _f32(la), _f32(beta), _f32(S0), _f32(theta)
+    if delta_window_maps(q.shape[0] * q.shape[1], q.shape[2], window):
+        return _delta_windows_maps(q, k, v, la, beta, S0, theta, window)
     o, S, _, _, _ = _delta_par_fwd(q, k, v, la, beta, S0, True, theta, window)
     return o, S
 

@@ -49,11 +49,15 @@ def test_matches_one_workgroup_per_scan(B, H, T, D, s0, monkeypatch):
             assert (p.float() - q.float()).abs().max() <= 2.0 ** -8 * p.float().abs().max(), n
 
 
-@pytest.mark.parametrize("B,H,T,window,s0", [(1, 2, 200, 64, True), (2, 5, 448, 128, False), (1, 1, 1000, 192, True)])
-def test_windows_match_the_window_loop(B, H, T, window, s0, monkeypatch):
-    """Carried windows in one walk against one call a window with the state rebased between (ragged last window and
-    chunk): the state is rotated in fp32 either way, by the rebase kernel there, in the walk here."""
+@pytest.mark.parametrize("maps", [False, True])
+@pytest.mark.parametrize("B,H,T,window,s0", [(1, 2, 200, 64, True), (2, 5, 448, 128, False), (1, 1, 1000, 192, True),
+                                             (1, 3, 768, 256, True)])
+def test_windows_match_the_window_loop(B, H, T, window, s0, maps, monkeypatch):
+    """Carried windows, in one walk and as the windows' affine maps, against one call a window with the state rebased
+    between (ragged last window and chunk): the state is rotated in fp32 every way, by the rebase kernel there, in the
+    walk or the maps' chain here; the maps come from the same bf16 operands as the window's own pass."""
     from pragnosia_amd import ops
+    monkeypatch.setattr(ops, "delta_window_maps", lambda *a: maps)
     x, _, _ = _inputs(B, H, T, 64, s0, seed=T)
     theta = (torch.rand(H, 32, generator=torch.Generator().manual_seed(1)) * 0.1).cuda()
     o, S = ops.aspin_delta_windows(*x, theta, window)

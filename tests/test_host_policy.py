@@ -51,3 +51,13 @@ def test_exact_chunked_is_what_the_library_takes():
             takes = lib().pragnosia_aspin_exact_chunk_bwd_workspace_bytes(heads, 1, T, Dk, Dv, int(delta)) >= 0
             assert exact_chunked(torch.float32, heads, T, Dk, Dv, delta) == takes, (heads, T, Dk, Dv, delta)
     assert not exact_chunked(torch.float32, 4, 31, 64, 64, False) and not exact_chunked(torch.float64, 4, 64, 64, 64, False)
+
+
+def test_carried_windows_take_the_faster_form():
+    """The delta rule's carried windows: maps for long sequences of few heads, one walk for the rest."""
+    from pragnosia_amd.ops import delta_window_maps
+    for heads, T, window in ((4, 131072, 2048), (12, 32768, 1024), (12, 8192, 512), (24, 32768, 1024), (4, 4096, 256)):
+        assert delta_window_maps(heads, T, window), (heads, T, window)
+    for heads, T, window in ((24, 8192, 512), (12, 32768, 64), (12, 2048, 512), (96, 16384, 2048), (48, 32768, 2048),
+                             (4, 1024, 4096), (1, 64, 64)):
+        assert not delta_window_maps(heads, T, window), (heads, T, window)
