@@ -41,11 +41,9 @@ FUSED_PROJ = False
 FUSED_PLUMBING = True
 
 HEAD_DIM_KERNEL = 64
-# The fused projection's rows (3 d + 2 h: 2134 for d 704) padded with zero rows to a multiple of this, so its output's
-# and its gradient's rows are 128-byte aligned: off alignment the GEMMs around them slow down, and the weight gradient
-# leaves its kernel (widths a multiple of 8). us at 8192 tokens, unpadded / padded, forward, input and weight gradient:
-# d 704 (2134 / 2176) 47 / 44, 49 / 39, 74 / 49; d 384 (1164 / 1216) 22 / 22, 22 / 18, 52 / 26; d 768 (2328 / 2368) 45 /
-# 45, 42 / 36, 55 / 55.
+# The fused projection's rows (3 d + 2 h: 2134 for d 704) may be padded with zero rows to a multiple of this, so its
+# output's and its gradient's rows are 128-byte aligned: off alignment the GEMMs of a training step slow down, and the
+# weight gradient leaves its kernel (widths a multiple of 8). `_proj_padding` says from how many tokens on.
 PROJ_ALIGN = 64
 _POS_CACHE: dict = {}
 
@@ -96,6 +94,24 @@ def _positions(T, device, wrap=None):
             pos = pos % wrap
         _POS_CACHE[key] = pos
     return pos
+
+
+def _proj_padding(width: int, tokens: int, low: bool) -> int:
+    """Zero rows appended to a training step's projection weight of `width` rows. What padding saves grows with the
+    tokens and with how far off alignment the rows are; the wider product, the zero block and its copy cost the same at
+    any. us a layer's training step under bf16 autocast (`low`), unpadded / padded: rows of 4 bytes' alignment (d 704:
+    2134) 512 tokens 206 / 202, 2048 260 / 254, 8192 479 / 444; of 8 (d 384: 1164, d 640: 1940) 512 tokens 173 / 182 and
+    195 / 196, 1536 203 / 198 and 227 / 227, 8192 311 / 281 and 428 / 396; of 16 (d 768: 2328) 1024 tokens 228 / 228, 4096
+    317 / 314, 32768 1354 / 1313. In fp32 the rows of d 704 alone are off 16 bytes: 2048 tokens 437 / 441, 4096 688 / 665,
+    8192 1272 / 1162; the others gain nothing. Without a backward only the wider product is left: d 704 in bf16, 2048
+    tokens 86 / 89, 16384 236 / 238."""
+    if low:
+        least = 4096 if width % 8 == 0 else 1536 if width % 4 == 0 else 512
+    elif width % 4 == 0:
+        return 0
+    else:
+        least = 4096
+    return -width % PROJ_ALIGN if tokens >= least else 0
 
 
 def _needs_grad(*ts):
@@ -358,9 +374,12 @@ class AssocCarrier(nn.Module):
                 and getattr(self, "beta_scale", None) is None and getattr(self, "sconv", None) is None):
             gated = not (self.delta or self.write_all)
             extra = [self.wi.weight] if gated else ([self.wb.weight] if self.delta else [])
-            if extra and (pad := -(3 * self.d + 2 * self.h) % PROJ_ALIGN):
-                extra.append(self.wa.weight.new_zeros(pad, self.d))
-            W = torch.cat([self.q.weight, self.k.weight, self.v.weight, self.wa.weight] + extra)
+            parts = [self.q.weight, self.k.weight, self.v.weight, self.wa.weight] + extra
+            low = z.dtype in (torch.bfloat16, torch.float16) or torch.is_autocast_enabled("cuda")
+            if extra and _needs_grad(z, *parts) and (pad := _proj_padding(3 * self.d + 2 * self.h,
+                                                                          z.shape[0] * z.shape[1], low)):
+                parts.append(self.wa.weight.new_zeros(pad, self.d))
+            W = torch.cat(parts)
             P = _op_mod.linear_w(z, W)
             q, k, v, la, beta = _op.aspin_prep_proj(
                 P, self.h, self.wa.bias, self.A, self.la_floor if self.hl_floor else None,

@@ -43,3 +43,29 @@ def test_layer_step_records_no_memset(d, head_dim, delta):
         torch.cuda.synchronize()
         want = step()[gate]
         assert want.abs() > 0 and (got - want).abs() <= 1e-4 * want.abs() + 1e-3, (got.item(), want.item())
+
+
+@pytest.mark.parametrize("d,head_dim,delta,B,T", [(128, 64, False, 1, 1536), (128, 64, True, 3, 517), (704, 64, False, 2, 300),
+                                                  (256, 128, True, 2, 2100)])
+def test_padded_projection_equals_unpadded(d, head_dim, delta, B, T, monkeypatch):
+    """A training step whose projection is padded for aligned rows gives the unpadded one's output, state and gradients:
+    the padded columns are read by nothing and their gradient is zero. The weight gradients differ by the unpadded
+    form's rounding to bf16 (2^-9 of each value), everything else by the order of sums in other GEMM tiles, at bf16."""
+    from pragnosia_amd import assoc
+    torch.manual_seed(d + T)
+    with torch.device("cuda"):
+        m = assoc.AssocCarrier(d, head_dim=head_dim, delta=delta)
+        x, t = torch.randn(B, T, d, requires_grad=True), torch.randn(B, T, d)
+    assert assoc._proj_padding(3 * d + 2 * m.h, B * T, True) > 0
+
+    def step():
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            y, (S, _) = m(x)
+        return y.detach(), S.detach(), *torch.autograd.grad(y, [x, *m.parameters()], t, allow_unused=True)
+
+    padded = step()
+    monkeypatch.setattr(assoc, "PROJ_ALIGN", 1)
+    for n, a, b in zip(["y", "S", "x", *dict(m.named_parameters())], padded, step()):
+        assert (a is None) == (b is None), n
+        if a is not None:
+            assert (a - b).norm() <= 2.0 ** -8 * b.norm(), (n, ((a - b).norm() / b.norm()).item())

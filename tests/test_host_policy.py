@@ -61,3 +61,15 @@ def test_carried_windows_take_the_faster_form():
     for heads, T, window in ((24, 8192, 512), (12, 32768, 64), (12, 2048, 512), (96, 16384, 2048), (48, 32768, 2048),
                              (4, 1024, 4096), (1, 64, 64)):
         assert not delta_window_maps(heads, T, window), (heads, T, window)
+
+
+def test_projection_padding_by_alignment_and_tokens():
+    """Zero rows for a training step's projection: to a multiple of 64, from fewer tokens the further off alignment its
+    rows are, never in fp32 where they are 16-byte aligned."""
+    from pragnosia_amd.assoc import _proj_padding
+    for width, least in ((2134, 512), (1164, 1536), (1940, 1536), (2328, 4096), (776, 4096)):
+        assert _proj_padding(width, least - 1, True) == 0
+        assert _proj_padding(width, least, True) == -width % 64 and (width + _proj_padding(width, least, True)) % 64 == 0
+    assert _proj_padding(2304, 1 << 20, True) == 0
+    assert _proj_padding(2134, 4096, False) == 42 and _proj_padding(2134, 4095, False) == 0
+    assert _proj_padding(1164, 1 << 20, False) == 0
