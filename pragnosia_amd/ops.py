@@ -1050,6 +1050,8 @@ def exact_chunked(dt: torch.dtype, heads: int, T: int, Dk: int, Dv: int, delta: 
     if not (dt == torch.float32 and EXACT_CHUNK_MIN_T <= T < 1 << 28 and 0 < heads < 1 << 24
             and 0 < Dk <= (EXACT_MAX_DK if delta else EXACT_CHUNK_MAX_D) and 0 < Dv <= EXACT_CHUNK_MAX_D):
         return False
+    if heads * (T + CHUNK) * (Dk + Dv + 128) < 1 << 34:  # far within both
+        return True
     nkt, nvt, chunks = (Dk + 63) // 64, (Dv + 63) // 64, heads * ((T + CHUNK - 1) // CHUNK)
     return (chunks + 8) * (2 * nkt + nvt) < 1 << 31 and (heads + 8) * ((Dv + 15) // 16) * nkt < 1 << 31
 
@@ -1061,9 +1063,13 @@ def _exact_parts(B: int, H: int, T: int, Dv: int, delta: bool) -> list[int]:
     return [n * CHUNK, 2 * n] + ([n * CHUNK, n * CHUNK, n * Dv, n * Dv] if delta else [])
 
 
-def _exact_views(buf: Tensor, sizes: list[int]) -> list[Optional[Tensor]]:
-    parts = list(buf.split(sizes))
-    return parts + [None] * (6 - len(parts))
+def _exact_ptrs(buf: Tensor, sizes: list[int]) -> list[Optional[ctypes.c_void_p]]:
+    """The addresses of `resid`'s parts (`_exact_parts`); None for those that the plain rule has not."""
+    at, out = buf.data_ptr(), []
+    for n in sizes:
+        out.append(ctypes.c_void_p(at))
+        at += 4 * n
+    return out + [None] * (6 - len(out))
 
 
 # Without a backward to keep them for, the chunked form's states and scores are scratch, and the sequences run in pieces
@@ -1081,6 +1087,8 @@ def _exact_pieces(heads: int, T: int, Dk: int, Dv: int, delta: bool) -> tuple[in
     per = 4 * (Dk * Dv + CHUNK * CHUNK + 2 * CHUNK)
     if delta:
         per += 4 * (2 * CHUNK * CHUNK + CHUNK * (2 * Dv + (Dk + 15) // 16 * 16))
+    if heads * NC * per <= EXACT_SCRATCH_BYTES:
+        return heads, NC
     chunks = min(NC, max(16, EXACT_SCRATCH_BYTES // (heads * per)))
     return max(1, min(heads, EXACT_SCRATCH_BYTES // (chunks * per))), chunks
 
@@ -1095,11 +1103,10 @@ def _exact_chunk_fwd(q: Tensor, k: Tensor, v: Tensor, la: Tensor, beta: Optional
     e = lambda *s: torch.empty(*s, device=q.device, dtype=torch.float32)
     sizes = _exact_parts(B, H, N * CHUNK, Dv, delta)
     ckpt, resid = e(B, H, N, Dk, Dv), e(sum(sizes))
-    scores, gates, M, X, R, U = _exact_views(resid, sizes)
     W = e(B * H * N * CHUNK, (Dk + 15) // 16 * 16) if delta else None
     check(lib().pragnosia_aspin_exact_chunk_fwd(_ptr(q), _ptr(k), _ptr(v), _ptr(la), _ptr(beta), _ptr(S0), _ptr(o),
-                                                _ptr(S), _ptr(ckpt), _ptr(scores), _ptr(gates), _ptr(M), _ptr(X),
-                                                _ptr(R), _ptr(U), _ptr(W), B, H, T, Dk, Dv, first, N, _stream(q)),
+                                                _ptr(S), _ptr(ckpt), *_exact_ptrs(resid, sizes), _ptr(W), B, H, T,
+                                                Dk, Dv, first, N, _stream(q)),
           "pragnosia_aspin_exact_chunk_fwd")
     return ckpt, resid
 
@@ -1110,8 +1117,8 @@ def _expect_exact(op: str, q: Tensor, k, v, la, beta=None, S0=None) -> None:
         raise PragnosiaError(f"{op}: q and v must be (B, H, T, D)")
     B, H, T, Dk = q.shape
     Dv = v.shape[-1]
-    if not (exact_chunked(_exact_dtype(q), B * H, T, Dk, Dv, beta is not None)
-            or (0 < Dk <= EXACT_MAX_DK and 0 < Dv <= EXACT_MAX_DV)):
+    if not ((0 < Dk <= EXACT_MAX_DK and 0 < Dv <= EXACT_MAX_DV)
+            or exact_chunked(_exact_dtype(q), B * H, T, Dk, Dv, beta is not None)):
         raise PragnosiaError(f"{op}: head dims Dk={Dk}, Dv={Dv} must be in 1..{EXACT_MAX_DK} x 1..{EXACT_MAX_DV}")
     _expect(op, q.device, k=(k, (B, H, T, Dk)), v=(v, (B, H, T, Dv)), la=(la, (B, H, T)), beta=(beta, (B, H, T)),
             S0=(S0, (B, H, Dk, Dv)))
@@ -1140,14 +1147,16 @@ def aspin_exact(q: Tensor, k: Tensor, v: Tensor, la: Tensor, beta: Optional[Tens
     o = torch.empty(B, H, T, Dv, device=dev, dtype=dt)
     S = torch.empty(B, H, Dk, Dv, device=dev, dtype=dt)
     if exact_chunked(dt, B * H, T, Dk, Dv, beta is not None):
-        if want_ckpt:
-            return (o, S, *_exact_chunk_fwd(q, k, v, la, beta, S0, o, S, 0, (T + CHUNK - 1) // CHUNK))
-        heads, chunks = _exact_pieces(B * H, T, Dk, Dv, beta is not None)
+        NC = (T + CHUNK - 1) // CHUNK
+        heads, chunks = (B * H, NC) if want_ckpt else _exact_pieces(B * H, T, Dk, Dv, beta is not None)
+        if heads == B * H and chunks == NC:
+            kept = _exact_chunk_fwd(q, k, v, la, beta, S0, o, S, 0, NC)
+            return (o, S, *kept) if want_ckpt else (o, S, q.new_empty(0), q.new_empty(0))
         flat = lambda t: None if t is None else t.view(B * H, 1, *t.shape[2:])
         whole = [flat(t) for t in (q, k, v, la, beta, S0, o, S)]
         for h in range(0, B * H, heads):
             part = [None if t is None else t[h:h + heads] for t in whole]
-            for c in range(0, (T + CHUNK - 1) // CHUNK, chunks):
+            for c in range(0, NC, chunks):
                 _exact_chunk_fwd(*part, c, chunks)
                 part[5] = part[7]  # the next piece starts from the state that this one left in S
         return o, S, q.new_empty(0), q.new_empty(0)
@@ -1211,11 +1220,10 @@ def aspin_exact_bwd(q: Tensor, k: Tensor, v: Tensor, la: Tensor, beta: Optional[
         if nbytes < 0:
             raise PragnosiaError(f"aspin_exact_bwd: shape rejected (B={B} H={H} T={T} Dk={Dk} Dv={Dv})")
         ws = torch.empty(nbytes, device=dev, dtype=torch.uint8)
-        scores, gates, M, X, R, U = _exact_views(resid, sizes)
         check(lib().pragnosia_aspin_exact_chunk_bwd(
-            _ptr(q), _ptr(k), _ptr(v), _ptr(la), _ptr(beta), _ptr(ckpt), _ptr(scores), _ptr(gates), _ptr(M), _ptr(X),
-            _ptr(R), _ptr(U), _ptr(do), _ptr(dS), _ptr(dq), _ptr(dk), _ptr(dv), _ptr(dla),
-            _ptr(dbeta) if delta else None, _ptr(dS0), _ptr(ws), nbytes, B, H, T, Dk, Dv, _stream(q)),
+            _ptr(q), _ptr(k), _ptr(v), _ptr(la), _ptr(beta), _ptr(ckpt), *_exact_ptrs(resid, sizes), _ptr(do), _ptr(dS),
+            _ptr(dq), _ptr(dk), _ptr(dv), _ptr(dla), _ptr(dbeta) if delta else None, _ptr(dS0), _ptr(ws), nbytes, B, H, T,
+            Dk, Dv, _stream(q)),
             "pragnosia_aspin_exact_chunk_bwd")
         return dq, dk, dv, dla, dbeta, dS0
     check(lib().pragnosia_aspin_exact_bwd(_ptr(q), _ptr(k), _ptr(v), _ptr(la), _ptr(beta), _ptr(ckpt), _ptr(resid),
