@@ -2,6 +2,7 @@
 Python binding declares exactly those; argument rejection happens on the host before any launch; the product
 package never imports the oracle."""
 import ctypes
+import hashlib
 import os
 import re
 
@@ -41,9 +42,21 @@ def test_binding_matches_header():
 
 
 def test_abi_version_and_error_strings(L):
-    assert L.pragnosia_abi_version() == 22
+    assert L.pragnosia_abi_version() == 23
     assert L.pragnosia_error_string(0) == b"ok"
     assert b"invalid argument" in L.pragnosia_error_string(-1)
+
+
+def test_abi_version_names_these_entry_points(L):
+    """The version is bumped with any change of the entry points: the header's declarations (comments and spacing aside)
+    are those that the version stands for."""
+    txt = ""
+    for fn in sorted(os.listdir(os.path.join(ROOT, "include"))):
+        txt += re.sub(r"/\*.*?\*/", "", open(os.path.join(ROOT, "include", fn)).read(), flags=re.S)
+    digest = hashlib.sha256("".join(txt.split()).encode()).hexdigest()[:16]
+    assert (L.pragnosia_abi_version(), digest) == (23, "d60a57fc6edb39f7"), "entry points changed: bump pragnosia_abi_version"
+    header = open(os.path.join(ROOT, "include", "pragnosia_hip.h")).read()
+    assert f"ABI version of this header ({L.pragnosia_abi_version()})" in header
 
 
 def test_arguments_rejected_before_launch(L):
