@@ -490,12 +490,12 @@ PGN_DEVICE unsigned row_base(const WaveIdx& x, int ld4, int c, bool ok) { return
 // ... and of row 16 (p / 4) + p % 4 past it: with it, load p of a lane is the B (or transposed A) operand's k = p-th
 PGN_DEVICE unsigned row_step(int p, int ld4) { return (unsigned)((16 * (p >> 2) + (p & 3)) * ld4); }
 
-// The state along the chunks, plain rule: S <- a S + X^T (f o Y) for 64 KT key rows and 16 value columns a workgroup
+// The state along the chunks, plain rule: S <- a S + X^T (f o Y) for 64 key rows and 16 value columns a workgroup
 // (key rows and value columns are independent here), X = K, Y = V, f = w forward; X = Q, Y = dO, f = e^L and S the
 // state's gradient, chunks in reverse, backward (which also leaves a <G, S_c>, one partial a wave, in hs). The state
 // entering (backward: the gradient leaving) every chunk goes to `states`. No LDS and no barrier: a wave's operands come
 // from memory two chunks ahead.
-template <int KT, bool BWD>
+template <bool BWD>
 __global__ __launch_bounds__(256) void exact_chain_plain(const float* __restrict__ xk, const float* __restrict__ yv,
                                                          const float* __restrict__ f, const float* __restrict__ eL,
                                                          const float* init, float* __restrict__ states,
@@ -507,25 +507,18 @@ __global__ __launch_bounds__(256) void exact_chain_plain(const float* __restrict
   const int bh = it.group, vb = it.sub % nvb, kb = it.sub / nvb;
   const int col = 16 * vb + x.i, kd4 = 4 * s.Dk, vd4 = 4 * s.Dv, sn = s.Dk * s.Dv;
   const bool cok = col < s.Dv;
-  unsigned kbase[KT], sbase[KT];  // an operand's and the state's offsets, the wave's m-th tile of 16 key rows
-#pragma unroll
-  for (int m = 0; m < KT; ++m) {
-    const int key = 64 * KT * kb + 16 * (x.w + 4 * m);
-    kbase[m] = row_base(x, kd4, key + x.i, key + x.i < s.Dk);
-    sbase[m] = cok ? (unsigned)(key + 4 * x.g) * vd4 + 4u * col : kNone;  // rows past Dk lie past the state's end
-  }
-  const unsigned vbase = row_base(x, vd4, col, cok);
-  f32x4 S[KT];
+  const int key = 64 * kb + 16 * x.w;  // the wave's 16 key rows
+  const unsigned kbase = row_base(x, kd4, key + x.i, key + x.i < s.Dk), vbase = row_base(x, vd4, col, cok);
+  const unsigned sbase = cok ? (unsigned)(key + 4 * x.g) * vd4 + 4u * col : kNone;  // rows past Dk: past the state's end
+  f32x4 S;
   {
     const __amdgpu_buffer_rsrc_t r = view(init == nullptr ? xk : init + (size_t)bh * sn, init == nullptr ? 0 : sn);
 #pragma unroll
-    for (int m = 0; m < KT; ++m)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) S[m][e] = bload(r, sbase[m] + e * vd4);
+    for (int e = 0; e < 4; ++e) S[e] = bload(r, sbase + e * vd4);
   }
   struct Set {
-    float k[KT][16], v[16], z[BWD ? KT : 1][4];
-    f32x4 f[4];
+    float k[16], v[16];
+    f32x4 f[4], z;
     float a;
   };
   auto load = [&](Set& u, int c) {
@@ -536,47 +529,33 @@ __global__ __launch_bounds__(256) void exact_chain_plain(const float* __restrict
     const unsigned vo = fresh(vbase);
 #pragma unroll
     for (int p = 0; p < 16; ++p) u.v[p] = bload(vr, vo + row_step(p, vd4));
+    const unsigned ko = fresh(kbase);
 #pragma unroll
-    for (int m = 0; m < KT; ++m) {
-      const unsigned ko = fresh(kbase[m]);
-#pragma unroll
-      for (int p = 0; p < 16; ++p) u.k[m][p] = bload(kr, ko + row_step(p, kd4));
-    }
+    for (int p = 0; p < 16; ++p) u.k[p] = bload(kr, ko + row_step(p, kd4));
 #pragma unroll
     for (int b = 0; b < 4; ++b) u.f[b] = *reinterpret_cast<const f32x4*>(f + ch * CT + 16 * b + 4 * x.g);
     u.a = eL[ch * CT + CT - 1];
     if constexpr (BWD) {
       const __amdgpu_buffer_rsrc_t zr = view(Sc + ch * sn, sn);
 #pragma unroll
-      for (int m = 0; m < KT; ++m)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) u.z[m][e] = bload(zr, sbase[m] + e * vd4);
+      for (int e = 0; e < 4; ++e) u.z[e] = bload(zr, sbase + e * vd4);
     }
   };
   auto step = [&](Set& u, int c) {
     const size_t ch = (size_t)bh * s.NC + c;
     const __amdgpu_buffer_rsrc_t out = view(states + ch * sn, sn);
 #pragma unroll
-    for (int m = 0; m < KT; ++m)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) bstore(out, sbase[m] + e * vd4, S[m][e]);
+    for (int e = 0; e < 4; ++e) bstore(out, sbase + e * vd4, S[e]);
     if constexpr (BWD) {
       float h = 0.f;
 #pragma unroll
-      for (int m = 0; m < KT; ++m)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) h += S[m][e] * u.z[m][e];
+      for (int e = 0; e < 4; ++e) h += S[e] * u.z[e];
       h = pgn::wave_sum(h * u.a);
       if (x.l == 0) hs[(ch * nvb * nkb + it.sub) * 4 + x.w] = h;
     }
+    S *= u.a;
 #pragma unroll
-    for (int m = 0; m < KT; ++m) S[m] *= u.a;
-#pragma unroll
-    for (int p = 0; p < 16; ++p) {
-      const float b = u.v[p] * u.f[p >> 2][p & 3];
-#pragma unroll
-      for (int m = 0; m < KT; ++m) S[m] = mfma4(u.k[m][p], b, S[m]);
-    }
+    for (int p = 0; p < 16; ++p) S = mfma4(u.k[p], u.v[p] * u.f[p >> 2][p & 3], S);
   };
   const int first = BWD ? s.NC - 1 : 0, dir = BWD ? -1 : 1;
   Set u0, u1;
@@ -594,9 +573,7 @@ __global__ __launch_bounds__(256) void exact_chain_plain(const float* __restrict
   if (last != nullptr) {
     const __amdgpu_buffer_rsrc_t r = view(last + (size_t)bh * sn, sn);
 #pragma unroll
-    for (int m = 0; m < KT; ++m)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) bstore(r, sbase[m] + e * vd4, S[m][e]);
+    for (int e = 0; e < 4; ++e) bstore(r, sbase + e * vd4, S[e]);
   }
 }
 
@@ -1191,7 +1168,7 @@ int chunk_fwd(const float* q, const float* k, const float* v, const float* la, c
     if (e != PRAGNOSIA_OK) return e;
   } else {
     const int nvb = (s.Dv + 15) / 16;
-    hipLaunchKernelGGL((exact_chain_plain<1, false>), dim3(items(s.BH, nvb * s.nkt)), dim3(256), 0, st, k, v, wt, eL,
+    hipLaunchKernelGGL((exact_chain_plain<false>), dim3(items(s.BH, nvb * s.nkt)), dim3(256), 0, st, k, v, wt, eL,
                        S0, Sc, Sfin, nullptr, nullptr, nvb, s.nkt, s);
     PGN_LAUNCHED();
   }
@@ -1220,7 +1197,7 @@ int chunk_bwd(const float* q, const float* k, const float* v, const float* la, c
     const int e = launch_chain_delta<true>(k, q, dO, beta, eL, wt, W, dv, nullptr, dSfin, G, dS0, Sc, hs, s, st);
     if (e != PRAGNOSIA_OK) return e;
   } else {
-    hipLaunchKernelGGL((exact_chain_plain<1, true>), dim3(items(s.BH, nvb * s.nkt)), dim3(256), 0, st, q, dO, eL, eL,
+    hipLaunchKernelGGL((exact_chain_plain<true>), dim3(items(s.BH, nvb * s.nkt)), dim3(256), 0, st, q, dO, eL, eL,
                        dSfin, G, dS0, Sc, hs, nvb, s.nkt, s);
     PGN_LAUNCHED();
   }
