@@ -131,9 +131,18 @@ def test_fp32_matches_oracle(scan, delta, B, H, T, Dk, Dv, s0):
 
 @pytest.mark.parametrize("B,H,T,Dk,Dv", [(1, 2, 77, 176, 176), (1, 1, 40, 384, 200)])
 def test_fp32_wide_heads_plain(scan, B, H, T, Dk, Dv):
-    """Head dims above 128, plain rule (the reference's wspin / w2spin: four or two heads of 176-384): the exact scan
-    over key and value blocks of at most 128, outputs, final state and every gradient within 1e-4 of the fp64
-    oracle."""
+    """Head dims above 128, plain rule (the reference's wspin / w2spin: four or two heads of 176-384), at lengths that
+    run in chunks over whole widths: outputs, final state and every gradient within 1e-4 of the fp64 oracle."""
+    e = _check_fp32(scan, *_fp32_case(B, H, T, Dk, Dv, False, seed=T + Dk, s0=True))
+    assert max(e.values()) < 1e-4, e
+
+
+@pytest.mark.parametrize("B,H,T,Dk,Dv", [(1, 2, 31, 176, 176), (2, 1, 9, 384, 200), (1, 1, 25, 300, 40), (2, 3, 31, 64, 64)])
+def test_fp32_wide_heads_plain_token_by_token(scan, B, H, T, Dk, Dv):
+    """The plain rule below the chunked form's least length, over several checkpoints: heads above 128 in key and value
+    blocks of at most 128, whose reads sum and whose gradients come back through the slices of q, k, v and S0."""
+    from pragnosia_amd import ops
+    assert T < ops.EXACT_CHUNK_MIN_T
     e = _check_fp32(scan, *_fp32_case(B, H, T, Dk, Dv, False, seed=T + Dk, s0=True))
     assert max(e.values()) < 1e-4, e
 
@@ -147,10 +156,11 @@ def test_fp32_wide_heads_delta(scan, B, H, T, Dk, Dv):
     assert max(e.values()) < 1e-4, e
 
 
-@pytest.mark.parametrize("delta,Dk,Dv", [(False, 128, 128), (True, 192, 96)])
+@pytest.mark.parametrize("delta,Dk,Dv", [(False, 128, 128), (True, 192, 96), (False, 176, 176), (False, 300, 40)])
 def test_fp64_wide_value_blocks(scan, delta, Dk, Dv):
     """fp64 at widths whose backward does not fit one launch's LDS (128 x 128 plain, 192 keys with the delta rule):
-    split into value blocks, forward, state and gradients within 1e-10 of the fp64 oracle."""
+    split into value blocks (and, the plain rule past 128 keys, key blocks), forward, state and gradients within 1e-10
+    of the fp64 oracle."""
     q, k, v, la, be, S0, wo, wS = (None if t is None else t.double()
                                    for t in _fp32_case(1, 2, 37, Dk, Dv, delta, seed=Dk + Dv, s0=True))
     ins = [q, k, v, la] + ([be] if delta else []) + [S0]

@@ -102,9 +102,9 @@ def test_short_conv_carrier(delta, kernel):
                                            ("xspin", 704, 4)])
 def test_wide_head_mixers_lm(mixer, d, heads):
     """The reference's few-wide-heads carriers (`src/model.py:636-643`) in a small LM: wspin at d 704 (four heads of
-    176) and w2spin at d 352 (two of 176) on the exact fp32 scan in key and value blocks of at most 128; xspin (the
-    delta rule, four heads) at d 256, where its heads are 64 wide (the bf16 kernels), and at d 704 (four heads of 176:
-    the exact fp32 scan with all 176 keys in one launch, value blocks). Logits of forward and forward_carried against
+    176) and w2spin at d 352 (two of 176) on the exact fp32 scan (in chunks over whole widths, token by token in key and
+    value blocks below 32 tokens); xspin (the delta rule, four heads) at d 256, where its heads are 64 wide (the bf16
+    kernels), and at d 704 (four heads of 176: the exact fp32 scan). Logits of forward and forward_carried against
     the oracle (fp32 exact path: 1e-4; xspin on the bf16 kernels: 2e-2), a finite backward, and the graphed greedy
     decode equal to the eager loop."""
     from pragnosia_amd.decode import GreedyDecoder, greedy_eager
