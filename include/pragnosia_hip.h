@@ -242,8 +242,8 @@ int pragnosia_aspin_exact_bwd(const void* q, const void* k, const void* v, const
  * may be one array), so a sequence can be run in pieces. It also writes (all required) states (B, H, N, Dk, Dv), the
  * state entering every chunk; scores (B, H, N, 64, 64); gates (2, B, H, N, 64), the decays from a chunk's start and to
  * its end; and for the delta rule M and X (B, H, N, 64, 64), R and U (B, H, N, 64, Dv) and the scratch W (B, H, N, 64,
- * Dk rounded up to 16); the backward reads those of all chunks. scores, gates, M, X and W are 16-byte aligned; the other
- * arrays need no more than a float's alignment (16-byte loads are used when all of them have it and Dk and Dv are
+ * Dk rounded up to 16); the backward reads those of all chunks. scores, gates, M, X and W are 16-byte aligned; the
+ * other arrays need no more than a float's alignment (16-byte loads are used when all of them have it and Dk and Dv are
  * multiples of 4). */
 int pragnosia_aspin_exact_chunk_fwd(const float* q, const float* k, const float* v, const float* la, const float* beta,
                                     const float* S0, float* o, float* S_final, float* states, float* scores,
@@ -497,13 +497,13 @@ int pragnosia_decode_tail(const float* logits, int64_t B, int64_t V, const float
                           int64_t* pos_out, int64_t* out, int64_t n_rows, int64_t* tok, float* h, float* p0s,
                           int64_t L, float* logits_rec, void* stream);
 
-/* Dense layers' weights as pragnosia_decode_gemm reads them. The table has n layers of PRAGNOSIA_FOLD_ENTRIES int64: five
- * row blocks' addresses ((rows, K) fp32), the five running row counts (a block may be empty), K, col_scale, its length G,
- * ln_bias, bias, Wt, csum, bias_out, and the layer's first workgroup (the sum of ceil(N / 16) over the layers before). A
- * layer's blocks are stacked to N rows and tiled into Wt (ceil(N / 16) 16 K floats, rows past N zero), the columns
- * scaled by col_scale ((G,) repeated over K, G a multiple of 4 dividing K; or 0); if non-zero, csum (N): the scaled
- * rows' sums, and bias_out (N): bias (or 0) plus W ln_bias (ln_bias (K) or 0), both summed in fp64. K a multiple of 16;
- * blocks, col_scale, ln_bias and Wt 16-byte aligned. `table` is read on the host, `device_table` is its copy. */
+/* Dense layers' weights as pragnosia_decode_gemm reads them. The table has n layers of PRAGNOSIA_FOLD_ENTRIES int64:
+ * five row blocks' addresses ((rows, K) fp32), the five running row counts (a block may be empty), K, col_scale, its
+ * length G, ln_bias, bias, Wt, csum, bias_out, and the layer's first workgroup (the sum of ceil(N / 16) over the layers
+ * before). A layer's blocks are stacked to N rows and tiled into Wt (ceil(N / 16) 16 K floats, rows past N zero), the
+ * columns scaled by col_scale ((G,) repeated over K, G a multiple of 4 dividing K; or 0); if non-zero, csum (N): the
+ * scaled rows' sums, and bias_out (N): bias (or 0) plus W ln_bias (ln_bias (K) or 0), both summed in fp64. K a multiple
+ * of 16; blocks, col_scale, ln_bias and Wt 16-byte aligned. `table` is read on the host, `device_table` is its copy. */
 #define PRAGNOSIA_FOLD_ENTRIES 19
 int pragnosia_decode_fold(const int64_t* table, const int64_t* device_table, int64_t n, void* stream);
 

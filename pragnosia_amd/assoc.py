@@ -101,10 +101,10 @@ def _proj_padding(width: int, tokens: int, low: bool) -> int:
     tokens and with how far off alignment the rows are; the wider product, the zero block and its copy cost the same at
     any. us a layer's training step under bf16 autocast (`low`), unpadded / padded: rows of 4 bytes' alignment (d 704:
     2134) 512 tokens 206 / 202, 2048 260 / 254, 8192 479 / 444; of 8 (d 384: 1164, d 640: 1940) 512 tokens 173 / 182 and
-    195 / 196, 1536 203 / 198 and 227 / 227, 8192 311 / 281 and 428 / 396; of 16 (d 768: 2328) 1024 tokens 228 / 228, 4096
-    317 / 314, 32768 1354 / 1313. In fp32 the rows of d 704 alone are off 16 bytes: 2048 tokens 437 / 441, 4096 688 / 665,
-    8192 1272 / 1162; the others gain nothing. Without a backward only the wider product is left: d 704 in bf16, 2048
-    tokens 86 / 89, 16384 236 / 238."""
+    195 / 196, 1536 203 / 198 and 227 / 227, 8192 311 / 281 and 428 / 396; of 16 (d 768: 2328) 1024 tokens 228 / 228,
+    4096 317 / 314, 32768 1354 / 1313. In fp32 the rows of d 704 alone are off 16 bytes: 2048 tokens 437 / 441, 4096 688
+    / 665, 8192 1272 / 1162; the others gain nothing. Without a backward only the wider product is left: d 704 in bf16,
+    2048 tokens 86 / 89, 16384 236 / 238."""
     if low:
         least = 4096 if width % 8 == 0 else 1536 if width % 4 == 0 else 512
     elif width % 4 == 0:
@@ -130,9 +130,8 @@ def assoc_scan(q, k, v, logalpha, S0=None, chunk: int = 64, recompute: bool = Fa
     (B, H, Dk, Dv) or None. Returns (o in q's dtype, S_final).
 
     As in the reference, the arithmetic is fp32, or fp64 for fp64 inputs (`rt`, `src/assoc.py:259-261`), with no
-    operand rounding: the exact kernels (any head dims for the plain rule, keys up to 384 for the delta rule; wide heads
-    run in blocks), S_final in that type. With `mm` a 16-bit type (the
-    reference's bf16 matmuls under autocast, `:149-153`) the bf16-operand MFMA kernels run instead (fp32 accumulation
+    operand rounding: the exact kernels (any head dims for the plain rule, keys up to 384 for the delta rule), S_final
+    in that type. With `mm` a 16-bit type (the reference's bf16 matmuls under autocast, `:149-153`) the bf16-operand MFMA kernels run instead (fp32 accumulation
     and state; head dim 64 or 128), S_final fp32. The result does not depend on `chunk` (the
     reference's own test), and both paths recompute in the backward what they do not save, so `chunk`, `recompute`
     and `kernel` are accepted for the signature. need_sent (this build's): also return the bf16 entering state of
@@ -408,8 +407,9 @@ class AssocCarrier(nn.Module):
         return self.on(o.to(dtype)).transpose(1, 2).reshape(B, T, H * Dk)
 
     def _gated_out(self, o):
-        """sigmoid(gate) W_o o without autograd: the gate on whichever is smaller, the d x d weight or the tokens' output
-        (at 16384 tokens of 768 under autocast, a pass of 40 us over the output becomes one of 5 over the weight)."""
+        """sigmoid(gate) W_o o without autograd: the gate on whichever is smaller, the d x d weight or the tokens'
+        output (us a layer, gate on the output / on the weight, under autocast: d 768, 1024 tokens 87 / 82, 16384 341 /
+        300; d 256, 512 tokens 60 / 57; in fp32 d 768, 1024 tokens 105 / 103, d 512, 1024 tokens 82 / 83)."""
         if o.numel() > self.o.weight.numel():
             return F.linear(o, self.o.weight * torch.sigmoid(self.gate))
         return F.linear(o, self.o.weight) * torch.sigmoid(self.gate)

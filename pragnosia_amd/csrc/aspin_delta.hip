@@ -2543,8 +2543,8 @@ int delta_par_fwd(const __bf16* q, const __bf16* k, const __bf16* v, const float
 template <int KH>
 int delta_par_bwd(const __bf16* q, const __bf16* k, const __bf16* v, const float* la, const float* beta,
                   const __bf16* sent, const __bf16* W, const __bf16* X, const __bf16* dO, const float* dS_final,
-                  __bf16* dq, __bf16* dk, __bf16* dv, float* dla, float* dbeta, float* dS0, unsigned char* ws, int64_t B,
-                  int64_t H, int64_t T, hipStream_t st) {
+                  __bf16* dq, __bf16* dk, __bf16* dv, float* dla, float* dbeta, float* dS0, unsigned char* ws,
+                  int64_t B, int64_t H, int64_t T, hipStream_t st) {
   const int NC = (int)((T + C - 1) / C), heads = (int)(B * H), hc = heads * NC, scans = heads * KH;
   constexpr size_t lds = walk_lds<KH, true>();
   const ParWorkspace L(B, H, T, 64 * KH);
@@ -2556,8 +2556,8 @@ int delta_par_bwd(const __bf16* q, const __bf16* k, const __bf16* v, const float
   if (!rc) rc = set_smem((const void*)delta_bwd_walk<KH>, lds);
   if (!rc) rc = set_smem((const void*)aspin_delta_bwd_local<KH>, local_smem<KH>());
   if (rc) return rc;
-  hipLaunchKernelGGL(delta_bwd_pre<KH>, dim3((unsigned)hc), dim3(256), bwd_pre_smem<KH>(), st, q, k, la, dO, y, F, (int)T,
-                     NC);
+  hipLaunchKernelGGL(delta_bwd_pre<KH>, dim3((unsigned)hc), dim3(256), bwd_pre_smem<KH>(), st, q, k, la, dO, y, F,
+                     (int)T, NC);
   PGN_LAUNCHED();
   hipLaunchKernelGGL(delta_bwd_walk<KH>, dim3(sub_grid(heads, 4 * KH)), dim3(320), lds, st, k, la, beta, X, y, F,
                      dS_final, dsc, dS0, (int)T, NC, heads);

@@ -10,8 +10,10 @@
 //     backward  Y = A^T dO, F = (Q o e^L)^T dO (delta_bwd_pre);  walk: dW = Y + w o (K G), drhs = X^T dW,
 //               G <- a G + F - K^T (beta e^L o drhs) (delta_bwd_walk);  the row sums of drhs (delta_bwd_rsum);
 //               aspin_delta_bwd_local
-// with the operations, roundings and sums of the one-workgroup kernels, so the results are theirs bit for bit; Y, F and
-// drhs pass through memory in fp32.
+// with the operations, roundings and sums of the one-workgroup kernels: outputs, states, W and X are theirs bit for
+// bit, and so are the gradients at head dim 128, whose one-workgroup backward is the same two kernels' work. At head
+// dim 64 that backward is one fused kernel that rounds the same operands but sums some gradients in another order; they
+// agree to bf16 rounding. Y, F and drhs pass through memory in fp32.
 //
 // A walking workgroup is bound by what one compute unit draws from memory (about 37 bytes a ns): a wave per 16 columns
 // with the scan's four in one workgroup moved 56 KB a chunk and took 1.5 us over it whatever the arithmetic. One wave
@@ -20,10 +22,11 @@
 // takes 0.7 us, of which the copies alone 0.55; the walking wave is next, bound by its own issue.
 // B4 H11 T2048 D64: forward 105 -> 55 us, backward 161 -> 82; B2 H12 T8192: 392 -> 137, 627 -> 215; B3 H6 T1000 D128:
 // 52 -> 41, 86 -> 74. Carried windows (B2 H12 T8192, 16 of 512): 158 us as affine maps of all windows and their prefix
-// (pragnosia_aspin_delta_window_maps / _prefix) -> 139; B16 H12 T1024, 2 of 512: 152 -> 94.
+// (pragnosia_aspin_delta_window_maps / _prefix) -> 139; B16 H12 T1024, 2 of 512: 152 -> 94; with few heads and long
+// sequences the maps are the faster ones (4 heads of 131072 in windows of 2048: 335 against 1502).
 
-// In workgroup numbering, the sub-items (value quarters, halves) of a head or (head, chunk) lie 8 apart: workgroup i runs
-// on XCD i mod 8, so they share one L2.
+// In workgroup numbering, the sub-items (value quarters, halves) of a head or (head, chunk) lie 8 apart: workgroup i
+// runs on XCD i mod 8, so they share one L2.
 struct Sub {
   int item, sub;
 };
@@ -47,17 +50,18 @@ constexpr int walk_lds() { return 2 * (walk_bytes<KH, BWD>() + walk_out_bytes<KH
 template <int KH>
 constexpr int walk_ahead() { return KH == 1 ? 6 : 4; }
 
-// The copying waves (thread b of 256): chunk `it` of the walk into LDS buffer it & 1 in the turn before the walking wave
-// uses it, from the register set loaded walk_ahead turns earlier; and the state and W that it left in the turn before
-// from LDS to memory (wave b / 64 key block and token block b / 64), which it would otherwise spend a third of its
-// issue slots on. Barriers: one before the walk, then one a turn, the turns rounded up to whole rounds of the sets
-// (spare ones copy the last chunk again and store nothing): with no condition inside a turn, each copy waits for its own
-// set's loads only.
+// The copying waves (thread b of 256): chunk `it` of the walk into LDS buffer it & 1 in the turn before the walking
+// wave uses it, from the register set loaded walk_ahead turns earlier; and the state and W that it left in the turn
+// before from LDS to memory (wave b / 64 key block and token block b / 64), which it would otherwise spend a third of
+// its issue slots on. Barriers: one before the walk, then one a turn, the turns rounded up to whole rounds of the sets
+// (spare ones copy the last chunk again and store nothing): with no condition inside a turn, each copy waits for its
+// own set's loads only.
 template <int KH, bool BWD>
 PGN_DEVICE void walk_copies(const __bf16* __restrict__ k, const __bf16* __restrict__ v, const __bf16* __restrict__ X,
                             const float* __restrict__ la, const float* __restrict__ be, __bf16* __restrict__ states,
-                            __bf16* __restrict__ W, const float* yb, const float* __restrict__ fb, unsigned char* smem, const DeltaRows<KH>& R, int qt, int T, int NC,
-                            int b, const WaveIdx& x) {
+                            __bf16* __restrict__ W, const float* yb, const float* __restrict__ fb,
+                            unsigned char* smem, const DeltaRows<KH>& R, int qt, int T, int NC, int b,
+                            const WaveIdx& x) {
   constexpr int DKEY = 64 * KH, A = walk_ahead<KH>();
   struct Set {
     bf16x8 k[KH][2], x[2], v;
@@ -74,10 +78,11 @@ PGN_DEVICE void walk_copies(const __bf16* __restrict__ k, const __bf16* __restri
 #pragma unroll
     for (int u = 0; u < 2; ++u) s.x[u] = load_seg(X + ((size_t)R.hw * NC + c) * C * C, C, b + 256 * u);
     if constexpr (!BWD) {  // row b / 2, 16-byte half b % 2 of the 16 columns (threads 128 apart copy the same)
-      const __amdgpu_buffer_rsrc_t vr = __builtin_amdgcn_make_buffer_rsrc(
-          const_cast<__bf16*>(v + R.vals(T) + (size_t)t0 * DKEY), (short)0, nr * DKEY * (int)sizeof(__bf16), 0x00020000);
-      s.v = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(
-                                           vr, (((b & 127) >> 1) * DKEY + 16 * qt + 8 * (b & 1)) * (int)sizeof(__bf16), 0, 0));
+      const __amdgpu_buffer_rsrc_t vr =
+          __builtin_amdgcn_make_buffer_rsrc(const_cast<__bf16*>(v + R.vals(T) + (size_t)t0 * DKEY), (short)0,
+                                            nr * DKEY * (int)sizeof(__bf16), 0x00020000);
+      const int at = (((b & 127) >> 1) * DKEY + 16 * qt + 8 * (b & 1)) * (int)sizeof(__bf16);
+      s.v = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(vr, at, 0, 0));
     }
     if constexpr (BWD) {
       s.y = *reinterpret_cast<const f32x4*>(yb + (size_t)c * kParVals + 4 * b);
@@ -124,12 +129,14 @@ PGN_DEVICE void walk_copies(const __bf16* __restrict__ k, const __bf16* __restri
       const int db = 4 * h + cw;
       const i32x2 sv = *reinterpret_cast<const i32x2*>(out + (db >> 1) * 1024 + 16 * x.l + 8 * (db & 1));
       // row j holds key rows d contiguously
-      __builtin_amdgcn_raw_buffer_store_b64(sv, sr, ((16 * qt + x.i) * DKEY + 16 * db + 4 * x.g) * (int)sizeof(__bf16), 0, 0);
+      const int at = ((16 * qt + x.i) * DKEY + 16 * db + 4 * x.g) * (int)sizeof(__bf16);
+      __builtin_amdgcn_raw_buffer_store_b64(sv, sr, at, 0, 0);
     }
     if constexpr (!BWD) {
       const f32x4 wv = *reinterpret_cast<const f32x4*>(out + 2 * KH * 1024 + cw * 1024 + 16 * x.l);
-      const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
-          W + R.vals(T) + (size_t)t0 * DKEY, (short)0, ok ? min(C, T - t0) * DKEY * (int)sizeof(__bf16) : 0, 0x00020000);
+      const __amdgpu_buffer_rsrc_t wr =
+          __builtin_amdgcn_make_buffer_rsrc(W + R.vals(T) + (size_t)t0 * DKEY, (short)0,
+                                            ok ? min(C, T - t0) * DKEY * (int)sizeof(__bf16) : 0, 0x00020000);
       __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(i32x2, quad_rows(wv, x.i)), wr,
                                             ((16 * cw + 4 * x.g + (x.i & 3)) * DKEY + 16 * qt + 4 * (x.i >> 2)) *
                                                 (int)sizeof(__bf16), 0, 0);
@@ -166,15 +173,15 @@ PGN_DEVICE void settle(f32x4 (&v)[N]) {
 }
 
 // ------------------------------------------------------------------------------------------------------------------
-// forward, walk: 5 waves per (scan, 16 value columns). WIN: the state is rebased by -shift theta (key-row pairs rotated)
-// after every `per` chunks but the last (carried windows).
+// forward, walk: 5 waves per (scan, 16 value columns). WIN: the state is rebased by -shift theta (key-row pairs
+// rotated) after every `per` chunks but the last (carried windows).
 template <int KH, bool WIN>
 __global__ __launch_bounds__(320) void delta_walk(const __bf16* __restrict__ k, const __bf16* __restrict__ v,
                                                   const float* __restrict__ la, const float* __restrict__ be,
                                                   const __bf16* __restrict__ X, const float* __restrict__ S0,
                                                   __bf16* __restrict__ W, __bf16* __restrict__ sent,
-                                                  float* __restrict__ Sfin, const float* __restrict__ theta, float shift,
-                                                  int per, int H, int T, int NC, int heads) {
+                                                  float* __restrict__ Sfin, const float* __restrict__ theta,
+                                                  float shift, int per, int H, int T, int NC, int heads) {
   constexpr int DKEY = 64 * KH;
   extern __shared__ __align__(16) unsigned char smem[];
   const WaveIdx x = wave_idx();
@@ -211,8 +218,8 @@ __global__ __launch_bounds__(320) void delta_walk(const __bf16* __restrict__ k, 
     const __bf16 *Xs = Ks + KH * TILE, *Vs = Xs + TILE;
     const float* vec = reinterpret_cast<const float*>(Ks + walk_elems<KH, false>());
     const float *Ls = vec, *eLs = vec + C, *ws = vec + 2 * C, *bs = vec + 3 * C;
-    // the turn's LDS operands in two bursts, each ahead of the products that it feeds, so the latency is paid once a burst
-    // (backward walk, B4 H11 T2048: 32 us with the reads beside their products, 25 so)
+    // the turn's LDS operands in two bursts, each ahead of the products that it feeds, so the latency is paid once a
+    // burst (backward walk, B4 H11 T2048: 32 us with the reads beside their products, 25 so)
     bf16x8 kf[4][2 * KH], xf[4][2];
     f32x4 vv[4], bv[4], ev[4], wv[4];
 #pragma unroll
@@ -475,8 +482,8 @@ __global__ __launch_bounds__(320) void delta_bwd_walk(const __bf16* __restrict__
   const DeltaRows<KH> R(bh);
   float* yb = y + (size_t)bh * NC * kParVals + qt * 1024;
   if (x.w > 0) {
-    walk_copies<KH, true>(k, nullptr, X, la, be, dSc, nullptr, yb, F + ((size_t)bh * NC * 4 + qt) * (KH * 1024), smem, R,
-                          qt, T, NC, threadIdx.x - 64, x);
+    walk_copies<KH, true>(k, nullptr, X, la, be, dSc, nullptr, yb, F + ((size_t)bh * NC * 4 + qt) * (KH * 1024), smem,
+                          R, qt, T, NC, threadIdx.x - 64, x);
     return;
   }
   const int j = 16 * qt + i;

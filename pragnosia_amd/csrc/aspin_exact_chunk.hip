@@ -24,9 +24,9 @@
 // length of its serial chain. Chunked, a head-token costs 4 D (64 + D) dense flops on the matrix cores, one state per
 // 64 tokens reaches memory, and everything but the state's own walk is parallel over chunks. B4 H4 T2048 D176 plain,
 // forward and backward: 283 ms token by token (in two key and two value blocks), 0.33 ms here; B2 H4 T1000 D192 delta:
-// 32 ms, 0.31 ms here; a forward and backward of 32 tokens (B1 H12 D64): 282 and 40 us plain, 297 and 68 us delta. Against
-// 64 bits the worst output is closer than the recurrence's, whose state takes T roundings instead of T / 64: relative
-// error 8.7e-7 against 9.7e-6 plain, 6.9e-7 against 2.7e-6 delta at those shapes.
+// 32 ms, 0.31 ms here; a forward and backward of 32 tokens (B1 H12 D64): 282 and 40 us plain, 297 and 68 us delta.
+// Against 64 bits the worst output is closer than the recurrence's, whose state takes T roundings instead of T / 64:
+// relative error 8.7e-7 against 9.7e-6 plain, 6.9e-7 against 2.7e-6 delta at those shapes.
 //
 // Decays: L is summed in fp64 and only differences (<= 0) are exponentiated, in fp32, so a long or steep run of decays
 // loses nothing to cancellation; log-decays below -1e4 (e^-1e4 = 0 in fp32) are taken as -1e4, which keeps the
@@ -76,8 +76,8 @@ struct Src {
   int ld, n_outer, n_k;
 };
 
-// A 64 x KS slice at k0, two 16-byte pieces a thread; scaled by ks[k] when given. VEC: 16-byte loads (ld, n_outer or n_k
-// multiples of 4 and p 16-byte aligned, so a piece is whole or absent); otherwise four guarded 4-byte loads.
+// A 64 x KS slice at k0, two 16-byte pieces a thread; scaled by ks[k] when given. VEC: 16-byte loads (ld, n_outer or
+// n_k multiples of 4 and p 16-byte aligned, so a piece is whole or absent); otherwise four guarded 4-byte loads.
 template <int KIND, bool VEC>
 PGN_DEVICE void fetch(f32x4 (&r)[2], const Src& s, int k0, int tid, const float* ks) {
 #pragma unroll
@@ -112,7 +112,8 @@ PGN_DEVICE void put(float* t, const f32x4 (&r)[2], int tid) {
   }
 }
 
-// Outer indices o .. o + 15, contraction 16 kk .. 16 kk + 15 of a staged slice (or of a 64 x 64 tile of pitch PR, kCols).
+// Outer indices o .. o + 15, contraction 16 kk .. 16 kk + 15 of a staged slice (or of a 64 x 64 tile of pitch PR,
+// kCols).
 template <int KIND>
 PGN_DEVICE f32x4 frag(const float* t, int o, int kk, const WaveIdx& x) {
   if constexpr (KIND == kRows) {
@@ -478,8 +479,8 @@ PGN_DEVICE float bload(__amdgpu_buffer_rsrc_t r, unsigned off) {
 PGN_DEVICE void bstore(__amdgpu_buffer_rsrc_t r, unsigned off, float v) {
   __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(int, v), r, (int)off, 0, 0);
 }
-// A value the compiler cannot derive others from across a chunk: the dozens of load addresses built on it are then a few
-// additions a chunk instead of as many registers held through the walk (174 -> 92 for the delta rule's forward with
+// A value the compiler cannot derive others from across a chunk: the dozens of load addresses built on it are then a
+// few additions a chunk instead of as many registers held through the walk (174 -> 92 for the delta rule's forward with
 // one key tile a wave).
 PGN_DEVICE unsigned fresh(unsigned v) {
   asm volatile("" : "+v"(v));
@@ -509,7 +510,8 @@ __global__ __launch_bounds__(256) void exact_chain_plain(const float* __restrict
   const bool cok = col < s.Dv;
   const int key = 64 * kb + 16 * x.w;  // the wave's 16 key rows
   const unsigned kbase = row_base(x, kd4, key + x.i, key + x.i < s.Dk), vbase = row_base(x, vd4, col, cok);
-  const unsigned sbase = cok ? (unsigned)(key + 4 * x.g) * vd4 + 4u * col : kNone;  // rows past Dk: past the state's end
+  // rows past Dk lie past the state's end
+  const unsigned sbase = cok ? (unsigned)(key + 4 * x.g) * vd4 + 4u * col : kNone;
   f32x4 S;
   {
     const __amdgpu_buffer_rsrc_t r = view(init == nullptr ? xk : init + (size_t)bh * sn, init == nullptr ? 0 : sn);
@@ -632,7 +634,8 @@ __global__ __launch_bounds__(256, KT == 1 || (KT <= 3 && !BWD) ? 2 : 1) void exa
   auto load_y = [&](int c) {
     const int t0 = s.token(c), n = min(CT, s.T - t0);
     const size_t row0 = (size_t)bh * s.T + t0, yrow = BWD ? row0 : ((size_t)bh * s.NC + c) * CT;
-    const __amdgpu_buffer_rsrc_t r = view(y + yrow * s.Dv, (BWD ? n : CT) * s.Dv), br = view(BWD ? wt : beta + row0, BWD ? 0 : n);
+    const __amdgpu_buffer_rsrc_t r = view(y + yrow * s.Dv, (BWD ? n : CT) * s.Dv);
+    const __amdgpu_buffer_rsrc_t br = view(BWD ? wt : beta + row0, BWD ? 0 : n);
     const unsigned o = fresh(ybase);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -1068,7 +1071,8 @@ bool chunk_shape_ok(int64_t B, int64_t H, int64_t T, int64_t Dk, int64_t Dv, boo
   if (delta && Dk > kMaxDkDelta) return false;
   if (Dk > 4096 || Dv > 4096 || T >= ((int64_t)1 << 28) || B * H >= ((int64_t)1 << 24)) return false;
   const int64_t nc = (T + CT - 1) / CT, tiles = 2 * ((Dk + 63) / 64) + (Dv + 63) / 64;
-  return (B * H * nc + 8) * tiles < ((int64_t)1 << 31) && (B * H + 8) * ((Dv + 15) / 16) * ((Dk + 63) / 64) < ((int64_t)1 << 31);
+  return (B * H * nc + 8) * tiles < ((int64_t)1 << 31) &&
+         (B * H + 8) * ((Dv + 15) / 16) * ((Dk + 63) / 64) < ((int64_t)1 << 31);
 }
 
 Shape shape_of(int64_t B, int64_t H, int64_t T, int64_t Dk, int64_t Dv) {
@@ -1238,7 +1242,8 @@ extern "C" int pragnosia_aspin_exact_chunk_fwd(const float* q, const float* k, c
   hipStream_t st = (hipStream_t)stream;
   // 16-byte loads where every row starts on one
   const bool vec = Dk % 4 == 0 && Dv % 4 == 0 && aligned16({q, k, v, states, U});
-#define PGN_FWD(D, V) return chunk_fwd<D, V>(q, k, v, la, beta, S0, o, S_final, states, scores, gates, M, X, R, U, W, s, st)
+#define PGN_FWD(D, V) \
+  return chunk_fwd<D, V>(q, k, v, la, beta, S0, o, S_final, states, scores, gates, M, X, R, U, W, s, st)
   if (delta) {
     if (vec) PGN_FWD(true, true);
     PGN_FWD(true, false);

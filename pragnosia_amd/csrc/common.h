@@ -128,7 +128,8 @@ PGN_DEVICE float swap_add(float a, float b) {
 }
 
 // Sum over each aligned group of N lanes, in every lane of it: the pairs of a butterfly over lane bits 0, 1, ... (the
-// mirrors are exchanges of bits 2 and 3 once the 4 and 8 lanes below hold equal sums). The lanes of a row of 16 must all be active, those of the wave for N > 16.
+// mirrors are exchanges of bits 2 and 3 once the 4 and 8 lanes below hold equal sums). The lanes of a row of 16 must
+// all be active, those of the wave for N > 16.
 template <int N>
 PGN_DEVICE float group_sum(float x) {
   if constexpr (N >= 2) x += dpp_move<0xB1>(x);   // quad_perm [1, 0, 3, 2]

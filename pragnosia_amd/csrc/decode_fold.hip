@@ -2,15 +2,15 @@
 // the layer's row blocks (up to five tensors of K columns, stacked) tiled as
 //     Wt[((t KS + s) 64 + l) 4 + e] = W'[16 t + l % 16][16 s + 4 (l / 16) + e]
 // (column tile t of 16 rows, 16-wide step s of KS = K / 16, lane l; rows past N zero) with W' = W diag(col_scale): a
-// LayerNorm's weight (K) or a per-head RMSNorm's (G, repeated), and for a folded LayerNorm the row sums of W' (csum) and
-// bias + W ln_bias, both summed in fp64.
+// LayerNorm's weight (K) or a per-head RMSNorm's (G, repeated), and for a folded LayerNorm the row sums of W' (csum)
+// and bias + W ln_bias, both summed in fp64.
 //
 // A decoder folds its whole model at the start of every generation (the parameters may have changed), so this is a
 // copy bound by memory, and by launches if each layer had its own: one launch takes a table of layers. One workgroup a
 // column tile, wave w the steps w, w + 4, ...; a lane reads 16 bytes of its row (a 64-byte piece of each of 16 rows a
-// load) and writes 16 of a contiguous KiB, and adds its row's sums on the way. 92M parameters (d 768, 12 layers, 49 dense
-// layers), host and device time: 2.8 ms as torch calls (concatenation, scaling, transposes, fp64 sums and products, then
-// copies into the step's buffers), 1.05 ms as 49 launches, 0.46 ms as one.
+// load) and writes 16 of a contiguous KiB, and adds its row's sums on the way. 92M parameters (d 768, 12 layers, 49
+// dense layers), host and device time: 2.8 ms as torch calls (concatenation, scaling, transposes, fp64 sums and
+// products, then copies into the step's buffers), 1.05 ms as 49 launches, 0.46 ms as one.
 #include "common.h"
 
 namespace {

@@ -248,13 +248,13 @@ int launch_nc(const Plan& p, const float* x, int B, int K, const float* csum, fl
   PGN_RETURN_LAUNCH();
 }
 
-// How many column tiles a workgroup takes: the count whose busiest CU has the least to do, the rounds of workgroups over
-// the CUs times a workgroup's operand pieces and products. Its x piece comes in half lines (64 bytes of a row) and costs
-// more than a contiguous weight tile: 4 for x, 3 a tile. Past three rounds of workgroups two of which fit a CU (S <= 3),
-// the last round is shared and the rounds count in fractions. us a call, cold weights, with 1 / 2 / 3 tiles: K 768, N 3072
-// (192 tiles): 16 rows 6.56 / 7.66 / 9.11, 32 rows 8.84 / 7.42 / 8.65, 64 rows 12.1 / 10.2 / 8.55; N 8192: 16 rows 9.68 /
-// 8.59 / 9.80, 32 rows 15.7 / 11.1 / 13.2, 64 rows 27.0 / 18.5 / 17.7; K 1024, N 4096: 48 rows 13.6 / 11.9 / 15.7, 64 rows
-// 17.0 / 12.1 / 17.0.
+// How many column tiles a workgroup takes: the count whose busiest CU has the least to do, the rounds of workgroups
+// over the CUs times a workgroup's operand pieces and products. Its x piece comes in half lines (64 bytes of a row) and
+// costs more than a contiguous weight tile: 4 for x, 3 a tile. Past three rounds of workgroups two of which fit a CU (S
+// <= 3), the last round is shared and the rounds count in fractions. us a call, cold weights, with 1 / 2 / 3 tiles: K
+// 768, N 3072 (192 tiles): 16 rows 6.56 / 7.66 / 9.11, 32 rows 8.84 / 7.42 / 8.65, 64 rows 12.1 / 10.2 / 8.55; N 8192:
+// 16 rows 9.68 / 8.59 / 9.80, 32 rows 15.7 / 11.1 / 13.2, 64 rows 27.0 / 18.5 / 17.7; K 1024, N 4096: 48 rows 13.6 /
+// 11.9 / 15.7, 64 rows 17.0 / 12.1 / 17.0.
 constexpr int64_t kCUs = 256;
 
 int pick_tiles(int S, int64_t NT, int64_t ZB, int64_t splits) {

@@ -142,10 +142,10 @@ __global__ __launch_bounds__(256) void gemv(const float* __restrict__ x, int B, 
 // The decode GEMV for B <= 4 sequences and K = 256 KV: one wave per RPW output rows (a one-wave workgroup, so
 // hundreds to thousands of them cover the chip and one round of loads covers the whole weight). Lane l reads the
 // 16-byte pieces 4 l + 256 u of each of its rows, so one load instruction reads 1 KiB contiguous. Every load of the
-// wave is issued before any is waited for, none behind a branch (an absent operand reads the weight and is not used) and
-// none left to the epilogue: at K 768 the LayerNorm form took 4.94 us a layer with its bias, LayerNorm bias and later
-// input pieces each a memory round trip of its own and its lane sums through the LDS unit, now 3.98 (launch 1.75, its
-// 8.3 MB of weights 1.7). The input is used as is (MODE 0), LayerNorm'd (MODE 1: the wave computes
+// wave is issued before any is waited for, none behind a branch (an absent operand reads the weight and is not used)
+// and none left to the epilogue: at K 768 the LayerNorm form took 4.94 us a layer with its bias, LayerNorm bias and
+// later input pieces each a memory round trip of its own and its lane sums through the LDS unit, now 3.98 (launch 1.75,
+// its 8.3 MB of weights 1.7). The input is used as is (MODE 0), LayerNorm'd (MODE 1: the wave computes
 // the LayerNorm of every input row itself, the row in registers, two wave reductions), or RMS-normalised per group
 // of 64 or 128 channels (MODE 2 or 3: the carrier's per-head RMSNorm; a group's channels sit on 16 or 32 consecutive
 // lanes of one piece, so its sum of squares is a four- or five-step exchange). No LDS, no barrier. NB = 1 (B = 1) or 4 (B <= 4, rows past

@@ -13,11 +13,11 @@
 // reads a value another has already advanced, and a captured graph of an even number of steps replays where the last
 // replay ended.
 //
-// Bound by its serial chain: one round trip for the logits, the reduction, one for the token's embedding. The candidates
-// are compared as unsigned keys (order_key) and reduced by lane moves in the vector unit, the waves' 16 keys by every
-// wave for itself after one barrier. Through the LDS permute unit, with float comparisons and one thread walking the 16
-// candidates, the reduction took longer than both round trips. us a launch, before / now: 1 sequence of 8192 logits 7.9 /
-// 3.7, 64 of them 8.3 / 4.2, 4 of 50257 19.0 / 9.8.
+// Bound by its serial chain: one round trip for the logits, the reduction, one for the token's embedding. The
+// candidates are compared as unsigned keys (order_key) and reduced by lane moves in the vector unit, the waves' 16 keys
+// by every wave for itself after one barrier. Through the LDS permute unit, with float comparisons and one thread
+// walking the 16 candidates, the reduction took longer than both round trips. us a launch, before / now: 1 sequence of
+// 8192 logits 7.9 / 3.7, 64 of them 8.3 / 4.2, 4 of 50257 19.0 / 9.8.
 #include "common.h"
 
 namespace {

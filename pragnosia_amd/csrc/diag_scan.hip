@@ -147,7 +147,8 @@ __global__ __launch_bounds__(NW * 64) void diag_fwd_kernel(
     if (SPW == 1 || lane >= 64 - CH) maps[p][wave][c] = own;
     __syncthreads();
     // incoming state: the block carry pushed through every earlier wave's map, the maps read kFold at a time
-    // (reads issued together, one wait per batch rather than one per wave), then through the wave's own earlier segments
+    // (reads issued together, one wait per batch rather than one per wave), then through the wave's own earlier
+    // segments
     float2 h = carry[p][c];
 #pragma unroll
     for (int s0 = 0; s0 < NW - 1; s0 += kFold) {
@@ -349,9 +350,9 @@ int launch_bwd(const float* g, const float* glr, const float* gli, const float* 
 // about 3.5 us), so with fewer 64-channel tiles than compute units the tiles are narrowed, down to 8 channels, while
 // one round of workgroups still holds them and a block (4096 / CH tokens) is not mostly past the sequence's end.
 // Narrow rows cost coalescing (at 192 tiles of 64, B16 T512 D768: 25 / 34 us forward / backward, 29 / 40 with 16
-// channels), idle units more: B4 T2048 D704, 44 tiles, 64 / 32 / 16 / 8 channels: 62 / 37 / 26 / 32 us forward, 76 / 45 /
-// 34 / 45 backward; B8 T512 D768, 96 tiles: 20 / 15 / 18 / 19 and 24 / 20 / 24 / 27; B1 T8192 D704, 11 tiles: 233 / 129 /
-// 77 / 58 and 287 / 158 / 99 / 79; B12 T512 D704, 132 tiles (264 of 32): 21 / 24 and 27 / 33.
+// channels), idle units more: B4 T2048 D704, 44 tiles, 64 / 32 / 16 / 8 channels: 62 / 37 / 26 / 32 us forward, 76 / 45
+// / 34 / 45 backward; B8 T512 D768, 96 tiles: 20 / 15 / 18 / 19 and 24 / 20 / 24 / 27; B1 T8192 D704, 11 tiles: 233 /
+// 129 / 77 / 58 and 287 / 158 / 99 / 79; B12 T512 D704, 132 tiles (264 of 32): 21 / 24 and 27 / 33.
 int channels_of(int64_t B, int64_t T, int64_t D) {
   const int64_t n64 = B * ((D + 63) / 64);
   int ch = 64;

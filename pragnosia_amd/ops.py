@@ -709,13 +709,14 @@ aspin_chunk_wide.register_autograd(_wide_backward, setup_context=_aspin_setup)
 # aspin chunked scan, delta rule: replaces delta_scan_kernel and its ops, src/assoc_kernel.py:332-704
 def delta_parallel(heads: int, NC: int, D: int, backward: bool) -> bool:
     """Whether the scan of `heads` sequences of NC chunks runs with only the state's recurrence along the chunks
-    (`pragnosia_aspin_delta_par_fwd` / `_bwd`: the same results) instead of one workgroup a scan. It spreads a scan's walk
-    over four workgroups and its other work over all chunks, which pays while one round of workgroups holds the walks and
-    there are chunks enough to cover its extra launches. us, one workgroup a scan / this form, forward and backward,
-    heads x chunks at head dim 64: 12 x 2 13/15, 14/19; 12 x 3 16/16, 19/20; 60 x 4 20/19, 25/27; 33 x 8 31/24, 44/33;
-    44 x 32 105/55, 161/82; 24 x 128 392/137, 627/215; past 64 heads 72 x 8 32/39, 45/51; 66 x 16 57/53, 84/76; 96 x 32
-    106/98, 163/187; 192 x 16 62/91, 87/176. At head dim 128: 6 x 4 19/20, 27/30; 6 x 6 24/21, 34/32; 30 x 8 31/31, 55/57;
-    24 x 32 94/67, 168/144; 12 x 64 173/97, 264/177; 36 x 16 55/68, 108/129."""
+    (`pragnosia_aspin_delta_par_fwd` / `_bwd`: the same results bit for bit, but for the gradients at head dim 64, which
+    agree to bf16 rounding) instead of one workgroup a scan. It spreads a scan's walk over four workgroups and its other
+    work over all chunks, which pays while one round of workgroups holds the walks and there are chunks enough to cover
+    its extra launches. us, one workgroup a scan / this form, forward and backward, heads x chunks at head dim 64: 12 x
+    2 13/15, 14/19; 12 x 3 16/16, 19/20; 60 x 4 20/19, 25/27; 33 x 8 31/24, 44/33; 44 x 32 105/55, 161/82; 24 x 128
+    392/137, 627/215; past 64 heads 72 x 8 32/39, 45/51; 66 x 16 57/53, 84/76; 96 x 32 106/98, 163/187; 192 x 16 62/91,
+    87/176. At head dim 128: 6 x 4 19/20, 27/30; 6 x 6 24/21, 34/32; 30 x 8 31/31, 55/57; 24 x 32 94/67, 168/144; 12 x
+    64 173/97, 264/177; 36 x 16 55/68, 108/129."""
     if D == 64:
         return heads <= (96 if NC >= 16 and not backward else 64) and NC >= (5 if backward else 4)
     return heads <= (24 if backward else 32) and NC >= (8 if backward else 6)
@@ -877,13 +878,14 @@ def aspin_delta_fused(q: Tensor, k: Tensor, v: Tensor, la: Tensor, beta: Tensor,
                       S0: Optional[Tensor]) -> tuple[Tensor, Tensor]:
     """The delta-rule scan keeping nothing for its backward but its inputs: (o bf16, S_final fp32). At head dim 64
     the forward is one kernel that forms each chunk's inverse X on chip and writes only o and S_final: X, W and the
-    per-chunk entering states never reach memory. Its backward first runs the state pass of the same kernel (no
-    output products), which writes the entering states, W and X (the same operations on the same inputs, so
-    bit-identical to what the forward formed), then the stored-state backward. At head dim 128, X, W and o come from
-    the two-kernel forward into temporaries freed on return. This is the trait of the third-party fused kernel the
-    reference's FUSED_SCAN switches to (`src/assoc.py:481-492`: state on chip, chunk states recomputed in the backward
-    instead of written per chunk and read back): the activation memory kept from forward to backward drops by 2 B/elem
-    of W, 2 B per entering-state element and 2 B per X element, for one more forward pass in the backward."""
+    per-chunk entering states never reach memory. Its backward first runs the state pass (of the same kernel, or for few
+    heads of the chunk-parallel form; no output products), which writes the entering states, W and X (the same
+    operations on the same inputs, so bit-identical to what the forward formed), then the stored-state backward. At head
+    dim 128, X, W and o come from the two-kernel forward into temporaries freed on return. This is the trait of the
+    third-party fused kernel the reference's FUSED_SCAN switches to (`src/assoc.py:481-492`: state on chip, chunk states
+    recomputed in the backward instead of written per chunk and read back): the activation memory kept from forward to
+    backward drops by 2 B/elem of W, 2 B per entering-state element and 2 B per X element, for one more forward pass in
+    the backward."""
     _require_gpu(q, k, v, la, beta, S0)
     _expect_scan("aspin_delta_fused", q, k, v, la, beta=beta, S0=S0, widths=(64, 128))
     if q.shape[-1] == 128:
@@ -895,16 +897,16 @@ def aspin_delta_fused(q: Tensor, k: Tensor, v: Tensor, la: Tensor, beta: Tensor,
 
 
 def delta_window_maps(heads: int, T: int, window: int) -> bool:
-    """Whether the carried windows of `heads` sequences of T tokens run as the windows' affine maps (every window at once,
-    twice, and a chain of one step a window) instead of one chunk-parallel walk over all chunks. The walk does less in
-    all but takes every chunk of a sequence in turn, so a long sequence of few heads is faster as maps. From the cost of
-    each, in us: a round of window workgroups over the compute units takes 3.5 and 2.9 a chunk, the chain 0.9 a window,
-    padding a partial last window five copies; the walk 0.72 a chunk and round of its four workgroups a head, the rest
-    0.0155 a chunk and head. Measured, maps / walk: 12 heads, 32768 tokens in windows of 1024 272 / 431, of 256 388 /
-    442, of 64 977 / 478; 12 heads of 8192 in 512 100 / 121; 4 heads of 131072 in 2048 335 / 1502; 24 heads of 32768 in
-    1024 493 / 541; 24 heads of 8192 in 512 156 / 136; 96 heads of 16384 in 2048 929 / 745; with a partial last window,
-    12 heads of 30000 in 1024 383 / 399, of 20000 in 512 286 / 273. Over 4 to 384 heads, 1024 to 131072 tokens and
-    windows of 64 to 2048 (246 sizes) the choice is the faster one or within 5% of it."""
+    """Whether the carried windows of `heads` sequences of T tokens run as the windows' affine maps (every window at
+    once, twice, and a chain of one step a window) instead of one chunk-parallel walk over all chunks. The walk does
+    less in all but takes every chunk of a sequence in turn, so a long sequence of few heads is faster as maps. From the
+    cost of each, in us: a round of window workgroups over the compute units takes 3.5 and 2.9 a chunk, the chain 0.9 a
+    window, padding a partial last window five copies; the walk 0.72 a chunk and round of its four workgroups a head,
+    the rest 0.0155 a chunk and head. Measured, maps / walk: 12 heads, 32768 tokens in windows of 1024 272 / 431, of 256
+    388 / 442, of 64 977 / 478; 12 heads of 8192 in 512 100 / 121; 4 heads of 131072 in 2048 335 / 1502; 24 heads of
+    32768 in 1024 493 / 541; 24 heads of 8192 in 512 156 / 136; 96 heads of 16384 in 2048 929 / 745; with a partial last
+    window, 12 heads of 30000 in 1024 383 / 399, of 20000 in 512 286 / 273. Over 4 to 384 heads, 1024 to 131072 tokens
+    and windows of 64 to 2048 (246 sizes) the choice is the faster one or within 5% of it."""
     up = lambda a, b: -(-a // b)
     NW, NC = up(T, window), up(T, CHUNK)
     rounds = up(2 * heads * NW, COMPUTE_UNITS) + up(heads * NW, COMPUTE_UNITS)
@@ -918,9 +920,9 @@ def _delta_windows_maps(q: Tensor, k: Tensor, v: Tensor, la: Tensor, beta: Tenso
     """The windows as affine maps (inputs already cast): given the chunk inverses the rule is linear in the state and
     independent per value column, so a window takes its entering state to S_out = M S_in + R. The state passes over all
     windows (R from zero entering states; M from identity states with zero values) in one launch
-    (`pragnosia_aspin_delta_window_maps`), the entering states chained by `pragnosia_aspin_delta_window_prefix`, then one
-    pass with outputs from them. A partial last window is zero-padded (zero keys, values, decay and strength leave the
-    state unchanged)."""
+    (`pragnosia_aspin_delta_window_maps`), the entering states chained by `pragnosia_aspin_delta_window_prefix`, then
+    one pass with outputs from them. A partial last window is zero-padded (zero keys, values, decay and strength leave
+    the state unchanged)."""
     B, H, T, D = q.shape
     NW = (T + window - 1) // window
     Tp = NW * window
@@ -931,8 +933,8 @@ def _delta_windows_maps(q: Tensor, k: Tensor, v: Tensor, la: Tensor, beta: Tenso
     qw, kw, vw = (t.view(BW, 1, window, D) for t in (q, k, v))
     lw, bw = la.view(BW, 1, window), beta.view(BW, 1, window)
     RM = torch.empty(2, BW, D, D, device=q.device, dtype=torch.float32)  # R, then M: both state passes, one launch
-    check(lib().pragnosia_aspin_delta_window_maps(_ptr(qw), _ptr(kw), _ptr(vw), _ptr(lw), _ptr(bw), _ptr(RM), BW, window,
-                                                  _stream(q)), "pragnosia_aspin_delta_window_maps")
+    check(lib().pragnosia_aspin_delta_window_maps(_ptr(qw), _ptr(kw), _ptr(vw), _ptr(lw), _ptr(bw), _ptr(RM), BW,
+                                                  window, _stream(q)), "pragnosia_aspin_delta_window_maps")
     Sin = torch.empty(BW, 1, D, D, device=q.device, dtype=torch.float32)
     check(lib().pragnosia_aspin_delta_window_prefix(_ptr(RM[1]), _ptr(RM[0]), _ptr(S0), _ptr(theta), float(window),
                                                     _ptr(Sin), B * H, H, NW, _stream(q)),
@@ -1006,8 +1008,8 @@ EXACT_CKPT = 8  # tokens per checkpointed state (PRAGNOSIA_EXACT_CKPT_TOKENS)
 EXACT_MAX_DK = 384  # key rows (kMaxDk)
 EXACT_MAX_DV = 128  # value columns (kMaxDv)
 EXACT_MAX_LDS = 160 * 1024
-# fp32 sequences of at least this many tokens run in chunked form on the fp32 matrix cores (aspin_exact_chunk.hip), whose
-# unit is a chunk of 64 tokens: below half a chunk the padding outweighs it. fp64 stays token by token.
+# fp32 sequences of at least this many tokens run in chunked form on the fp32 matrix cores (aspin_exact_chunk.hip),
+# whose unit is a chunk of 64 tokens: below half a chunk the padding outweighs it. fp64 stays token by token.
 EXACT_CHUNK_MIN_T = 32
 EXACT_CHUNK_MAX_D = 4096
 
@@ -1044,9 +1046,9 @@ def _dtype_code(dt: torch.dtype) -> int:
 
 
 def exact_chunked(dt: torch.dtype, heads: int, T: int, Dk: int, Dv: int, delta: bool) -> bool:
-    """Whether the exact scan of `heads` sequences of T tokens runs in chunked form (key and value widths up to 4096, the
-    delta rule's keys up to 384) rather than token by token. Its grids count tiles of chunks in 31 bits (chunk_shape_ok
-    of the kernels); what is past that stays token by token too."""
+    """Whether the exact scan of `heads` sequences of T tokens runs in chunked form (key and value widths up to 4096,
+    the delta rule's keys up to 384) rather than token by token. Its grids count tiles of chunks in 31 bits
+    (chunk_shape_ok of the kernels); what is past that stays token by token too."""
     if not (dt == torch.float32 and EXACT_CHUNK_MIN_T <= T < 1 << 28 and 0 < heads < 1 << 24
             and 0 < Dk <= (EXACT_MAX_DK if delta else EXACT_CHUNK_MAX_D) and 0 < Dv <= EXACT_CHUNK_MAX_D):
         return False
@@ -1057,8 +1059,8 @@ def exact_chunked(dt: torch.dtype, heads: int, T: int, Dk: int, Dv: int, delta: 
 
 
 def _exact_parts(B: int, H: int, T: int, Dv: int, delta: bool) -> list[int]:
-    """Sizes (floats) of what the chunked form keeps in `resid`: per chunk the scores and the two decay vectors, then for
-    the delta rule M and X, R and U (multiples of 64, so each part of the buffer is 16-byte aligned)."""
+    """Sizes (floats) of what the chunked form keeps in `resid`: per chunk the scores and the two decay vectors, then
+    for the delta rule M and X, R and U (multiples of 64, so each part of the buffer is 16-byte aligned)."""
     n = B * H * ((T + CHUNK - 1) // CHUNK) * CHUNK
     return [n * CHUNK, 2 * n] + ([n * CHUNK, n * CHUNK, n * Dv, n * Dv] if delta else [])
 
@@ -1074,9 +1076,9 @@ def _exact_ptrs(buf: Tensor, sizes: list[int]) -> list[Optional[ctypes.c_void_p]
 
 # Without a backward to keep them for, the chunked form's states and scores are scratch, and the sequences run in pieces
 # whose scratch stays within this: 2^20 tokens of four heads of 176 take 10 GB whole (plain; 21 delta). ms whole / in
-# pieces of 512 MiB: 2^18 tokens of four heads of 176 9.5 / 7.2 plain, 19.8 / 19.7 delta; 131072 tokens of twelve heads of
-# 64 2.8 / 2.9, 6.3 / 6.4; cutting heads costs more, 64 x 1024 tokens of twelve heads of 64 (1.4 GiB) 1.03 / 1.17 delta,
-# so the bound is above what such calls take.
+# pieces of 512 MiB: 2^18 tokens of four heads of 176 9.5 / 7.2 plain, 19.8 / 19.7 delta; 131072 tokens of twelve heads
+# of 64 2.8 / 2.9, 6.3 / 6.4; cutting heads costs more, 64 x 1024 tokens of twelve heads of 64 (1.4 GiB) 1.03 / 1.17
+# delta, so the bound is above what such calls take.
 EXACT_SCRATCH_BYTES = 2 << 30
 
 
@@ -1093,8 +1095,8 @@ def _exact_pieces(heads: int, T: int, Dk: int, Dv: int, delta: bool) -> tuple[in
     return max(1, min(heads, EXACT_SCRATCH_BYTES // (chunks * per))), chunks
 
 
-def _exact_chunk_fwd(q: Tensor, k: Tensor, v: Tensor, la: Tensor, beta: Optional[Tensor], S0: Optional[Tensor], o: Tensor,
-                     S: Tensor, first: int, chunks: int) -> tuple[Tensor, Tensor]:
+def _exact_chunk_fwd(q: Tensor, k: Tensor, v: Tensor, la: Tensor, beta: Optional[Tensor], S0: Optional[Tensor],
+                     o: Tensor, S: Tensor, first: int, chunks: int) -> tuple[Tensor, Tensor]:
     """The chunked exact forward of (at most) `chunks` chunks from the chunk `first` on, into o and S (inputs already
     cast, all contiguous): (ckpt, resid) of these chunks."""
     B, H, T, Dk = q.shape
@@ -1112,7 +1114,8 @@ def _exact_chunk_fwd(q: Tensor, k: Tensor, v: Tensor, la: Tensor, beta: Optional
 
 
 def _expect_exact(op: str, q: Tensor, k, v, la, beta=None, S0=None) -> None:
-    """q, k (B, H, T, Dk); v (B, H, T, Dv); la, beta (B, H, T); S0 (B, H, Dk, Dv); token by token Dk <= 384, Dv <= 128."""
+    """q, k (B, H, T, Dk); v (B, H, T, Dv); la, beta (B, H, T); S0 (B, H, Dk, Dv); token by token Dk <= 384, Dv <=
+    128."""
     if q.dim() != 4 or v is None or v.dim() != 4:
         raise PragnosiaError(f"{op}: q and v must be (B, H, T, D)")
     B, H, T, Dk = q.shape
@@ -1222,8 +1225,8 @@ def aspin_exact_bwd(q: Tensor, k: Tensor, v: Tensor, la: Tensor, beta: Optional[
         ws = torch.empty(nbytes, device=dev, dtype=torch.uint8)
         check(lib().pragnosia_aspin_exact_chunk_bwd(
             _ptr(q), _ptr(k), _ptr(v), _ptr(la), _ptr(beta), _ptr(ckpt), *_exact_ptrs(resid, sizes), _ptr(do), _ptr(dS),
-            _ptr(dq), _ptr(dk), _ptr(dv), _ptr(dla), _ptr(dbeta) if delta else None, _ptr(dS0), _ptr(ws), nbytes, B, H, T,
-            Dk, Dv, _stream(q)),
+            _ptr(dq), _ptr(dk), _ptr(dv), _ptr(dla), _ptr(dbeta) if delta else None, _ptr(dS0), _ptr(ws), nbytes, B, H,
+            T, Dk, Dv, _stream(q)),
             "pragnosia_aspin_exact_chunk_bwd")
         return dq, dk, dv, dla, dbeta, dS0
     check(lib().pragnosia_aspin_exact_bwd(_ptr(q), _ptr(k), _ptr(v), _ptr(la), _ptr(beta), _ptr(ckpt), _ptr(resid),

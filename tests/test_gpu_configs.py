@@ -102,10 +102,9 @@ def test_cfg3_one_pass_windows_full_size():
 
 def test_cfg3_delta_windows_full_size():
     """configs[3]'s shape with the delta write rule (beta = sigmoid(N(0, 1)) per token and head): the 16 windows of 512
-    through `aspin_delta_windows` (every window at once from its affine state map: two state passes, the prefix of
-    the maps with the -512 theta rebase, one output pass) against (i) the window-by-window loop on the GPU
-    (aspin_delta + aspin_rebase per window) and (ii) the CPU oracle's window loop (`oracle.aspin.assoc_scan` with
-    beta per window, `oracle.aspin.rebase` between), outputs and the final state, on the same bf16 inputs; also with
+    through `aspin_delta_windows` (one walk that rebases the state by -512 theta past each window) against (i) the
+    window-by-window loop on the GPU (aspin_delta + aspin_rebase per window) and (ii) the CPU oracle's window loop
+    (`oracle.aspin.assoc_scan` with beta per window, `oracle.aspin.rebase` between), outputs and the final state, on the same bf16 inputs; also with
     an entering state."""
     from pragnosia_amd import ops  # noqa: F401
     from pragnosia_amd.assoc import rotate

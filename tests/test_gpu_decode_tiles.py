@@ -1,5 +1,6 @@
 """The decode step's dense layers where a workgroup takes two column tiles (a partial last group, a ragged last tile, a
-partial row block) and the one-wave GEMV with operands left out, against fp64 torch; the step tail's argmax at its edges.
+partial row block) and the one-wave GEMV with operands left out, against fp64 torch; the step tail's argmax at its
+edges.
 
 Tolerance: sums of K fp32 products in any order, each within K 2^-24 of the sum of magnitudes at the worst and about
 sqrt(K) 2^-24 as rounding errors go: 1e-5 of the largest output holds both at these K with inputs of unit size."""

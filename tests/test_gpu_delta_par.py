@@ -1,8 +1,9 @@
-"""GPU: the chunk-parallel form of the delta scan (`pragnosia_aspin_delta_par_fwd` / `_bwd`) against the one-workgroup-a-scan
-kernels, which the oracle comparisons of test_gpu_delta.py hold. The two perform the same operations on the same rounded
-operands and sum in the same order, so at head dim 128 (the same two-kernel backward) everything is equal bit for bit;
-at head dim 64 the other backward is one fused kernel that rounds where this one does but sums the decay and strength
-gradients in another order: outputs and states equal, gradients to bf16 rounding (2^-8) of their largest value."""
+"""GPU: the chunk-parallel form of the delta scan (`pragnosia_aspin_delta_par_fwd` / `_bwd`) against the
+one-workgroup-a-scan kernels, which the oracle comparisons of test_gpu_delta.py hold. The two perform the same
+operations on the same rounded operands and sum in the same order, so at head dim 128 (the same two-kernel backward)
+everything is equal bit for bit; at head dim 64 the other backward is one fused kernel that rounds where this one does
+but sums the decay and strength gradients in another order: outputs and states equal, gradients to bf16 rounding (2^-8)
+of their largest value."""
 import pytest
 import torch
 import torch.nn.functional as F
@@ -35,8 +36,8 @@ def _both(x, do, dS, monkeypatch):
 @pytest.mark.parametrize("B,H,T,D,s0", [
     (1, 1, 1, 64, False), (1, 3, 63, 64, True), (1, 1, 64, 64, True), (2, 1, 65, 64, True), (1, 2, 320, 64, False),
     (3, 3, 384, 64, True), (1, 2, 385, 64, True), (1, 1, 833, 64, True), (7, 10, 130, 64, True),
-    (1, 1, 17, 128, True), (1, 3, 64, 128, False), (3, 3, 200, 128, True), (1, 2, 256, 128, True), (1, 1, 321, 128, True),
-    (2, 17, 130, 128, True),
+    (1, 1, 17, 128, True), (1, 3, 64, 128, False), (3, 3, 200, 128, True), (1, 2, 256, 128, True),
+    (1, 1, 321, 128, True), (2, 17, 130, 128, True),
 ])
 def test_matches_one_workgroup_per_scan(B, H, T, D, s0, monkeypatch):
     x, do, dS = _inputs(B, H, T, D, s0, seed=T + D)
@@ -74,8 +75,8 @@ def test_windows_match_the_window_loop(B, H, T, window, s0, maps, monkeypatch):
 
 def test_fused_forward_keeps_states_on_chip():
     """The scan that keeps nothing for its backward takes no memory beside o and S either, at a size whose plain forward
-    runs chunk-parallel and writes 22 MiB of states, W and X (the allocator may hand out up to 1 MiB more than asked for,
-    in two arrays), and gives the plain forward's outputs."""
+    runs chunk-parallel and writes 22 MiB of states, W and X (the allocator may hand out up to 1 MiB more than asked
+    for, in two arrays), and gives the plain forward's outputs."""
     from pragnosia_amd import ops
     x, _, _ = _inputs(2, 12, 2560, 64, True, seed=3)
     assert ops.delta_parallel(24, 40, 64, False)

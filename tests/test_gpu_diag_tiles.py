@@ -1,5 +1,5 @@
-"""GPU parity of the complex diagonal scan at each channel-tile width that its dispatch picks (64, 32, 16 or 8 channels a
-workgroup, by how many 64-channel tiles there are), with ragged channels and lengths around a time block's end.
+"""GPU parity of the complex diagonal scan at each channel-tile width that its dispatch picks (64, 32, 16 or 8 channels
+a workgroup, by how many 64-channel tiles there are), with ragged channels and lengths around a time block's end.
 
 Tolerance: fp32 sums along at most 1100 tokens of contributions that decay; 1e-5 in the maximum norm over the result's
 largest value (the oracle comparison of the other shapes measures 1e-6 to 3e-6)."""

@@ -137,7 +137,8 @@ def test_fp32_wide_heads_plain(scan, B, H, T, Dk, Dv):
     assert max(e.values()) < 1e-4, e
 
 
-@pytest.mark.parametrize("B,H,T,Dk,Dv", [(1, 2, 31, 176, 176), (2, 1, 9, 384, 200), (1, 1, 25, 300, 40), (2, 3, 31, 64, 64)])
+@pytest.mark.parametrize("B,H,T,Dk,Dv", [(1, 2, 31, 176, 176), (2, 1, 9, 384, 200), (1, 1, 25, 300, 40),
+                                         (2, 3, 31, 64, 64)])
 def test_fp32_wide_heads_plain_token_by_token(scan, B, H, T, Dk, Dv):
     """The plain rule below the chunked form's least length, over several checkpoints: heads above 128 in key and value
     blocks of at most 128, whose reads sum and whose gradients come back through the slices of q, k, v and S0."""

@@ -112,12 +112,13 @@ def test_chunked_non_finite_values_stay_where_the_recurrence_takes_them(delta, n
 
 
 @pytest.mark.parametrize("delta", [False, True])
-@pytest.mark.parametrize("B,H,T,Dk,Dv,mib", [(1, 2, 12000, 48, 32, 1), (3, 5, 4400, 32, 64, 4), (20, 9, 130, 64, 64, 1)])
+@pytest.mark.parametrize("B,H,T,Dk,Dv,mib", [(1, 2, 12000, 48, 32, 1), (3, 5, 4400, 32, 64, 4),
+                                             (20, 9, 130, 64, 64, 1)])
 def test_chunked_without_a_backward_bounds_its_scratch(delta, B, H, T, Dk, Dv, mib, monkeypatch):
-    """Without gradients the states, scores and inverses are scratch of a piece of the sequences (or of a group of heads)
-    at a time: the same outputs bit for bit, and no more memory than the bound (or 16 chunks of a head, a piece's least)
-    beside the outputs. The allocator may hand out up to 1 MiB more than asked for, in five arrays; whole, the scratch is
-    8 MiB and more."""
+    """Without gradients the states, scores and inverses are scratch of a piece of the sequences (or of a group of
+    heads) at a time: the same outputs bit for bit, and no more memory than the bound (or 16 chunks of a head, a piece's
+    least) beside the outputs. The allocator may hand out up to 1 MiB more than asked for, in five arrays; whole, the
+    scratch is 8 MiB and more."""
     from pragnosia_amd import ops
     x, _, _ = _inputs(B, H, T, Dk, Dv, delta, seed=19, s0=True)
     a = [x[n].cuda() if n in x else None for n in ("q", "k", "v", "la", "beta", "S0")]

@@ -45,8 +45,8 @@ def test_layer_step_records_no_memset(d, head_dim, delta):
         assert want.abs() > 0 and (got - want).abs() <= 1e-4 * want.abs() + 1e-3, (got.item(), want.item())
 
 
-@pytest.mark.parametrize("d,head_dim,delta,B,T", [(128, 64, False, 1, 1536), (128, 64, True, 3, 517), (704, 64, False, 2, 300),
-                                                  (256, 128, True, 2, 2100)])
+@pytest.mark.parametrize("d,head_dim,delta,B,T", [(128, 64, False, 1, 1536), (128, 64, True, 3, 517),
+                                                  (704, 64, False, 2, 300), (256, 128, True, 2, 2100)])
 def test_padded_projection_equals_unpadded(d, head_dim, delta, B, T, monkeypatch):
     """A training step whose projection is padded for aligned rows gives the unpadded one's output, state and gradients:
     the padded columns are read by nothing and their gradient is zero. The weight gradients differ by the unpadded

@@ -1,6 +1,7 @@
 """Every tensor whose address an op hands to the library has a dtype that the op states, not torch's default one: the
-kernels take a buffer's element size for granted, so one in a narrower default would be written past its end. On the CPU,
-with the library replaced by one that accepts every call and float64 (which no call below passes on) as the default."""
+kernels take a buffer's element size for granted, so one in a narrower default would be written past its end. On the
+CPU, with the library replaced by one that accepts every call and float64 (which no call below passes on) as the
+default."""
 import pytest
 import torch
 
@@ -52,8 +53,8 @@ def prep():
 
 def prep_proj():
     s = b(2, 3, 10, 64)
-    ops.aspin_prep_proj_bwd(b(2, 10, 582), 3, f(3), f(3), None, None, f(3), 0.0, False, f(3, 32), torch.arange(10), s, s,
-                            s, f(2, 3, 10), None)
+    ops.aspin_prep_proj_bwd(b(2, 10, 582), 3, f(3), f(3), None, None, f(3), 0.0, False, f(3, 32), torch.arange(10), s,
+                            s, s, f(2, 3, 10), None)
 
 
 def delta():

@@ -50,7 +50,8 @@ def test_exact_chunked_is_what_the_library_takes():
         for heads, T, Dk, Dv in cases:
             takes = lib().pragnosia_aspin_exact_chunk_bwd_workspace_bytes(heads, 1, T, Dk, Dv, int(delta)) >= 0
             assert exact_chunked(torch.float32, heads, T, Dk, Dv, delta) == takes, (heads, T, Dk, Dv, delta)
-    assert not exact_chunked(torch.float32, 4, 31, 64, 64, False) and not exact_chunked(torch.float64, 4, 64, 64, 64, False)
+    assert not exact_chunked(torch.float32, 4, 31, 64, 64, False)
+    assert not exact_chunked(torch.float64, 4, 64, 64, 64, False)
 
 
 def test_carried_windows_take_the_faster_form():
@@ -69,7 +70,8 @@ def test_projection_padding_by_alignment_and_tokens():
     from pragnosia_amd.assoc import _proj_padding
     for width, least in ((2134, 512), (1164, 1536), (1940, 1536), (2328, 4096), (776, 4096)):
         assert _proj_padding(width, least - 1, True) == 0
-        assert _proj_padding(width, least, True) == -width % 64 and (width + _proj_padding(width, least, True)) % 64 == 0
+        pad = _proj_padding(width, least, True)
+        assert pad == -width % 64 and (width + pad) % 64 == 0
     assert _proj_padding(2304, 1 << 20, True) == 0
     assert _proj_padding(2134, 4096, False) == 42 and _proj_padding(2134, 4095, False) == 0
     assert _proj_padding(1164, 1 << 20, False) == 0
