@@ -707,19 +707,24 @@ aspin_chunk_wide.register_autograd(_wide_backward, setup_context=_aspin_setup)
 
 # ---------------------------------------------------------------------------------------------------------------
 # aspin chunked scan, delta rule: replaces delta_scan_kernel and its ops, src/assoc_kernel.py:332-704
-def delta_parallel(heads: int, NC: int, D: int, backward: bool) -> bool:
-    """Whether the scan of `heads` sequences of NC chunks runs with only the state's recurrence along the chunks
-    (`pragnosia_aspin_delta_par_fwd` / `_bwd`: the same results bit for bit, but for the gradients at head dim 64, which
-    agree to bf16 rounding) instead of one workgroup a scan. It spreads a scan's walk over four workgroups and its other
-    work over all chunks, which pays while one round of workgroups holds the walks and there are chunks enough to cover
-    its extra launches. us, one workgroup a scan / this form, forward and backward, heads x chunks at head dim 64: 12 x
-    2 13/15, 14/19; 12 x 3 16/16, 19/20; 60 x 4 20/19, 25/27; 33 x 8 31/24, 44/33; 44 x 32 105/55, 161/82; 24 x 128
-    392/137, 627/215; past 64 heads 72 x 8 32/39, 45/51; 66 x 16 57/53, 84/76; 96 x 32 106/98, 163/187; 192 x 16 62/91,
-    87/176. At head dim 128: 6 x 4 19/20, 27/30; 6 x 6 24/21, 34/32; 30 x 8 31/31, 55/57; 24 x 32 94/67, 168/144; 12 x
-    64 173/97, 264/177; 36 x 16 55/68, 108/129."""
+def delta_parallel(heads: int, NC: int, D: int, backward: bool, states: bool = True) -> bool:
+    """Whether the scan of `heads` sequences of NC chunks (`states`: a forward whose entering states are wanted) runs with
+    only the state's recurrence along the chunks (`pragnosia_aspin_delta_par_fwd` / `_bwd`: the same results bit for bit,
+    but for the gradients at head dim 64, which agree to bf16 rounding) instead of one workgroup a scan. It spreads a
+    scan's walk over four workgroups and its other work over all chunks, which pays while one round of workgroups holds
+    the walks and there are chunks enough to cover its extra launches. us, one workgroup a scan / this form, forward and
+    backward, heads x chunks at head dim 64: 12 x 2 13/15, 14/19; 12 x 3 16/16, 19/20; 60 x 4 20/19, 25/27; 33 x 8 31/24,
+    44/33; 44 x 32 105/55, 161/82; 24 x 128 392/137, 627/215; past 64 heads 72 x 8 32/39, 45/51; 66 x 16 57/53, 84/76; 96
+    x 32 106/98, 163/187; 192 x 16 62/91, 87/176. At head dim 128: 6 x 4 19/20, 27/30; 6 x 6 24/21, 34/32; 30 x 8 31/31,
+    55/57; 24 x 32 94/67, 168/144; 12 x 64 173/97, 264/177; 36 x 16 55/68, 108/129. This form writes the states in any
+    case; the other saves it where they are not wanted, at head dim 128 up to 8 us: 12 x 6 20.7/20.9, 12 x 10 29.1/26.4;
+    18 x 8 25.2/27.5, 18 x 10 29.6/29.3; 24 x 12 35.6/37.1, 24 x 16 44.5/42.0; 32 x 8 26.6/30.7, 32 x 12 36.6/38.2, 32 x
+    16 45.5/44.0 (a training step of 24 x 10, states wanted, 92.8/85.7)."""
     if D == 64:
         return heads <= (96 if NC >= 16 and not backward else 64) and NC >= (5 if backward else 4)
-    return heads <= (24 if backward else 32) and NC >= (8 if backward else 6)
+    if backward:
+        return heads <= 24 and NC >= 8
+    return heads <= 32 and NC >= (6 if states or heads <= 12 else 10 if heads <= 18 else 14)
 
 
 def _delta_par_fwd(q: Tensor, k: Tensor, v: Tensor, la: Tensor, beta: Tensor, S0: Optional[Tensor], want_o: bool,
@@ -755,7 +760,7 @@ def aspin_delta(q: Tensor, k: Tensor, v: Tensor, la: Tensor, beta: Tensor, S0: O
     B, H, T, D = q.shape
     NC = (T + CHUNK - 1) // CHUNK
     dev = q.device
-    if delta_parallel(B * H, NC, D, False):
+    if delta_parallel(B * H, NC, D, False, want_sent):
         o, S, sent, W, X = _delta_par_fwd(q, k, v, la, beta, S0, True)
         return o, S, (sent if want_sent else q.new_empty(0, dtype=torch.bfloat16)), W, X
     o = torch.empty(B, H, T, D, device=dev, dtype=torch.bfloat16)

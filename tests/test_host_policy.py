@@ -75,3 +75,18 @@ def test_projection_padding_by_alignment_and_tokens():
     assert _proj_padding(2304, 1 << 20, True) == 0
     assert _proj_padding(2134, 4096, False) == 42 and _proj_padding(2134, 4095, False) == 0
     assert _proj_padding(1164, 1 << 20, False) == 0
+
+
+def test_delta_form_by_heads_and_chunks():
+    """The chunk-parallel delta form at head dim 128: forward from six chunks where the states are wanted, else from more
+    chunks the more heads there are, backward from eight; at 64 from four and five."""
+    from pragnosia_amd.ops import delta_parallel
+    for heads, least in ((1, 6), (12, 6), (13, 10), (18, 10), (19, 14), (32, 14)):
+        assert delta_parallel(heads, least, 128, False, False)
+        assert not delta_parallel(heads, least - 1, 128, False, False)
+        assert delta_parallel(heads, 6, 128, False) and not delta_parallel(heads, 5, 128, False)
+    assert not delta_parallel(33, 1000, 128, False) and not delta_parallel(25, 1000, 128, True)
+    assert delta_parallel(24, 8, 128, True) and not delta_parallel(24, 7, 128, True)
+    assert delta_parallel(64, 4, 64, False) and not delta_parallel(64, 3, 64, False)
+    assert delta_parallel(96, 16, 64, False) and not delta_parallel(96, 15, 64, False)
+    assert delta_parallel(64, 5, 64, True) and not delta_parallel(65, 100, 64, True)
