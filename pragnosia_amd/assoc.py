@@ -163,7 +163,9 @@ def _exact_scan(q, k, v, logalpha, beta, S0, want):
     every write (r = v - P^T k), so its keys stay in one launch, up to EXACT_MAX_DK = 384."""
     Dk, Dv = q.shape[-1], v.shape[-1]
     dt = torch.float64 if q.dtype == torch.float64 else torch.float32
-    if _op_mod.exact_chunked(dt, q.shape[0] * q.shape[1], q.shape[2], Dk, Dv, beta is not None):
+    # up to 64 wide both forms take the call whole; the op picks
+    if (Dk <= 64 and Dv <= 64) or _op_mod.exact_chunked(dt, q.shape[0] * q.shape[1], q.shape[2], Dk, Dv,
+                                                        beta is not None, bool(want)):
         o, S, _, _ = _op.aspin_exact(q, k, v, logalpha, beta, S0, want)
         return o, S
     if beta is not None and Dk > _op_mod.EXACT_MAX_DK:

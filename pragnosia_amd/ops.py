@@ -1013,7 +1013,7 @@ EXACT_CKPT = 8  # tokens per checkpointed state (PRAGNOSIA_EXACT_CKPT_TOKENS)
 EXACT_MAX_DK = 384  # key rows (kMaxDk)
 EXACT_MAX_DV = 128  # value columns (kMaxDv)
 EXACT_MAX_LDS = 160 * 1024
-# fp32 sequences of at least this many tokens run in chunked form on the fp32 matrix cores (aspin_exact_chunk.hip),
+# fp32 sequences of at least this many tokens may run in chunked form on the fp32 matrix cores (aspin_exact_chunk.hip),
 # whose unit is a chunk of 64 tokens: below half a chunk the padding outweighs it. fp64 stays token by token.
 EXACT_CHUNK_MIN_T = 32
 EXACT_CHUNK_MAX_D = 4096
@@ -1050,12 +1050,43 @@ def _dtype_code(dt: torch.dtype) -> int:
     return 1 if dt == torch.float64 else 0
 
 
-def exact_chunked(dt: torch.dtype, heads: int, T: int, Dk: int, Dv: int, delta: bool) -> bool:
-    """Whether the exact scan of `heads` sequences of T tokens runs in chunked form (key and value widths up to 4096,
-    the delta rule's keys up to 384) rather than token by token. Its grids count tiles of chunks in 31 bits
-    (chunk_shape_ok of the kernels); what is past that stays token by token too."""
+def exact_chunk_pays(heads: int, T: int, Dk: int, Dv: int, delta: bool, grad: bool) -> bool:
+    """Whether the chunked form of the exact scan is the faster one, forward (grad False) or forward and backward. It pads
+    every chunk to 64 tokens and forms 64 x 64 scores whatever the widths, and has four to nine launches; token by token a
+    call is one launch each way (more past 128 wide, where the chunked form wins throughout) whose workgroups, one a head,
+    take a token in turn. From the cost of each in us: token by token a step of 0.24 to 0.3 plus what the widths add, all
+    heads at once up to about 40000 value columns and in proportion past them; chunked its launches, a step a chunk, and
+    the chunks' products. us, token by token / chunked, forward and step, heads x tokens x width: plain 12 x 64 x 64 33/16,
+    543/39; 4096 x 64 x 64 207/194, 4663/581; 1024 x 32 x 64 30/37, 571/108; 1024 x 64 x 16 25/23, 127/69; 4096 x 64 x 8
+    28/64, 120/209; delta 12 x 32 x 64 22/26, 291/68; 12 x 64 x 64 41/29, 574/76; 1024 x 64 x 32 36/68, 241/205; 4096 x
+    256 x 16 160/691, 784/2389. At 620 sizes (1 to 4096 heads, 32 to 300 tokens, 8 to 128 wide) the choice is the faster
+    one or within 5% of it but for 13, within 23% there."""
+    if Dk > 128 or Dv > 128:
+        return True
+    NC, products = (T + CHUNK - 1) // CHUNK, Dk * Dv + 32 * (Dk + Dv)
+    rows = 4 * exact_rows_per_lane(Dk)  # token by token the key rows are padded to 8, 16, 32, 64 or 128
+    wide = max(rows, Dv, 16)
+    if grad:
+        step, full = (1.23 if delta else 1.03) + 0.002 * rows * Dv, heads * wide / 37700
+        launches, chunk, each = (38, 4.9, 0.1 + 1.6e-5 * products) if delta else (17, 2.3, 0.036 + 9e-6 * products)
+        launches += (0.058 if delta else 0.028) * (Dk + Dv)
+    else:
+        step = (0.3 + 0.0043 * rows) if delta else (0.24 + 0.0033 * rows)
+        full = heads * wide * max(1, wide / 64) / 40500
+        launches, chunk, each = (15, 2.0, 0.028 + 5.1e-6 * products) if delta else (6.7, 1.04, 0.0094 + 2.7e-6 * products)
+        launches += (0.021 if delta else 0.013) * (Dk + Dv)
+    chunked, token = launches + NC * (chunk + heads * each), T * step  # both without what one launch takes
+    return chunked * chunked < token * token * (1 + full * full)
+
+
+def exact_chunked(dt: torch.dtype, heads: int, T: int, Dk: int, Dv: int, delta: bool, grad: bool = True) -> bool:
+    """Whether the exact scan of `heads` sequences of T tokens (`grad`: keeping what a backward reads) runs in chunked form
+    (key and value widths up to 4096, the delta rule's keys up to 384) rather than token by token: where it pays
+    (`exact_chunk_pays`) and its grids, which count tiles of chunks in 31 bits (chunk_shape_ok of the kernels), hold it."""
     if not (dt == torch.float32 and EXACT_CHUNK_MIN_T <= T < 1 << 28 and 0 < heads < 1 << 24
             and 0 < Dk <= (EXACT_MAX_DK if delta else EXACT_CHUNK_MAX_D) and 0 < Dv <= EXACT_CHUNK_MAX_D):
+        return False
+    if not exact_chunk_pays(heads, T, Dk, Dv, delta, grad):
         return False
     if heads * (T + CHUNK) * (Dk + Dv + 128) < 1 << 34:  # far within both
         return True
@@ -1138,8 +1169,8 @@ def aspin_exact(q: Tensor, k: Tensor, v: Tensor, la: Tensor, beta: Optional[Tens
     """The scan with fp32 operands (fp64 when q is fp64), plain rule, or the delta rule when beta is given.
     q, k (B, H, T, Dk), v (B, H, T, Dv), la and beta (B, H, T), S0 (B, H, Dk, Dv) or None. Returns (o (B, H, T, Dv),
     S_final (B, H, Dk, Dv), ckpt, resid) in the compute dtype; ckpt and resid are what the backward reads, empty unless
-    want_ckpt (else they are scratch, of about EXACT_SCRATCH_BYTES at the most). fp32 sequences of EXACT_CHUNK_MIN_T
-    tokens or more run in chunked form (`exact_chunked`; any widths, the delta rule's keys up to 384): ckpt is the state
+    want_ckpt (else they are scratch, of about EXACT_SCRATCH_BYTES at the most). fp32 sequences run in chunked form where
+    that pays (`exact_chunked`; any widths, the delta rule's keys up to 384): ckpt is the state
     entering every 64 tokens, resid one flat buffer of the chunks' scores, decays and (delta) inverses and residuals.
     The rest runs token by token, Dk <= 384 and Dv <= 128 (wide keys take fewer value columns: exact_value_cap; the
     library refuses what does not fit its LDS): ckpt is the state entering every 8 tokens, resid the delta rule's
@@ -1154,7 +1185,7 @@ def aspin_exact(q: Tensor, k: Tensor, v: Tensor, la: Tensor, beta: Optional[Tens
     dev = q.device
     o = torch.empty(B, H, T, Dv, device=dev, dtype=dt)
     S = torch.empty(B, H, Dk, Dv, device=dev, dtype=dt)
-    if exact_chunked(dt, B * H, T, Dk, Dv, beta is not None):
+    if exact_chunked(dt, B * H, T, Dk, Dv, beta is not None, want_ckpt):
         NC = (T + CHUNK - 1) // CHUNK
         heads, chunks = (B * H, NC) if want_ckpt else _exact_pieces(B * H, T, Dk, Dv, beta is not None)
         if heads == B * H and chunks == NC:

@@ -36,13 +36,15 @@ def test_backward_splits_sooner():
     assert seg_chunks(192, 8, range(1, 9), "bwd") == 8
 
 
-def test_exact_chunked_is_what_the_library_takes():
+def test_exact_chunked_is_what_the_library_takes(monkeypatch):
     """The exact scan runs in chunked form only where the library's chunked entry points take the sizes; the rest stays
     with the token-by-token form, which takes more sequences."""
     import torch
 
+    from pragnosia_amd import ops
     from pragnosia_amd._lib import lib
     from pragnosia_amd.ops import exact_chunked
+    monkeypatch.setattr(ops, "exact_chunk_pays", lambda *a: True)
     cases = [(1, 32, 1, 1), (4, 2048, 176, 176), (1, 1 << 20, 352, 352), ((1 << 24) - 1, 32, 1, 1), (1 << 24, 32, 1, 1),
              (1, (1 << 28) - 1, 16, 16), (1, 1 << 28, 16, 16), (1 << 20, 65536, 64, 64), (1 << 20, 16384, 4, 4),
              ((1 << 24) - 1, 64, 8, 4096), (2, 100, 400, 16), (2, 100, 4097, 16), (2, 100, 16, 4097)]
@@ -90,3 +92,17 @@ def test_delta_form_by_heads_and_chunks():
     assert delta_parallel(64, 4, 64, False) and not delta_parallel(64, 3, 64, False)
     assert delta_parallel(96, 16, 64, False) and not delta_parallel(96, 15, 64, False)
     assert delta_parallel(64, 5, 64, True) and not delta_parallel(65, 100, 64, True)
+
+
+def test_exact_form_by_heads_tokens_and_width():
+    """The exact scan's chunked form where its products cost less than the token-by-token steps: wide heads, few heads over
+    many tokens, and most training steps; not many narrow heads over few tokens."""
+    from pragnosia_amd.ops import exact_chunk_pays
+    #  heads, T, Dk, Dv, delta, grad
+    for case in ((4, 32, 176, 176, False, False), (4096, 32, 16, 200, True, True), (12, 64, 64, 64, False, False),
+                 (12, 32, 64, 64, True, True), (4096, 64, 64, 64, False, True), (1024, 256, 32, 32, False, False),
+                 (12, 64, 64, 64, True, False), (1, 256, 8, 8, True, False)):
+        assert exact_chunk_pays(*case), case
+    for case in ((4096, 64, 8, 8, False, False), (4096, 64, 8, 8, False, True), (12, 32, 64, 64, True, False),
+                 (1024, 64, 32, 32, True, False), (4096, 256, 16, 16, True, True), (1024, 32, 64, 64, False, False)):
+        assert not exact_chunk_pays(*case), case
