@@ -61,6 +61,32 @@ class MLP(nn.Module):
         return x + linear(F.gelu(linear(layer_norm(x, self.n), self.a)), self.b)
 
 
+def _rows(W, x):
+    """F.embedding(x, W) as an indexed selection: the same values, and a gradient that adds rows into a cleared table
+    (in fp32 also for a 16-bit table, as F.embedding's sums are), with no sort."""
+    acc = W if W.dtype in (torch.float32, torch.float64) else W.float()
+    return acc.index_select(0, x.reshape(-1)).to(W.dtype).view(*x.shape, W.shape[1])
+
+
+class Embedding(nn.Embedding):
+    """nn.Embedding for a training step that may be captured in a HIP graph. Past 3072 indices torch's gradient sorts
+    them and compacts the sorted list with a partition kernel whose look-back state a memset clears. Captured, a memset
+    has not taken effect here on replays after the first; the step of 4 x 2048 tokens faulted in that kernel. So a
+    capture (and a traced step, which may be captured later) of more indices selects rows by index, whose gradient is
+    an indexed addition: the order of a row's fp32 sum then varies from replay to replay. An eager step, and any step
+    of fewer indices, is torch's."""
+
+    SORTED_FROM = 3073  # indices from which torch's gradient takes the sort
+
+    def forward(self, x):
+        if (self.weight.is_cuda and x.numel() >= self.SORTED_FROM and torch.is_grad_enabled()
+                and self.padding_idx is None and self.max_norm is None
+                and not (self.scale_grad_by_freq or self.sparse)
+                and (torch.compiler.is_compiling() or torch.cuda.is_current_stream_capturing())):
+            return _rows(self.weight, x)
+        return super().forward(x)
+
+
 class LM(nn.Module):
     def __init__(self, vocab=8192, d=768, layers=12, mlp_mult=4, ctx=512, mixer="aspin", norm="ln", short_conv=0,
                  **unused):
@@ -68,8 +94,8 @@ class LM(nn.Module):
         if mixer not in MIXERS:
             raise PragnosiaError(f"LM: mixer {mixer!r} is outside this build (supported: {sorted(MIXERS)})")
         self.vocab, self.d, self.layers, self.ctx, self.mixer, self.norm = vocab, d, layers, ctx, mixer, norm
-        self.e = nn.Embedding(vocab, d)
-        self.p = nn.Embedding(ctx, d)
+        self.e = Embedding(vocab, d)
+        self.p = Embedding(ctx, d)
         self.mix = nn.ModuleList([MIXERS[mixer](d) for _ in range(layers)])
         self.mlp = nn.ModuleList([MLP(d, mlp_mult) for _ in range(layers)])
         self.n = nn.LayerNorm(d)
