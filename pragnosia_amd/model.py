@@ -29,7 +29,7 @@ import torch.utils.checkpoint
 
 from ._lib import PragnosiaError
 from .assoc import AssocCarrier
-from .ops import layer_norm, linear
+from .ops import capturing, layer_norm, linear
 from .spin import SpinCarrier
 
 MIXERS = {
@@ -81,8 +81,7 @@ class Embedding(nn.Embedding):
     def forward(self, x):
         if (self.weight.is_cuda and x.numel() >= self.SORTED_FROM and torch.is_grad_enabled()
                 and self.padding_idx is None and self.max_norm is None
-                and not (self.scale_grad_by_freq or self.sparse)
-                and (torch.compiler.is_compiling() or torch.cuda.is_current_stream_capturing())):
+                and not (self.scale_grad_by_freq or self.sparse) and capturing()):
             return _rows(self.weight, x)
         return super().forward(x)
 

@@ -54,6 +54,36 @@ def colsum(x: Tensor) -> Tensor:
     return (torch.ones(1, rows, device=x.device, dtype=x2.dtype) @ x2).reshape(x.shape[1:])
 
 
+def capturing() -> bool:
+    """Whether the call runs in a HIP graph's capture, or in a trace whose result may be captured later."""
+    return torch.compiler.is_compiling() or torch.cuda.is_current_stream_capturing()
+
+
+class _OverRows(torch.autograd.Function):
+    """v (d,) rounded to `dtype` as `rows` equal rows; the gradient's column sum is a GEMM against ones in v's dtype."""
+
+    @staticmethod
+    def forward(ctx, v, rows, dtype):
+        ctx.dtype = v.dtype
+        return v.to(dtype).expand(rows, -1)
+
+    @staticmethod
+    def backward(ctx, g):
+        with torch.autocast("cuda", enabled=False):
+            g = g.to(ctx.dtype)
+            return (g.new_ones(1, g.shape[0]) @ g)[0], None, None
+
+
+def over_rows(v: Tensor, like: Tensor, dtype=None) -> Tensor:
+    """v (d,), in `dtype` (its own if None), broadcast to like's shape (..., d). In a capture its gradient is a sum in
+    v's dtype that records no memset: the one autograd applies to a broadcast operand over many rows is a multi-block
+    reduction (see `colsum`). An eager step keeps autograd's, whose host share is the smaller."""
+    dtype = dtype or v.dtype
+    if not (like.is_cuda and like.numel() and torch.is_grad_enabled() and v.requires_grad and capturing()):
+        return v.to(dtype).expand(like.shape)
+    return _OverRows.apply(v, like.numel() // like.shape[-1], dtype).view(like.shape)
+
+
 @torch.library.custom_op("pragnosia::wgrad", mutates_args=())
 def wgrad(dy: Tensor, x: Tensor) -> Tensor:
     """The weight gradient of y = x Wᵀ over token rows, dy (K, M) and x (K, N) bf16 → dW = dyᵀ x (M, N) fp32: the

@@ -11,7 +11,7 @@ import torch
 import torch.nn as nn
 
 from ._lib import PragnosiaError
-from .ops import layer_norm, linear
+from .ops import capturing, layer_norm, linear, over_rows
 from .scan import scan_hip
 
 
@@ -57,13 +57,21 @@ class SpinCarrier(nn.Module):
             raise PragnosiaError("SpinCarrier runs on a ROCm GPU only; there is no CPU path")
         z = layer_norm(x, self.ln)  # self.ln(x), in the dtype the projections compute in
         mag, ang = self.lam()
-        # per-token log-magnitude <= 0: the recurrence gate scales the channel's timescale
-        logmag = -self.gate_c * torch.sigmoid(linear(z, self.Wr)) * (-torch.log(mag))
+        # per-token log-magnitude <= 0: the recurrence gate scales the channel's timescale. The channels' parameters and
+        # the gate are broadcast over the tokens by `over_rows`: captured, autograd's own sums over many tokens (from
+        # 3 x 1999 x 256 on, not at 64 x 128) record memsets, three a layer
+        r = torch.sigmoid(linear(z, self.Wr))
+        logmag = -self.gate_c * r * over_rows(-torch.log(mag), r)
         # per-token input normalisation sqrt(1 - |lambda_t|^2), its argument clamped to bound the derivative
         gam = torch.sqrt((1.0 - torch.exp(2.0 * logmag)).clamp_min(1e-6))
         u = self.B(z) * gam * torch.sigmoid(linear(z, self.Wi))
-        y, h = scan_hip(u, logmag, ang.expand_as(logmag), h0)
-        return x + torch.sigmoid(self.gate) * self.C(y), h
+        y, h = scan_hip(u, logmag, over_rows(ang, logmag), h0)
+        out = self.C(y)
+        gate = torch.sigmoid(self.gate)
+        if capturing():
+            # the sum in fp32, then rounded to the product's type, in which autograd gives it
+            gate = over_rows(gate.to(out.dtype).to(gate.dtype).expand(self.d), out, out.dtype)
+        return x + gate * out, h
 
     def forward_windows(self, x, window: int, h0=None):
         """Consecutive windows of `window` tokens with the state carried from each into the next: nothing in this

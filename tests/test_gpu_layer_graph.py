@@ -1,4 +1,4 @@
-"""GPU: one AssocCarrier's training step captured in a HIP graph, at the widths of the models trained on it."""
+"""GPU: one carrier layer's training step captured in a HIP graph, at the widths of the models trained on it."""
 import pytest
 import torch
 
@@ -43,6 +43,42 @@ def test_layer_step_records_no_memset(d, head_dim, delta):
         torch.cuda.synchronize()
         want = step()[gate]
         assert want.abs() > 0 and (got - want).abs() <= 1e-4 * want.abs() + 1e-3, (got.item(), want.item())
+
+
+@pytest.mark.parametrize("d,B,T", [(704, 4, 2048), (256, 3, 1999)])
+def test_diagonal_layer_step_records_no_memset(d, B, T):
+    """SpinCarrier: the timescales, frequencies and the gate are broadcast over all tokens, and their gradients' sums
+    record no memset. The replays give the eager step's gradients to the order of fp32 sums; the gate's, a sum
+    that autograd rounds to the product's type, to one step of bf16 (2^-7)."""
+    from pragnosia_amd.spin import SpinCarrier
+    torch.manual_seed(d)
+    with torch.device("cuda"):
+        m = SpinCarrier(d, gated="rf")
+        x, t = torch.zeros(B, T, d), torch.randn(B, T, d)
+    params = list(m.parameters())
+
+    def step():
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            y, _ = m(x)
+        return torch.autograd.grad(y, params, t)
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        for _ in range(2):
+            step()
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        out = step()
+    assert _memset_nodes(graph) == 0
+    for _ in range(6):
+        x.normal_()
+        graph.replay()
+        got = [o.clone() for o in out]
+        torch.cuda.synchronize()
+        for (n, _), a, b in zip(m.named_parameters(), got, step()):
+            assert (a - b).norm() <= (2.0 ** -7 if n == "gate" else 1e-5) * b.norm(), n
 
 
 @pytest.mark.parametrize("d,head_dim,delta,B,T", [(128, 64, False, 1, 1536), (128, 64, True, 3, 517),
