@@ -52,7 +52,13 @@ def rotate(x, theta, pos):
     """Rotation of interleaved channel pairs (x[..., 2i], x[..., 2i+1]) by angle pos * theta[h, i]
     (`src/assoc.py:34-39`): x (B, H, T, dk), theta (H, dk/2), pos (T,). A utility with the reference's signature;
     the module's own rotations run inside the prep, rebase and decode kernels."""
-    ang = pos.reshape(1, 1, -1, 1).to(theta.dtype) * theta.reshape(1, theta.shape[0], 1, theta.shape[1])
+    if theta.is_cuda and _op_mod.capturing():
+        # autograd's sum of theta's gradient over the positions (4 heads of 176, 2048 of them) would record a memset
+        th = _op_mod.over_rows(theta.reshape(-1), (pos.numel(), theta.numel()))
+        th = th.reshape(-1, *theta.shape).transpose(0, 1).unsqueeze(0)
+    else:
+        th = theta.reshape(1, theta.shape[0], 1, theta.shape[1])
+    ang = pos.reshape(1, 1, -1, 1).to(theta.dtype) * th
     c, s = torch.cos(ang), torch.sin(ang)
     even, odd = x[..., 0::2], x[..., 1::2]
     return torch.stack((even * c - odd * s, even * s + odd * c), dim=-1).flatten(-2)

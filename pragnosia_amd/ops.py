@@ -8,6 +8,7 @@ itself a custom op. There is no CPU path: a CPU tensor raises.
 from __future__ import annotations
 
 import ctypes
+import math
 from typing import Optional
 
 import torch
@@ -74,14 +75,14 @@ class _OverRows(torch.autograd.Function):
             return (g.new_ones(1, g.shape[0]) @ g)[0], None, None
 
 
-def over_rows(v: Tensor, like: Tensor, dtype=None) -> Tensor:
-    """v (d,), in `dtype` (its own if None), broadcast to like's shape (..., d). In a capture its gradient is a sum in
+def over_rows(v: Tensor, shape, dtype=None) -> Tensor:
+    """v (d,), in `dtype` (its own if None), broadcast to `shape` (..., d). In a capture its gradient is a sum in
     v's dtype that records no memset: the one autograd applies to a broadcast operand over many rows is a multi-block
     reduction (see `colsum`). An eager step keeps autograd's, whose host share is the smaller."""
     dtype = dtype or v.dtype
-    if not (like.is_cuda and like.numel() and torch.is_grad_enabled() and v.requires_grad and capturing()):
-        return v.to(dtype).expand(like.shape)
-    return _OverRows.apply(v, like.numel() // like.shape[-1], dtype).view(like.shape)
+    if not (v.is_cuda and v.numel() and torch.is_grad_enabled() and v.requires_grad and capturing()):
+        return v.to(dtype).expand(shape)
+    return _OverRows.apply(v, math.prod(shape[:-1]), dtype).view(shape)
 
 
 @torch.library.custom_op("pragnosia::wgrad", mutates_args=())

@@ -61,16 +61,16 @@ class SpinCarrier(nn.Module):
         # the gate are broadcast over the tokens by `over_rows`: captured, autograd's own sums over many tokens (from
         # 3 x 1999 x 256 on, not at 64 x 128) record memsets, three a layer
         r = torch.sigmoid(linear(z, self.Wr))
-        logmag = -self.gate_c * r * over_rows(-torch.log(mag), r)
+        logmag = -self.gate_c * r * over_rows(-torch.log(mag), r.shape)
         # per-token input normalisation sqrt(1 - |lambda_t|^2), its argument clamped to bound the derivative
         gam = torch.sqrt((1.0 - torch.exp(2.0 * logmag)).clamp_min(1e-6))
         u = self.B(z) * gam * torch.sigmoid(linear(z, self.Wi))
-        y, h = scan_hip(u, logmag, over_rows(ang, logmag), h0)
+        y, h = scan_hip(u, logmag, over_rows(ang, logmag.shape), h0)
         out = self.C(y)
         gate = torch.sigmoid(self.gate)
         if capturing():
             # the sum in fp32, then rounded to the product's type, in which autograd gives it
-            gate = over_rows(gate.to(out.dtype).to(gate.dtype).expand(self.d), out, out.dtype)
+            gate = over_rows(gate.to(out.dtype).to(gate.dtype).expand(self.d), out.shape, out.dtype)
         return x + gate * out, h
 
     def forward_windows(self, x, window: int, h0=None):

@@ -7,17 +7,19 @@ from test_gpu_training import _memset_nodes
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("d,head_dim,delta", [(384, 128, False), (704, 64, False), (768, 64, True)])
-def test_layer_step_records_no_memset(d, head_dim, delta):
+@pytest.mark.parametrize("d,head_dim,delta,T", [(384, 128, False, 400), (704, 64, False, 400), (768, 64, True, 400),
+                                                (704, 176, False, 2048), (352, 176, True, 1000)])
+def test_layer_step_records_no_memset(d, head_dim, delta, T):
     """The step's graph holds no memset node (a reduction of the d x d gated weight to the scalar gate's gradient would
-    record one from d 384 on), and its replays, with eager steps and synchronisations between them, give the eager
-    step's gradients: the gate's to fp32 rounding of sums of d^2 terms, which cancel to some hundredths."""
+    record one from d 384 on, and of the rotation's over 2048 positions to its frequencies' one each for q and k), and
+    its replays, with eager steps and synchronisations between them, give the eager step's gradients: the gate's to fp32
+    rounding of sums of d^2 terms, which cancel to some hundredths, the others to fp32 sums in another order."""
     from pragnosia_amd.assoc import AssocCarrier
     torch.manual_seed(d)
     with torch.device("cuda"):
         m = AssocCarrier(d, head_dim=head_dim, delta=delta)
     m.need_sent = False
-    x, t = torch.zeros(4, 400, d, device="cuda"), torch.randn(4, 400, d, device="cuda")
+    x, t = torch.zeros(4, T, d, device="cuda"), torch.randn(4, T, d, device="cuda")
     params = [p for n, p in m.named_parameters()]
 
     def step():
@@ -39,9 +41,12 @@ def test_layer_step_records_no_memset(d, head_dim, delta):
     for _ in range(6):
         x.normal_()
         graph.replay()
-        got = out[gate].clone()
+        got = [None if o is None else o.clone() for o in out]
         torch.cuda.synchronize()
-        want = step()[gate]
+        eager = step()
+        for (n, _), a, b in zip(m.named_parameters(), got, eager):
+            assert (a is None) == (b is None) and (a is None or n == "gate" or (a - b).norm() <= 1e-4 * b.norm()), n
+        got, want = got[gate], eager[gate]
         assert want.abs() > 0 and (got - want).abs() <= 1e-4 * want.abs() + 1e-3, (got.item(), want.item())
 
 
